@@ -46,7 +46,8 @@ enum {
     PHG_MASS = 0, PHG_LAPLACE = 1, PHG_HELMHOLTZ = 2, PHG_JAC_MASS = 3,
     PHG_DIFF1 = 4, PHG_DIFF2 = 5, PHG_DIFF1_COS = 6, PHG_DIFF2_COS = 7
 };
-/* orthogonalisation of the Arnoldi step: modified Gram-Schmidt, classical
+/* orthogonalisation of the Arnoldi step: modified Gram-Schmidt (phg_gmres: its
+ * coefficients as a triangular solve in dots computed together), classical
  * Gram-Schmidt with one re-orthogonalisation pass, or one classical pass
  * (single pass: block solver only) */
 enum { PHG_MGS = 0, PHG_CGS2 = 1, PHG_CGS1 = 2 };
@@ -200,13 +201,13 @@ typedef struct {
     int diag_scale;  /* 1: right-precondition with the inverse diagonal, x = D^-1 y
                         (the batched FP64 solves without another preconditioner;
                         the stopping test stays on ||b - A x|| / ||b||)    */
-    int persistent;  /* phg_gmres with PHG_MGS: 1 (default) runs each restart
-                        cycle as one cooperative kernel whose workgroups
-                        exchange the dot partials through device memory; 0
-                        launches a kernel per MGS pass (captured in a
-                        hipGraph).  Both give the same bits and, measured at
-                        level 7, the same speed; 1 falls back to 0 where
-                        the device cannot keep every workgroup resident   */
+    int persistent;  /* phg_gmres: 1 (default) runs each restart cycle as one
+                        cooperative kernel whose workgroups exchange the dot
+                        partials through device memory (restart <= 32, up to
+                        262,144 rows); 0 launches kernels for each pass
+                        (captured in a hipGraph).  Both give the same bits;
+                        1 falls back to 0 for other shapes and where the
+                        device cannot keep every workgroup resident      */
 } phg_gmres_opts;
 
 typedef struct {
@@ -215,7 +216,7 @@ typedef struct {
     int refinements;      /* outer refinement steps (mixed forms)         */
     double rel_residual;  /* true FP64 ||b - A x|| / ||b|| at exit          */
     int converged;
-    int cycle_launches;   /* persistent MGS cycles: kernels launched, and  */
+    int cycle_launches;   /* persistent cycles: kernels launched, and      */
     double cycle_ms;      /* their summed duration (HIP events recorded on
                              the solve's stream around each launch); 0
                              for the other forms                        */

@@ -1,0 +1,61 @@
+// Restarted GMRES as persistent cooperative launches (persist.hip): the
+// workspace that a matrix keeps for it, and its entry.
+#pragma once
+#include "phg_internal.h"
+
+namespace phg {
+
+// Exchange rows in uncached device memory from a process-lifetime pool.
+struct XchChunk {
+    unsigned long long* p = nullptr;
+    size_t n = 0;
+    int dev = -1;
+};
+struct XchRows {
+    XchChunk c;
+    XchRows() = default;
+    XchRows(const XchRows&) = delete;
+    XchRows& operator=(const XchRows&) = delete;
+    ~XchRows() { give_back(); }
+    unsigned long long* p() const { return c.p; }
+    void give_back();
+    hipError_t alloc(size_t count);
+};
+
+// A column's state between launches, and its summary for the host.
+struct PState {
+    double bnorm, beta, rel;
+    int iters, cycles, converged, active;
+};
+
+constexpr int XCH_MAXG = 256;       // most workgroups of a launch
+constexpr int PERSIST_NOT_HERE = 2;  // the shape does not run here: nothing was done
+
+struct PersistWork {
+    DevBuf<char> W;              // the vector that the products gather, per column
+    DevBuf<PState> st;           // per column
+    DevBuf<int> abort_dev;
+    PState* host = nullptr;      // pinned: host_k states, then the abort flag
+    int host_k = 0;
+    XchRows xch;                 // two rings of ring_slots words
+    size_t ring_slots = 0;
+    int ring_k = 0, ring_g = 0;  // shape of the launches since the rings were cleared
+    int parity = 0;
+    hipEvent_t ev[2] = {nullptr, nullptr};  // around each launch
+    PersistWork() = default;
+    PersistWork(const PersistWork&) = delete;
+    PersistWork& operator=(const PersistWork&) = delete;
+    ~PersistWork();
+};
+
+// A x_q = b_q for the K columns of B and X (n x K, row-major), each column by
+// itself; o as gmres_batch_solve_pc takes it, also with PHG_MGS.  diag:
+// right-preconditioned with the inverse diagonal (FP64).  stall: a column
+// stops when a whole cycle lowers its residual by less than 1 %.  A launch
+// runs at most max_cycles restart cycles.  The columns' results are left in
+// w->host.  launches (summed count) and ms (summed duration) may be null.
+int persist_solve(phg_matrix_s* A, PersistWork* w, int K, const double* B, double* X,
+                  const phg_gmres_opts& o, bool diag, bool stall, int max_cycles, int* launches,
+                  double* ms, hipStream_t s);
+
+}  // namespace phg

@@ -401,8 +401,8 @@ class Matrix:
     def solve(self, x, b, restart=30, rtol=1e-10, max_iters=200000, ortho=MGS, precision=F64,
               inner_rtol=1e-5, use_x0=False, graph=True, persistent=True, stream=None):
         """Solves A x = b (Solver::solve) with GMRES(restart); returns the info dict.
-        persistent: MGS restart cycles as one cooperative kernel (same bits as
-        a kernel per MGS pass)."""
+        persistent: restart cycles as one cooperative kernel (same bits as
+        kernels for each pass)."""
         o = GmresOpts()
         lib().phg_gmres_default_opts(C.byref(o))
         o.restart, o.max_iters, o.rtol = restart, max_iters, rtol
