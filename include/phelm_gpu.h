@@ -202,12 +202,16 @@ typedef struct {
                         (the batched FP64 solves without another preconditioner;
                         the stopping test stays on ||b - A x|| / ||b||)    */
     int persistent;  /* phg_gmres: 1 (default) runs each restart cycle as one
-                        cooperative kernel whose workgroups exchange the dot
+                        kernel whose workgroups, all resident, exchange the dot
                         partials through device memory (restart <= 32, up to
                         262,144 rows); 0 launches kernels for each pass
                         (captured in a hipGraph).  Both give the same bits;
                         1 falls back to 0 for other shapes and where the
-                        device cannot keep every workgroup resident      */
+                        device cannot keep every workgroup resident.
+                        phg_gmres_batch: 1 runs the columns that way where
+                        it is the faster form for (rows, nrhs, restart,
+                        precision, ortho), 0 never; the two add their dot
+                        partials in other groups                        */
 } phg_gmres_opts;
 
 typedef struct {
@@ -257,7 +261,8 @@ int phg_block_gmres(phg_matrix_t A, int nrhs, const double *d_B, double *d_X,
 /* d_B, d_X: n_rows x nrhs FP64, row-major (entry (i, q) at i * nrhs + q).
  * opts->restart <= 32, opts->ortho PHG_CGS2 or PHG_CGS1, opts->precision
  * PHG_F64 or mixed (PHG_F32 / PHG_BF16 inner Krylov, FP64 refinement).
- * A column's result does not depend on the other columns of the call.
+ * A column's result does not depend on the other columns of the call (the
+ * form that runs, opts->persistent, follows from the sizes alone).
  * infos: nrhs host entries (may be NULL).  Returns PHG_ERR_NOCONV unless
  * every column converged. */
 int phg_gmres_batch(phg_matrix_t A, int nrhs, const double *d_B, double *d_X,

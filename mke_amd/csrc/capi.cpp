@@ -66,6 +66,7 @@ phg_matrix_s::~phg_matrix_s()
     for (auto& w : work) w.reset();
     phg::block_destroy(bwork);
     for (auto* b : batch) phg::batch_destroy(b);
+    for (auto* b : pbatch) phg::persist_destroy(b);
 }
 
 using namespace phg;

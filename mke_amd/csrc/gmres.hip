@@ -18,10 +18,9 @@
 // basis vectors' own products, which the step before has computed: see
 // mgs_solve in krylov.h.
 //
-// Up to 262,144 rows and m <= 32 a restart cycle is one persistent
-// cooperative launch (persist.hip).  Here are the driver and the form with a
-// launch per pass, for larger matrices and restarts and where the cooperative
-// launch is refused.  Its kernels per Arnoldi step: the SpMV with the first
+// Up to 262,144 rows and m <= 32 a restart cycle is one persistent launch
+// (persist.hip).  Here are the driver and the form with a launch per pass, for
+// larger matrices and restarts.  Its kernels per Arnoldi step: the SpMV with the first
 // pass's dots, the update with the dots of the next pass or of the next
 // basis vector and the norm (twice for CGS2), and after each of them one
 // workgroup that adds the block partials and does the step's small dense
@@ -717,7 +716,7 @@ int gmres_solve(phg_matrix_s* A, const double* b, double* x, const phg_gmres_opt
         // one launch per restart cycle
         int launches = 0;
         double ms = 0.0;
-        rc = persist_solve(A, &w->persist, 1, b, x, o, false, false, 1, &launches, &ms, s);
+        rc = persist_solve(A, &w->persist, 1, b, x, o, false, false, 1, 1, &launches, &ms, s);
         if (rc == PHG_OK) {
             const PState& h = w->persist.host[0];
             if (info) {

@@ -25,6 +25,10 @@
 // or on the other columns: a column's result is bit-identical whatever else
 // is in the batch, provided KP is the same.  A restart cycle is captured in
 // one hipGraph and replayed; the host reads a K-entry summary per cycle.
+//
+// Where the columns' rows fit the chip in few enough launches, the solve runs
+// as persistent launches instead (persist.hip; persistent_rounds below has
+// the rule and what both sides measured).
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -32,6 +36,7 @@
 #include <mutex>
 
 #include "ell.h"
+#include "persist.h"
 #include "phg_internal.h"
 
 namespace phg {
@@ -1115,6 +1120,56 @@ void set_shape_rpt(int n, int kp, int prec, int rpt)
     g_shape_rpt[{n, kp, prec}] = rpt;
 }
 
+// How many persistent launches (persist.hip) the K columns may take for that
+// form to be the faster one, from the time per Arnoldi step of both.  The
+// kernels here: 26 us for the four launches of a step with one Gram-Schmidt
+// pass, 43 us for the six with two, and the vectors they read and write at
+// 4.2 TB/s.  A persistent launch: 6.8 to 12 us, and 0.01 us per workgroup of
+// a column.  Measured at levels 4 to 7 with 1 to 64 columns the model is
+// within 15 % of either; per step, here and persistent: level 5 x 8 columns
+// FP64 CGS2 48 and 12 us, level 6 x 64 303 and 144, level 7 x 1 56 and 14,
+// level 7 x 16 277 and 234; level 7 x 16 FP32 CGS1 103 and 145; mass solves
+// (restart 8, CGS1) level 6 x 24 61 and 52, level 6 x 64 101 and 143.
+int persistent_rounds(int n, int kp, int m, bool f64, bool twice)
+{
+    const double passes = twice ? 2.0 : 1.0, es = f64 ? 8.0 : 4.0;
+    const double vectors = 0.5 * (m + 1) * (passes + 1.0) + 5.0 + 16.0 / m;
+    const double here = 9.0 + 17.0 * passes + (double)n * kp * es * vectors / 4.2e6;
+    const double there = (f64 ? 9.0 : 6.8) + (passes - 1.0) * (f64 ? 3.0 : 2.7) +
+                         0.01 * n / 1024.0 + 24.0 / m;
+    return (int)(here / there);
+}
+
+// The columns as persistent launches, where that is the faster form;
+// PERSIST_NOT_HERE otherwise.
+int batch_persistent(phg_matrix_s* A, int K, const double* B, double* X, const phg_gmres_opts& o,
+                     phg_gmres_info* infos, hipStream_t s)
+{
+    const int rounds = persistent_rounds(A->n_rows, next_pow2(K), o.restart,
+                                         o.precision == PHG_F64, o.ortho == PHG_CGS2);
+    PersistWork*& w = A->pbatch[o.precision == PHG_F64 ? 0 : 1];
+    if (!w) w = new PersistWork();
+    // a launch ends after some 4,000 Arnoldi steps (50 ms) for the host to look
+    const int max_cycles = std::max(1, 4096 / o.restart);
+    const int rc = persist_solve(A, w, K, B, X, o, o.precision == PHG_F64 && o.diag_scale, true,
+                                 max_cycles, rounds, nullptr, nullptr, s);
+    if (rc) return rc;
+    bool all = true;
+    for (int q = 0; q < K; ++q) {
+        const PState& h = w->host[q];
+        all = all && h.converged;
+        if (infos) {
+            memset(&infos[q], 0, sizeof infos[q]);
+            infos[q].iterations = h.iters;
+            infos[q].restarts = h.cycles;
+            infos[q].refinements = o.precision == PHG_F64 ? 0 : h.cycles;
+            infos[q].rel_residual = h.rel;
+            infos[q].converged = h.converged;
+        }
+    }
+    return all ? PHG_OK : PHG_ERR_NOCONV;
+}
+
 // Deterministic right-hand sides for timing: values in [-1, 1) from a hash.
 __global__ void bk_fill_hash(size_t n, double* __restrict__ x)
 {
@@ -1177,6 +1232,15 @@ int gmres_batch_solve_pc(phg_matrix_s* A, int K, const double* B, double* X,
         rc = o.precision == PHG_F64 ? pc->reserve(kp) : pc->reserve_f32(kp);
         if (rc) return rc;
     }
+    const bool diag = o.precision == PHG_F64 && o.diag_scale && !pc;
+    if (diag) rc = ensure_ell64_diag(A, s);
+    else if (o.precision == PHG_F32) rc = ensure_ell32(A, s);
+    else if (o.precision == PHG_BF16) rc = ensure_ell16(A, s);
+    if (rc) return rc;
+    if (!pc && o.persistent) {
+        rc = batch_persistent(A, K, B, X, o, infos, s);
+        if (rc != PERSIST_NOT_HERE) return rc;
+    }
     BatchWork* w = nullptr;
     const int slot = o.precision == PHG_F64 ? 0 : 1;
     // the autotuner times the plain form, so a preconditioned solve keeps the
@@ -1186,21 +1250,11 @@ int gmres_batch_solve_pc(phg_matrix_s* A, int K, const double* B, double* X,
     rc = prepare_batch(A, slot, o.precision == PHG_F64 ? PHG_F64 : PHG_F32, o.restart, kp, rpt,
                        pc != nullptr, &w);
     if (rc) return rc;
-    if (o.precision == PHG_F64) {
-        if (o.diag_scale && !pc) {  // right preconditioning by D^-1: solve (A D^-1) y = b, x = D^-1 y
-            rc = ensure_ell64_diag(A, s);
-            if (rc) return rc;
-            return batch_run<double, double>(A, A->ell64d, w, K, B, X, o, infos, nullptr, s);
-        }
-        return batch_run<double, double>(A, A->ell64, w, K, B, X, o, infos, pc, s);
-    }
-    if (o.precision == PHG_F32) {
-        rc = ensure_ell32(A, s);
-        if (rc) return rc;
+    // diag: right preconditioning by D^-1: solve (A D^-1) y = b, x = D^-1 y
+    if (o.precision == PHG_F64)
+        return batch_run<double, double>(A, diag ? A->ell64d : A->ell64, w, K, B, X, o, infos, pc, s);
+    if (o.precision == PHG_F32)
         return batch_run<float, float>(A, A->ell32, w, K, B, X, o, infos, pc, s);
-    }
-    rc = ensure_ell16(A, s);
-    if (rc) return rc;
     return batch_run<float, uint16_t>(A, A->ell16, w, K, B, X, o, infos, pc, s);
 }
 
@@ -1242,6 +1296,7 @@ int gmres_batch_tune(phg_matrix_s* A, int K, const phg_gmres_opts* opts, hipStre
     o.inner_rtol = 0.0;
     o.use_x0 = 0;
     o.graph = 1;
+    o.persistent = 0;  // the form whose shape is being chosen
     DevBuf<double> B, X;
     PHG_HIP(B.alloc((size_t)n * K));
     PHG_HIP(X.alloc((size_t)n * K));

@@ -1,4 +1,4 @@
-// Restarted GMRES as persistent cooperative launches (persist.hip): the
+// Restarted GMRES as persistent launches (persist.hip): the
 // workspace that a matrix keeps for it, and its entry.
 #pragma once
 #include "phg_internal.h"
@@ -52,10 +52,12 @@ struct PersistWork {
 // itself; o as gmres_batch_solve_pc takes it, also with PHG_MGS.  diag:
 // right-preconditioned with the inverse diagonal (FP64).  stall: a column
 // stops when a whole cycle lowers its residual by less than 1 %.  A launch
-// runs at most max_cycles restart cycles.  The columns' results are left in
-// w->host.  launches (summed count) and ms (summed duration) may be null.
+// runs at most max_cycles restart cycles of the columns that fit the device
+// together; columns that need more than max_rounds launches do not run here.
+// The columns' results are left in w->host.  launches (summed count) and ms
+// (summed duration) may be null.
 int persist_solve(phg_matrix_s* A, PersistWork* w, int K, const double* B, double* X,
-                  const phg_gmres_opts& o, bool diag, bool stall, int max_cycles, int* launches,
-                  double* ms, hipStream_t s);
+                  const phg_gmres_opts& o, bool diag, bool stall, int max_cycles, int max_rounds,
+                  int* launches, double* ms, hipStream_t s);
 
 }  // namespace phg

@@ -1,5 +1,5 @@
-// Restarted GMRES(m), m <= 32, as persistent cooperative launches: all
-// workgroups are resident, a column of the right-hand side belongs to G
+// Restarted GMRES(m), m <= 32, as persistent launches: all workgroups of a
+// launch are resident, a column of the right-hand side belongs to G
 // workgroups of KR_ROWS rows each, and a restart cycle keeps everything that
 // it owns on the chip.  A thread holds its rows of every basis vector, of
 // the work vector and of the matrix in registers; only the vector that the
@@ -17,10 +17,13 @@
 // Columns are independent: each group of G workgroups runs its own cycles
 // and stops by itself, so the batched solves of small meshes (gmres_batch)
 // run here as one launch.
-#include <atomic>
+#include <unistd.h>
+
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <thread>
 
 #include "krylov.h"
 #include "persist.h"
@@ -103,6 +106,10 @@ constexpr xch_t XCH_EMPTY = 0x7FF4DEADBEEF0001ull;  // a signalling-NaN pattern 
 constexpr long XCH_SPIN = 1L << 22;                  // polls before a wait gives up
 // (PHG_XCH_SPIN overrides it: the failure-path test forces a give-up with
 // a limit of a few polls; every workgroup still exits normally)
+// polls of a launch's first exchange (some 0.1 s), and launches until it succeeds
+constexpr long XCH_START = 1L << 17;
+constexpr int XCH_TRIES = 64;
+enum { ABORT_WAIT = 1, ABORT_START = 2 };  // bits of the host's abort word
 constexpr int XCH_RING = 4;   // rows of a column's ring
 constexpr int XCH_V = 32;     // values of a slot
 constexpr int PS_M = 32;      // largest restart
@@ -132,10 +139,19 @@ constexpr int PS_M = 32;      // largest restart
 // gathered with agent-scope loads; no cache-wide write-back or invalidation
 // is needed.  Every wait is bounded: after `spin` polls a workgroup raises
 // the abort flag and leaves, and the others leave at their next look at it.
+//
+// The first exchange of a launch shows that its workgroups are resident
+// together: each stays until it has seen the others' slots.  If something
+// else holds the CUs (another process's launch, half of it waiting for this
+// one's other half), that exchange ends after start_spin polls, and the host
+// launches again: x and the state of the columns are written only after
+// later exchanges, so nothing is lost.  Within a process launches take turns
+// (launch_mutex).  A cooperative launch would give the same guarantee but is
+// refused to every process of a GPU except the first that asks.
 struct Hop {
     xch_t* ring;
     int G, bid, e;  // G: slots of a row (padded workgroup count)
-    long spin;
+    long spin, start_spin;
     int *abort_dev, *abort_host;
 };
 
@@ -153,10 +169,11 @@ struct HopLds {
 template <int NQ>
 __device__ __forceinline__ bool hop_poll(const Hop& h, const xch_t* row, int val, double* sum)
 {
+    const long spin = h.e == 0 ? h.start_spin : h.spin;
     const unsigned off = ((threadIdx.x >> 5) * XCH_V + val) * (unsigned)sizeof(xch_t);
     xch_t u[NQ];
-    bool ok = false;
-    for (long it = 0; it < h.spin; ++it) {
+    bool ok = false, left = false;
+    for (long it = 0; it < spin; ++it) {
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
             u[q] = ld_agent((const xch_t*)((const char*)(row + KR_GRP * q * XCH_V) + off));
@@ -167,7 +184,15 @@ __device__ __forceinline__ bool hop_poll(const Hop& h, const xch_t* row, int val
             ok = true;
             break;
         }
-        if ((it & 63) == 63 && ld_agent(h.abort_dev)) break;
+        if ((it & 63) == 63 && ld_agent(h.abort_dev)) {
+            left = true;
+            break;
+        }
+    }
+    if (!ok && !left) {
+        st_agent(h.abort_dev, 1);
+        __hip_atomic_fetch_or(h.abort_host, h.e == 0 ? ABORT_START : ABORT_WAIT, __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_SYSTEM);
     }
     double a[2] = {0.0, 0.0};
 #pragma unroll
@@ -208,11 +233,7 @@ __device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool check, HopLds
     else if (h.G == 176) ok = hop_poll<11>(h, row, val, &sum);
     else ok = hop_poll<16>(h, row, val, &sum);
     l->g[t >> 5][i] = sum;
-    if (!ok) {
-        l->bad = 1;
-        st_agent(h.abort_dev, 1);
-        __hip_atomic_store(h.abort_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (!ok) l->bad = 1;
     __syncthreads();
     *tot = krylov_join(l->g, i);
     ++h.e;
@@ -222,20 +243,20 @@ __device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool check, HopLds
 // --------------------------------------------------------------- kernel --
 template <typename VT, typename MT>
 struct PArgs {
-    int n, K, G, Gp, m, width, width64;
+    int n, ld, G, Gp, m, width, width64;
     const int* col;
     const MT* val;
     const int* col64;
     const double* val64;
     const double* dscale;  // x += dscale * (V y), or null
-    const double* B;       // n x K, column q at q
+    const double* B;       // row-major, ld columns; column q at q
     double* X;
-    VT* W;                 // K vectors of ldw
+    VT* W;                 // a vector of ldw per column
     size_t ldw;
-    xch_t *ring, *other;   // K x XCH_RING rows of Gp slots each
+    xch_t *ring, *other;   // XCH_RING rows of Gp slots per column
     PState *st, *host;
     int *abort_dev, *abort_host;
-    long spin;
+    long spin, start_spin;
     double rtol, inner_rtol;
     int max_iters, max_cycles, first, use_x0, stall;
 };
@@ -357,9 +378,9 @@ k_persist(PArgs<VT, MT> a)
     __shared__ double s_h[PS_M + 8];  // Hessenberg column of the last step
     const int t = threadIdx.x, lane = t & 63, li = lane & 31;
     const int q = (int)blockIdx.x / a.G, bid = (int)blockIdx.x % a.G;
-    const int n = a.n, K = a.K, m = a.m;
-    Hop h{a.ring + (size_t)q * XCH_RING * a.Gp * XCH_V, a.Gp, bid, 0, a.spin, a.abort_dev,
-          a.abort_host};
+    const int n = a.n, ld = a.ld, m = a.m;
+    Hop h{a.ring + (size_t)q * XCH_RING * a.Gp * XCH_V, a.Gp, bid, 0, a.spin, a.start_spin,
+          a.abort_dev, a.abort_host};
     if (t < XCH_RING * XCH_V)
         st_agent(a.other + (size_t)q * XCH_RING * a.Gp * XCH_V +
                      ((size_t)(t >> 5) * a.Gp + bid) * XCH_V + (t & 31), XCH_EMPTY);
@@ -378,11 +399,11 @@ k_persist(PArgs<VT, MT> a)
 #pragma unroll
         for (int r = 0; r < KR_RPT; ++r) {
             const int rr = base + r * KR_BS;
-            b[r] = rr < n ? B[(size_t)rr * K] : 0.0;
+            b[r] = rr < n ? B[(size_t)rr * ld] : 0.0;
             r0[r] = b[r];
         }
         if (a.use_x0) {
-            krylov_rows<double, double, false, KR_RPT>(n, a.width64, base, a.col64, a.val64, X, K,
+            krylov_rows<double, double, false, KR_RPT>(n, a.width64, base, a.col64, a.val64, X, ld,
                                                        1.0, xo, ax);
 #pragma unroll
             for (int r = 0; r < KR_RPT; ++r) r0[r] = b[r] - ax[r];
@@ -390,7 +411,7 @@ k_persist(PArgs<VT, MT> a)
 #pragma unroll
         for (int r = 0; r < KR_RPT; ++r) {
             const int rr = base + r * KR_BS;
-            if (rr < n && !a.use_x0) st_agent(X + (size_t)rr * K, 0.0);
+            if (rr < n && !a.use_x0) st_agent(X + (size_t)rr * ld, 0.0);
             w[r] = (VT)r0[r];
             if (rr < n) st_agent(W + rr, w[r]);
         }
@@ -524,7 +545,7 @@ k_persist(PArgs<VT, MT> a)
             for (int i = 0; i < PS_M; ++i) s = fma(to_d(V.at(i / KR_T, i % KR_T, r)), s_y[i], s);
             if (rr < n) {
                 if (a.dscale) s = a.dscale[rr] * s;
-                double* x = X + (size_t)rr * K;
+                double* x = X + (size_t)rr * ld;
                 st_agent(x, ld_agent(x) + s);
             }
         }
@@ -533,12 +554,12 @@ k_persist(PArgs<VT, MT> a)
         // r = b - A x in FP64, the next cycle's vector
         double res[KR_RPT], xo[KR_RPT];
         const int rb = opaque(base);
-        krylov_rows<double, double, true, KR_RPT>(n, a.width64, rb, a.col64, a.val64, X, K, 1.0,
+        krylov_rows<double, double, true, KR_RPT>(n, a.width64, rb, a.col64, a.val64, X, ld, 1.0,
                                                   xo, res);
 #pragma unroll
         for (int r = 0; r < KR_RPT; ++r) {
             const int rr = rb + r * KR_BS;
-            res[r] = rr < n ? B[(size_t)rr * K] - res[r] : 0.0;
+            res[r] = rr < n ? B[(size_t)rr * ld] - res[r] : 0.0;
             w[r] = (VT)res[r];
             if (rr < n) st_agent(W + rr, w[r]);
         }
@@ -574,54 +595,97 @@ __global__ void k_ring_reset(xch_t* ring, size_t count, int G, int Gp, int* abor
     if (i == 0) *abort_dev = 0;
 }
 
-// Set once a cooperative launch was refused by the runtime: later solves of
-// the process take the launch-per-pass forms directly.
-std::atomic<bool>& coop_refused()
+// Launches of one device take turns: two that each hold half of the CUs would
+// wait for each other until they give up.
+std::mutex& launch_mutex(int dev)
 {
-    static std::atomic<bool> refused{false};
-    return refused;
+    static std::mutex m[64];
+    return m[dev & 63];
 }
 
 // Workgroups of the kernel that the device holds at once, per template
 // instance, computed once (thread-safe static initialisation).
 template <typename VT, typename MT, int ORTHO>
-int coop_capacity()
+int capacity()
 {
-    static const int capacity = [] {
-        int dev = 0, cus = 0, coop = 0, per = 0;
+    static const int n = [] {
+        int dev = 0, cus = 0, per = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &per, (const void*)k_persist<VT, MT, ORTHO>, KR_BS, 0) != hipSuccess)
             return 0;
-        return coop ? cus * per : 0;
+        return cus * per;
     }();
-    return capacity;
+    return n;
+}
+
+// Columns q0 .. q0 + K - 1 of the ld in B and X.
+template <typename VT, typename MT, int ORTHO>
+int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int ld, const double* B,
+           double* X, const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles,
+           int first, hipStream_t s)
+{
+    const int n = A->n_rows, G = (n + KR_ROWS - 1) / KR_ROWS, Gp = hop_slots(G);
+    const size_t ldw = ((size_t)n + 63) / 64 * 64, slots = (size_t)K * XCH_RING * Gp * XCH_V;
+    if (w->ring_k != K || w->ring_g != G) {
+        // another shape than the last launch's, or after a give-up
+        hipLaunchKernelGGL(k_ring_reset, dim3((unsigned)((2 * slots + 255) / 256)), dim3(256), 0, s,
+                           w->xch.p(), 2 * slots, G, Gp, w->abort_dev.p);
+        PHG_HIP(hipGetLastError());
+        w->ring_k = K;
+        w->ring_g = G;
+    }
+    PArgs<VT, MT> a;
+    a.n = n, a.ld = ld, a.G = G, a.Gp = Gp, a.m = o.restart, a.width = E.width;
+    a.width64 = A->ell64.width;
+    a.col = E.col.p, a.val = E.val.p, a.col64 = A->ell64.col.p, a.val64 = A->ell64.val.p;
+    a.dscale = dscale, a.B = B + q0, a.X = X + q0, a.W = (VT*)w->W.p + (size_t)q0 * ldw, a.ldw = ldw;
+    a.ring = w->xch.p() + (w->parity ? slots : 0);
+    a.other = w->xch.p() + (w->parity ? 0 : slots);
+    w->parity ^= 1;
+    a.st = w->st.p + q0, a.host = w->host + q0;
+    a.abort_dev = w->abort_dev.p, a.abort_host = (int*)(w->host + w->host_k);
+    a.spin = XCH_SPIN;
+    if (const char* e = getenv("PHG_XCH_SPIN")) a.spin = std::max(1L, atol(e));
+    a.start_spin = std::min(a.spin, XCH_START);
+    a.rtol = o.rtol;
+    a.inner_rtol = o.precision == PHG_F64 ? 0.0 : o.inner_rtol;
+    a.max_iters = o.max_iters, a.max_cycles = max_cycles, a.use_x0 = o.use_x0;
+    a.stall = stall, a.first = first;
+    for (int q = q0; q < q0 + K; ++q) w->host[q].active = -1;  // until the kernel writes it
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_persist<VT, MT, ORTHO>), dim3(G * K), dim3(KR_BS), 0, s, a);
+    PHG_HIP(hipGetLastError());
+    return PHG_OK;
 }
 
 template <typename VT, typename MT, int ORTHO>
 int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
-        const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles, int* launches,
-        double* ms, hipStream_t s)
+        const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles, int max_rounds,
+        int* launches, double* ms, hipStream_t s)
 {
     const int n = A->n_rows, G = (n + KR_ROWS - 1) / KR_ROWS;
-    if (coop_refused().load() || G * K > std::min(coop_capacity<VT, MT, ORTHO>(), XCH_MAXG))
-        return PERSIST_NOT_HERE;
-    const int Gp = hop_slots(G);
-    const size_t ldw = ((size_t)n + 63) / 64 * 64, slots = (size_t)K * XCH_RING * Gp * XCH_V;
+    // columns of a launch, and launches for all columns, of equal size
+    const int fit = std::min(capacity<VT, MT, ORTHO>(), XCH_MAXG) / G;
+    if (fit < 1) return PERSIST_NOT_HERE;
+    const int rounds = (K + fit - 1) / fit, per = (K + rounds - 1) / rounds;
+    if (rounds > max_rounds) return PERSIST_NOT_HERE;
+    const size_t ldw = ((size_t)n + 63) / 64 * 64;
+    const size_t slots = (size_t)per * XCH_RING * hop_slots(G) * XCH_V;
     const size_t bytes = (size_t)K * ldw * sizeof(VT);
     if (w->W.n < bytes) PHG_HIP(w->W.alloc(bytes));
-    if (w->st.n < (size_t)K) {
-        PHG_HIP(w->st.alloc(K));
+    if (w->host_k < K) {
         if (w->host) (void)hipHostFree(w->host);
         w->host = nullptr;
-        // K states, then the abort flag
+        w->host_k = 0;
+        PHG_HIP(w->st.alloc(K));
+        // K states, then the abort word
         PHG_HIP(hipHostMalloc((void**)&w->host, sizeof(PState) * (K + 1), hipHostMallocDefault));
         w->host_k = K;
     }
     if (!w->abort_dev.p) PHG_HIP(w->abort_dev.alloc(1));
     if (w->ring_slots < slots) {
+        w->ring_slots = 0;
         PHG_HIP(w->xch.alloc(2 * slots));
         w->ring_slots = slots;
         w->ring_k = 0;
@@ -630,59 +694,55 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
         PHG_HIP(hipEventCreate(&w->ev[0]));
         PHG_HIP(hipEventCreate(&w->ev[1]));
     }
-    int* abort_host = (int*)(w->host + w->host_k);
-    PArgs<VT, MT> a;
-    a.n = n, a.K = K, a.G = G, a.Gp = Gp, a.m = o.restart, a.width = E.width, a.width64 = A->ell64.width;
-    a.col = E.col.p, a.val = E.val.p, a.col64 = A->ell64.col.p, a.val64 = A->ell64.val.p;
-    a.dscale = dscale, a.B = B, a.X = X, a.W = (VT*)w->W.p, a.ldw = ldw;
-    a.st = w->st.p, a.host = w->host, a.abort_dev = w->abort_dev.p, a.abort_host = abort_host;
-    a.spin = XCH_SPIN;
-    if (const char* e = getenv("PHG_XCH_SPIN")) a.spin = std::max(1L, atol(e));
-    a.rtol = o.rtol;
-    a.inner_rtol = o.precision == PHG_F64 ? 0.0 : o.inner_rtol;
-    a.max_iters = o.max_iters, a.max_cycles = max_cycles, a.use_x0 = o.use_x0;
-    a.stall = stall;
+    int dev = 0;
+    PHG_HIP(hipGetDevice(&dev));
+    std::unique_lock<std::mutex> turn(launch_mutex(dev), std::try_to_lock);
+    if (!turn.owns_lock()) {
+        // another thread's solve runs: wait for this stream's earlier work
+        // first, so that nobody waits for that while it is this one's turn
+        PHG_HIP(hipStreamSynchronize(s));
+        turn.lock();
+    }
+    volatile int* abort_host = (int*)(w->host + w->host_k);
+    int tries = 0;
     for (int first = 1;; first = 0) {
-        if (w->ring_k != K || w->ring_g != G) {
-            // another shape than the last launch's, or after a give-up
-            hipLaunchKernelGGL(k_ring_reset, dim3((unsigned)((2 * slots + 255) / 256)), dim3(256),
-                               0, s, w->xch.p(), 2 * slots, G, Gp, w->abort_dev.p);
-            PHG_HIP(hipGetLastError());
-            w->ring_k = K;
-            w->ring_g = G;
-        }
-        a.first = first;
-        a.ring = w->xch.p() + (w->parity ? slots : 0);
-        a.other = w->xch.p() + (w->parity ? 0 : slots);
-        w->parity ^= 1;
-        *abort_host = 0;
-        void* args[] = {&a};
-        if (ms) PHG_HIP(hipEventRecord(w->ev[0], s));
-        const hipError_t e = hipLaunchCooperativeKernel((const void*)k_persist<VT, MT, ORTHO>,
-                                                        dim3(G * K), dim3(KR_BS), args, 0, s);
-        if (e != hipSuccess) {
-            // refused here: the launch-per-pass form for this solve and, from
-            // now on, for this process
-            (void)hipGetLastError();
-            coop_refused().store(true);
-            w->ring_k = 0;
-            if (first) return PERSIST_NOT_HERE;
+        for (int q = 0; q < K; ++q)
+            if (first) w->host[q].active = 1;
+        // the columns still running, and one by one those of a launch that
+        // did not start
+        for (bool again = false;; again = true) {
+            *abort_host = 0;
+            if (ms) PHG_HIP(hipEventRecord(w->ev[0], s));
+            const int step = again ? 1 : per;
+            for (int q0 = 0; q0 < K; q0 += step) {
+                const int kq = std::min(step, K - q0);
+                bool any = false;
+                for (int q = q0; q < q0 + kq; ++q)
+                    any = any || (again ? w->host[q].active == -1 : w->host[q].active == 1);
+                if (!any) continue;
+                const int rc = launch<VT, MT, ORTHO>(A, E, w, q0, kq, K, B, X, o, dscale, stall,
+                                                     max_cycles, first, s);
+                if (rc) return rc;
+                if (launches) ++*launches;
+            }
+            if (ms) PHG_HIP(hipEventRecord(w->ev[1], s));
+            const hipError_t e = hipStreamSynchronize(s);
+            if (e != hipSuccess) w->ring_k = 0;
             PHG_HIP(e);
-        }
-        if (ms) PHG_HIP(hipEventRecord(w->ev[1], s));
-        const hipError_t se = hipStreamSynchronize(s);
-        if (se != hipSuccess) w->ring_k = 0;
-        PHG_HIP(se);
-        if (*(volatile int*)abort_host) {
+            if (ms) {
+                float t = 0.0f;
+                PHG_HIP(hipEventElapsedTime(&t, w->ev[0], w->ev[1]));
+                *ms += t;
+            }
+            if (!*abort_host) break;
             w->ring_k = 0;
-            set_error("gmres: a workgroup of the persistent solve timed out waiting for the others");
-            return PHG_ERR_HIP;
-        }
-        if (launches) ++*launches;
-        if (ms) {
-            float t = 0.0f;
-            PHG_HIP(hipEventElapsedTime(&t, w->ev[0], w->ev[1]));
-            *ms += t;
+            if ((*abort_host & ABORT_WAIT) || ++tries >= XCH_TRIES) {
+                set_error("gmres: a workgroup of the persistent solve timed out waiting for the "
+                          "others");
+                return PHG_ERR_HIP;
+            }
+            // two processes that collided do not try again at the same moment
+            std::this_thread::sleep_for(std::chrono::microseconds(100 * (1 + (getpid() * 7 + tries) % 32)));
         }
         bool any = false;
         for (int q = 0; q < K; ++q) any = any || w->host[q].active;
@@ -691,38 +751,36 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
     return PHG_OK;
 }
 
-template <typename VT, typename MT>
+template <typename VT, typename MT, typename... Rest>
 int run_ortho(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
-              const phg_gmres_opts& o, const double* d, bool stall, int max_cycles, int* launches,
-              double* ms, hipStream_t s)
+              const phg_gmres_opts& o, Rest... rest)
 {
     switch (o.ortho) {
-    case PHG_MGS:
-        return run<VT, MT, PHG_MGS>(A, E, w, K, B, X, o, d, stall, max_cycles, launches, ms, s);
-    case PHG_CGS2:
-        return run<VT, MT, PHG_CGS2>(A, E, w, K, B, X, o, d, stall, max_cycles, launches, ms, s);
-    default:
-        return run<VT, MT, PHG_CGS1>(A, E, w, K, B, X, o, d, stall, max_cycles, launches, ms, s);
+    case PHG_MGS: return run<VT, MT, PHG_MGS>(A, E, w, K, B, X, o, rest...);
+    case PHG_CGS2: return run<VT, MT, PHG_CGS2>(A, E, w, K, B, X, o, rest...);
+    default: return run<VT, MT, PHG_CGS1>(A, E, w, K, B, X, o, rest...);
     }
 }
 
 }  // namespace
 
+void persist_destroy(PersistWork* w) { delete w; }
+
 int persist_solve(phg_matrix_s* A, PersistWork* w, int K, const double* B, double* X,
-                  const phg_gmres_opts& o, bool diag, bool stall, int max_cycles, int* launches,
-                  double* ms, hipStream_t s)
+                  const phg_gmres_opts& o, bool diag, bool stall, int max_cycles, int max_rounds,
+                  int* launches, double* ms, hipStream_t s)
 {
-    if (o.restart > PS_M || (A->n_rows + KR_ROWS - 1) / KR_ROWS > XCH_MAXG / K)
-        return PERSIST_NOT_HERE;
+    if (o.restart > PS_M || A->n_rows > KR_ROWS * XCH_MAXG) return PERSIST_NOT_HERE;
+    const double* none = nullptr;
     if (o.precision == PHG_F64)
         return run_ortho<double, double>(A, diag ? A->ell64d : A->ell64, w, K, B, X, o,
-                                         diag ? A->dinv.p : nullptr, stall, max_cycles, launches,
-                                         ms, s);
+                                         diag ? (const double*)A->dinv.p : none, stall, max_cycles,
+                                         max_rounds, launches, ms, s);
     if (o.precision == PHG_F32)
-        return run_ortho<float, float>(A, A->ell32, w, K, B, X, o, nullptr, stall, max_cycles,
-                                       launches, ms, s);
-    return run_ortho<float, uint16_t>(A, A->ell16, w, K, B, X, o, nullptr, stall, max_cycles,
-                                      launches, ms, s);
+        return run_ortho<float, float>(A, A->ell32, w, K, B, X, o, none, stall, max_cycles,
+                                       max_rounds, launches, ms, s);
+    return run_ortho<float, uint16_t>(A, A->ell16, w, K, B, X, o, none, stall, max_cycles,
+                                      max_rounds, launches, ms, s);
 }
 
 }  // namespace phg

@@ -97,9 +97,11 @@ struct Ell {
 struct GmresWork;  // gmres.hip
 struct BlockWork;  // block.hip
 struct BatchWork;  // gmres_batch.hip
+struct PersistWork;  // persist.hip
 void destroy_gmres_work(GmresWork* w);
 void block_destroy(BlockWork* w);
 void batch_destroy(BatchWork* w);
+void persist_destroy(PersistWork* w);
 struct GmresWorkDeleter {
     void operator()(GmresWork* w) const { destroy_gmres_work(w); }
 };
@@ -129,6 +131,7 @@ struct phg_matrix_s {
     std::unique_ptr<phg::GmresWork, phg::GmresWorkDeleter> work[6];
     phg::BlockWork* bwork = nullptr;  // block GMRES workspace
     phg::BatchWork* batch[2] = {nullptr, nullptr};  // batched GMRES: FP64, mixed
+    phg::PersistWork* pbatch[2] = {nullptr, nullptr};  // its persistent form
     ~phg_matrix_s();
 };
 

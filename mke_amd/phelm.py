@@ -401,7 +401,7 @@ class Matrix:
     def solve(self, x, b, restart=30, rtol=1e-10, max_iters=200000, ortho=MGS, precision=F64,
               inner_rtol=1e-5, use_x0=False, graph=True, persistent=True, stream=None):
         """Solves A x = b (Solver::solve) with GMRES(restart); returns the info dict.
-        persistent: restart cycles as one cooperative kernel (same bits as
+        persistent: restart cycles as one kernel each (same bits as
         kernels for each pass)."""
         o = GmresOpts()
         lib().phg_gmres_default_opts(C.byref(o))

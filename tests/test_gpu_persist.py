@@ -91,3 +91,57 @@ def test_start_vector_and_zero_right_side():
         assert info["converged"] and info["iterations"] == 0 and not z.any()
     assert torch.equal(got[0], got[1])
     A.close()
+
+
+def _batch(A, B, x0=None, persistent=1, **kw):
+    """phg_gmres_batch with opts.persistent given."""
+    import ctypes as C
+    from mke_amd.phelm import GmresInfo, GmresOpts, check
+    o = GmresOpts()
+    P.lib().phg_gmres_default_opts(C.byref(o))
+    o.rtol, o.persistent = 1e-10, persistent
+    for k, v in kw.items():
+        setattr(o, k, v)
+    X = torch.zeros_like(B) if x0 is None else x0.clone()
+    o.use_x0 = int(x0 is not None)
+    infos = (GmresInfo * B.shape[1])()
+    check(P.lib().phg_gmres_batch(A.h, B.shape[1], B.data_ptr(), X.data_ptr(), C.byref(o), infos,
+                                  None), "phg_gmres_batch")
+    return X, [i.iterations for i in infos], [i.converged for i in infos]
+
+
+@pytest.mark.parametrize("n,K", [(1, 3), (1000, 64), (1025, 1), (5000, 13), (40000, 7), (60000, 9),
+                                 (262144, 2)])
+@pytest.mark.parametrize("opts", [dict(ortho=P.CGS2), dict(ortho=P.CGS1, restart=8, diag_scale=1),
+                                  dict(ortho=P.CGS1, precision=P.F32),
+                                  dict(ortho=P.CGS2, precision=P.BF16, restart=17)])
+def test_batch_persistent_and_launches(n, K, opts):
+    """Column by column the persistent form reaches the residual that the
+    launches reach, in as many steps up to one (their dots are added in other
+    groups, so a residual at the stopping bound may fall on either side), a
+    column's bits do not depend on the other columns, and with a start
+    vector.  The last column is zero."""
+    print("batch n=%d K=%d %s" % (n, K, opts), flush=True)
+    csr = _line(n, 7, n + K)
+    A = P.Matrix.from_csr(n, n, *csr)
+    Bh = np.random.default_rng(n).standard_normal((n, K))
+    if K > 1:
+        Bh[:, -1] = 0.0
+    B = torch.as_tensor(Bh, device=DEV)
+    for x0 in (None, torch.as_tensor(np.random.default_rng(1).standard_normal((n, K)), device=DEV)):
+        X, its, done = _batch(A, B, x0, 1, **opts)
+        Y, ref, _ = _batch(A, B, x0, 0, **opts)
+        assert all(done) and max(abs(a - b) for a, b in zip(its, ref)) <= 1, (its, ref)
+        for q in range(K):
+            x = np.ascontiguousarray(X[:, q].cpu().numpy())
+            scale = np.linalg.norm(Bh[:, q]) or 1.0
+            assert np.linalg.norm(Bh[:, q] - O.spmv(*csr, x)) <= 1.001e-10 * scale, q
+        # both forms' errors are at most ||A^-1|| times the stopping residual,
+        # and the diagonal is at least 3 x what the inverse's bound 1 / (0.5 s) needs
+        assert float((X - Y).norm()) <= 1e-8 * max(1.0, float(Y.norm()))
+        some = [0, K - 1] if K > 1 else [0]
+        Z, _, _ = _batch(A, B[:, some].contiguous(), None if x0 is None else
+                         x0[:, some].contiguous(), 1, **opts)
+        for i, q in enumerate(some):
+            assert torch.equal(Z[:, i], X[:, q]), q
+    A.close()
