@@ -59,6 +59,8 @@ struct GmresState {
     double hcol[GM_MAXM];         // Hessenberg column of the step
     double beta, bnorm, rel, hn, rtol, inner_rtol;
     int m, active, k, iters, iters0, max_iters, converged, cycles;
+    const double* b;  // the caller's arrays: one captured cycle serves them all
+    double* x;
 };
 
 struct GmresWork {
@@ -73,7 +75,7 @@ struct GmresWork {
     // captured restart cycle
     hipStream_t cap = nullptr;
     hipGraphExec_t exec = nullptr;
-    const void* key[4] = {nullptr, nullptr, nullptr, nullptr};
+    const void* key[2] = {nullptr, nullptr};
     int key_m = 0, key_ortho = -1;
     ~GmresWork()
     {
@@ -144,11 +146,11 @@ __device__ __forceinline__ VT basis_at(const VT* V, size_t ldv, int i, int row)
 template <typename VT>
 __global__ void __launch_bounds__(KR_BS)
 k_residual(int n, int R, int width, const int* __restrict__ col, const double* __restrict__ val,
-           const double* __restrict__ b, const double* __restrict__ x, VT* __restrict__ W0, int S,
-           double* __restrict__ part, const GmresState* __restrict__ st)
+           VT* __restrict__ W0, int S, double* __restrict__ part, const GmresState* __restrict__ st)
 {
     __shared__ double sh[KR_BS / 64][GM_MAXM + 1];
     if (st->converged) return;
+    const double *b = st->b, *x = st->x;
     const int base = lblock() * KR_BS * R + threadIdx.x;
     double a = 0.0;
     for (int r = 0; r < R; ++r) {
@@ -436,8 +438,7 @@ k_solve_y(GmresState* __restrict__ st)
 // x += sum_i y_i v_i, accumulated in FP64.
 template <typename VT>
 __global__ void __launch_bounds__(KR_BS)
-k_xupdate(int n, const VT* __restrict__ V, size_t ldv, double* __restrict__ x,
-          const GmresState* __restrict__ st)
+k_xupdate(int n, const VT* __restrict__ V, size_t ldv, const GmresState* __restrict__ st)
 {
     __shared__ double ys[GM_MAXM];
     if (st->converged) return;
@@ -457,7 +458,7 @@ k_xupdate(int n, const VT* __restrict__ V, size_t ldv, double* __restrict__ x,
         for (int q = 0; q < 8; ++q) s = fma(to_d(v[q]), ys[i + q], s);
     }
     for (; i < k; ++i) s = fma(to_d(V[(size_t)i * ldv + row]), ys[i], s);
-    x[row] += s;
+    st->x[row] += s;
 }
 
 __global__ void k_fill0(int n, double* __restrict__ x)
@@ -558,8 +559,7 @@ void update(const Ell<MT>& E, GmresWork* w, VT* dst, int j, bool dots, bool norm
 }
 
 template <typename VT, typename MT>
-void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* b, double* x,
-                   int m, bool cgs, hipStream_t s)
+void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, bool cgs, hipStream_t s)
 {
     const int n = w->n, G = w->G, S = w->S;
     const size_t ldv = w->ldv;
@@ -588,9 +588,9 @@ void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double
     }
     hipLaunchKernelGGL(k_solve_y, one, dim3(64), 0, s, st);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_xupdate<VT>), dim3((n + KR_BS - 1) / KR_BS), block, 0, s,
-                       n, V, ldv, x, st);
+                       n, V, ldv, st);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual<VT>), grid, block, 0, s, n, w->R, A->ell64.width,
-                       A->ell64.col.p, A->ell64.val.p, b, x, W0, S, part, st);
+                       A->ell64.col.p, A->ell64.val.p, W0, S, part, st);
     hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, mgs, 0, 0, 1, S, part, G, st);
 }
 
@@ -614,12 +614,14 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
     init.rtol = o.rtol;
     init.inner_rtol = (o.precision == PHG_F64) ? 0.0 : o.inner_rtol;
     init.max_iters = o.max_iters;
+    init.b = b;
+    init.x = x;
     PHG_HIP(hipMemcpyAsync(st, &init, sizeof init, hipMemcpyHostToDevice, s));
     if (!o.use_x0) hipLaunchKernelGGL(k_fill0, dim3((n + 255) / 256), dim3(256), 0, s, n, x);
     hipLaunchKernelGGL(k_sumsq, grid, block, 0, s, n, w->R, b, S, part);
     hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_BNORM, 0, 0, 0, 1, S, part, G, st);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual<VT>), grid, block, 0, s, n, w->R, A->ell64.width,
-                       A->ell64.col.p, A->ell64.val.p, b, x, W0, S, part, st);
+                       A->ell64.col.p, A->ell64.val.p, W0, S, part, st);
     hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, 0, 0, 0, 1, S, part, G, st);
     PHG_HIP(hipGetLastError());
 
@@ -627,7 +629,7 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
     bool graph_ready = false;
     if (o.graph) {
         graph_ready = true;
-        const void* key[4] = {b, x, E.val.p, A->ell64.val.p};
+        const void* key[2] = {E.val.p, A->ell64.val.p};
         const bool same = w->exec && w->key_m == m && w->key_ortho == o.ortho &&
                           !memcmp(key, w->key, sizeof key);
         if (!same) {
@@ -646,7 +648,7 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
             }
             hipGraph_t g = nullptr;
             PHG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-            enqueue_cycle<VT, MT>(A, E, w, b, x, m, cgs, cs);
+            enqueue_cycle<VT, MT>(A, E, w, m, cgs, cs);
             PHG_HIP(hipStreamEndCapture(cs, &g));
             hipError_t e = hipGraphInstantiate(&w->exec, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
@@ -665,7 +667,7 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
         if (graph_ready) {
             PHG_HIP(hipGraphLaunch(w->exec, s));
         } else {
-            enqueue_cycle<VT, MT>(A, E, w, b, x, m, cgs, s);
+            enqueue_cycle<VT, MT>(A, E, w, m, cgs, s);
             PHG_HIP(hipGetLastError());
         }
     }

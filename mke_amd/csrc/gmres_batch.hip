@@ -71,6 +71,14 @@ struct BSum {
     int active, converged, iters, cycles;
 };
 
+// The caller's arrays, read by the kernels of the captured cycle: a graph
+// serves every pair of them (capturing one again takes 2 ms and more, as long
+// as a whole preconditioned solve at level 7).
+struct BIo {
+    const double* B;
+    double* X;
+};
+
 struct BatchWork {
     int n = 0, m = 0, kp = 0, G = 0, prec = 0, rpt = 0;
     DevBuf<char> V, W;    // (m+1) x n x kp and 2 x n x kp of the Krylov type
@@ -78,6 +86,7 @@ struct BatchWork {
     DevBuf<double> part;  // (m+2) x kp x G block partials
     DevBuf<BCol> cols;    // kp
     DevBuf<BSum> sum;     // kp
+    DevBuf<BIo> io;
     BSum* host = nullptr;
     DevBuf<int> nact;      // columns still running in the current cycle
     int* hnact = nullptr;  // its host copy (pinned)
@@ -85,7 +94,7 @@ struct BatchWork {
     // one graph per chunk of Arnoldi steps of a cycle, then the cycle's end
     hipGraphExec_t exec[BB_NCHUNK + 1] = {};
     bool captured = false;
-    const void* key[4] = {nullptr, nullptr, nullptr, nullptr};
+    const void* key[2] = {nullptr, nullptr};
     int key_m = 0, key_ortho = -1, key_k = 0, key_maxit = 0;
     const void* key_pc = nullptr;
     double key_rtol = 0.0, key_inner = 0.0;
@@ -644,7 +653,7 @@ bk_solve_y(int K, BCol* __restrict__ cols)
 // diagonal right preconditioner); X is n x K (the caller's layout).
 template <typename VT, int RPT>
 __global__ void __launch_bounds__(BB_BS)
-bk_xupdate(int n, int KP, int K, const VT* __restrict__ V, size_t bs, double* __restrict__ X,
+bk_xupdate(int n, int KP, int K, const VT* __restrict__ V, size_t bs, const BIo* __restrict__ io,
            const BCol* __restrict__ cols, const double* __restrict__ dscale)
 {
     const int q = threadIdx.x & (KP - 1);
@@ -654,6 +663,7 @@ bk_xupdate(int n, int KP, int K, const VT* __restrict__ V, size_t bs, double* __
     const BCol* c = cols + q;
     const int k = c->k;
     if (c->converged || k == 0) return;
+    double* __restrict__ X = io->X;
     for (int t = 0; t < RPT; ++t) {
         const int row = base + t * RB;
         if (row >= n) break;
@@ -667,10 +677,11 @@ bk_xupdate(int n, int KP, int K, const VT* __restrict__ V, size_t bs, double* __
 template <typename VT, int RPT>
 __global__ void __launch_bounds__(BB_BS)
 bk_residual(int n, int KP, int K, int width, const int* __restrict__ col,
-            const double* __restrict__ val, const double* __restrict__ B,
-            const double* __restrict__ X, VT* __restrict__ W0, double* __restrict__ part, int G,
-            const BCol* __restrict__ cols)
+            const double* __restrict__ val, const BIo* __restrict__ io, VT* __restrict__ W0,
+            double* __restrict__ part, int G, const BCol* __restrict__ cols)
 {
+    const double* __restrict__ B = io->B;
+    const double* __restrict__ X = io->X;
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
     const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
@@ -730,8 +741,9 @@ bk_sumsq(int n, int KP, int K, const double* __restrict__ B, double* __restrict_
 }
 
 __global__ void bk_set_bnorm(int KP, int K, const double* __restrict__ part, int G,
-                             BCol* __restrict__ cols)
+                             BCol* __restrict__ cols, BIo arrays, BIo* __restrict__ io)
 {
+    if (lblock() == 0 && threadIdx.x == 0) *io = arrays;
     const int q = lblock() * (BB_BS / 64) + ((int)threadIdx.x >> 6);
     if (q >= K) return;
     const double s = wave_sum_partials(part + (size_t)q * G, G);
@@ -854,6 +866,7 @@ int prepare_batch(phg_matrix_s* A, int slot, int prec, int m, int kp, int rpt, b
         PHG_HIP(b->part.alloc((size_t)(m + 2) * kp * blocks_for(n, kp, 1)));
         PHG_HIP(b->cols.alloc(kp));
         PHG_HIP(b->sum.alloc(kp));
+        PHG_HIP(b->io.alloc(1));
         PHG_HIP(hipHostMalloc((void**)&b->host, sizeof(BSum) * kp, hipHostMallocDefault));
         PHG_HIP(b->nact.alloc(1));
         PHG_HIP(hipHostMalloc((void**)&b->hnact, sizeof(int), hipHostMallocDefault));
@@ -933,9 +946,8 @@ void enqueue_batch_steps(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K,
 // The end of a cycle: y, the x update, the true residual and the next
 // cycle's start (the host summary).
 template <typename VT, typename MT, int RPT>
-void enqueue_batch_finish(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K,
-                          const double* B, double* X, double rtol, int max_iters,
-                          BatchPrecond* pc, hipStream_t s)
+void enqueue_batch_finish(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, double rtol,
+                          int max_iters, BatchPrecond* pc, hipStream_t s)
 {
     const int n = w->n, KP = w->kp, G = w->G;
     const size_t bs = (size_t)n * KP;
@@ -947,11 +959,11 @@ void enqueue_batch_finish(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K
     const int cb = (K + 3) / 4;
     hipLaunchKernelGGL(bk_solve_y, dim3(cb), block, 0, s, K, cols);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_xupdate<VT, RPT>), grid, block, 0, s, n, KP, K,
-                       pc ? (const VT*)w->Z.p : (const VT*)V, bs, X, cols,
+                       pc ? (const VT*)w->Z.p : (const VT*)V, bs, w->io.p, cols,
                        (!pc && (const void*)E.val.p == (const void*)A->ell64d.val.p)
                            ? A->dinv.p : (const double*)nullptr);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT, RPT>), grid, block, 0, s, n, KP, K,
-                       A->ell64.width, A->ell64.col.p, A->ell64.val.p, B, X, W0, part, G, cols);
+                       A->ell64.width, A->ell64.col.p, A->ell64.val.p, w->io.p, W0, part, G, cols);
     hipLaunchKernelGGL(bk_cycle_start, dim3(cb), block, 0, s, KP, K, part, G, cols, w->sum.p,
                        rtol, max_iters);
 }
@@ -976,9 +988,10 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
         hipLaunchKernelGGL(bk_fill0, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, tot, X);
     }
     hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_sumsq<RPT>), grid, block, 0, s, n, KP, K, B, part, G);
-    hipLaunchKernelGGL(bk_set_bnorm, dim3(cb), block, 0, s, KP, K, part, G, cols);
+    hipLaunchKernelGGL(bk_set_bnorm, dim3(cb), block, 0, s, KP, K, part, G, cols,
+                       BIo{B, X}, w->io.p);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT, RPT>), grid, block, 0, s, n, KP, K,
-                       A->ell64.width, A->ell64.col.p, A->ell64.val.p, B, X, W0, part, G, cols);
+                       A->ell64.width, A->ell64.col.p, A->ell64.val.p, w->io.p, W0, part, G, cols);
     hipLaunchKernelGGL(bk_cycle_start, dim3(cb), block, 0, s, KP, K, part, G, cols, w->sum.p,
                        o.rtol, o.max_iters);
     PHG_HIP(hipGetLastError());
@@ -988,7 +1001,7 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
     auto chunk_lo = [&](int c) { return c == 0 ? 0 : std::min(m, bb_chunk_end(c - 1)); };
     auto chunk_hi = [&](int c) { return c == nch - 1 ? m : std::min(m, bb_chunk_end(c)); };
     if (o.graph) {
-        const void* key[4] = {B, X, E.val.p, A->ell64.val.p};
+        const void* key[2] = {E.val.p, A->ell64.val.p};
         const bool same = w->captured && w->key_m == m && w->key_ortho == o.ortho &&
                           w->key_k == K && w->key_rtol == o.rtol && w->key_inner == inner &&
                           w->key_maxit == o.max_iters && w->key_pc == (const void*)pc &&
@@ -1010,8 +1023,7 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
                                                      passes, o.rtol, inner, o.max_iters, pc,
                                                      cs);
                 else
-                    enqueue_batch_finish<VT, MT, RPT>(A, E, w, K, B, X, o.rtol, o.max_iters, pc,
-                                                      cs);
+                    enqueue_batch_finish<VT, MT, RPT>(A, E, w, K, o.rtol, o.max_iters, pc, cs);
                 PHG_HIP(hipStreamEndCapture(cs, &g));
                 hipError_t e = hipGraphInstantiate(&w->exec[c], g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
@@ -1051,7 +1063,7 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
         if (o.graph) {
             PHG_HIP(hipGraphLaunch(w->exec[nch], s));
         } else {
-            enqueue_batch_finish<VT, MT, RPT>(A, E, w, K, B, X, o.rtol, o.max_iters, pc, s);
+            enqueue_batch_finish<VT, MT, RPT>(A, E, w, K, o.rtol, o.max_iters, pc, s);
             PHG_HIP(hipGetLastError());
         }
     }
