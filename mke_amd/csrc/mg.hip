@@ -34,6 +34,7 @@ using namespace phg;
 
 namespace {
 constexpr int MG_COARSE = 2;
+constexpr int MG_FUSE = 8;  // most columns (a power of two, 8 lanes each in a wavefront)
 constexpr double MG_OMEGA = 0.8;
 }  // namespace
 
@@ -85,6 +86,39 @@ struct phg_mg_s {
 
 namespace {
 
+// An ELL row's columns and values, loaded without a branch (past the width
+// the last slot again), and its product with x in slot order.
+template <typename T, typename MT>
+struct MgRow {
+    int c[ELL_MAXW];
+    T v[ELL_MAXW];
+    __device__ __forceinline__ void load(int n, int width, int row, const int* __restrict__ col,
+                                         const MT* __restrict__ val)
+    {
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) {
+            const size_t o = ell_slot(k, width, n, row);
+            c[k] = col[o];
+            v[k] = (T)val[o];
+        }
+    }
+    // x(k): the entry that slot k multiplies
+    template <typename F>
+    __device__ __forceinline__ T dot(int width, F x) const
+    {
+        T xv[ELL_MAXW];
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) xv[k] = x(c[k]);
+        T s = T(0);
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) {
+            const T t = s + v[k] * xv[k];
+            s = k < width ? t : s;
+        }
+        return s;
+    }
+};
+
 // The V-cycle kernels in the vector type T (double, or float for the
 // mixed-precision form) over matrix values MT.
 template <typename T, typename MT>
@@ -96,24 +130,10 @@ __global__ void mg_jacobi(int n, int KP, int width, const int* __restrict__ col,
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= (size_t)n * KP) return;
     const int row = (int)(e / KP), q = (int)(e % KP);
-    T s = T(0), x = T(0);
-    if (xin) {
-        int c[ELL_MAXW];
-        T v[ELL_MAXW], xv[ELL_MAXW];
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) {
-            const size_t o = (size_t)k * n + row;
-            c[k] = k < width ? col[o] : 0;
-            v[k] = k < width ? (T)val[o] : T(0);
-        }
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) xv[k] = k < width ? xin[(size_t)c[k] * KP + q] : T(0);
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k)
-            if (k < width) s += v[k] * xv[k];
-        x = xin[e];
-    }
-    xout[e] = x + w * dinv[row] * (b[e] - s);
+    MgRow<T, MT> r;
+    r.load(n, width, row, col, val);
+    const T s = r.dot(width, [&](int j) { return xin[(size_t)j * KP + q]; });
+    xout[e] = xin[e] + w * dinv[row] * (b[e] - s);
 }
 
 template <typename T, typename MT>
@@ -124,21 +144,9 @@ __global__ void mg_residual(int n, int KP, int width, const int* __restrict__ co
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= (size_t)n * KP) return;
     const int row = (int)(e / KP), q = (int)(e % KP);
-    int c[ELL_MAXW];
-    T v[ELL_MAXW], xv[ELL_MAXW];
-#pragma unroll
-    for (int k = 0; k < ELL_MAXW; ++k) {
-        const size_t o = (size_t)k * n + row;
-        c[k] = k < width ? col[o] : 0;
-        v[k] = k < width ? (T)val[o] : T(0);
-    }
-#pragma unroll
-    for (int k = 0; k < ELL_MAXW; ++k) xv[k] = k < width ? x[(size_t)c[k] * KP + q] : T(0);
-    T s = T(0);
-#pragma unroll
-    for (int k = 0; k < ELL_MAXW; ++k)
-        if (k < width) s += v[k] * xv[k];
-    r[e] = b[e] - s;
+    MgRow<T, MT> a;
+    a.load(n, width, row, col, val);
+    r[e] = b[e] - a.dot(width, [&](int j) { return x[(size_t)j * KP + q]; });
 }
 
 template <typename T>
@@ -167,6 +175,215 @@ __global__ void mg_prolong_add(int nf, int KP, const int* __restrict__ p0,
     if (c == -2) v = a >= 0 ? xc[(size_t)a * KP + q] : T(0);  // the vertex itself
     else v = T(0.5) * ((a >= 0 ? xc[(size_t)a * KP + q] : T(0)) + (c >= 0 ? xc[(size_t)c * KP + q] : T(0)));
     xf[e] += v;
+}
+
+// Both Jacobi sweeps from x = 0 in one launch: the first one's value of a
+// neighbour is w d b, formed where it is gathered (the same operations as
+// two launches of mg_jacobi: the same bits).
+template <typename T, typename MT>
+__global__ void mg_jacobi_zero2(int n, int KP, int width, const int* __restrict__ col,
+                                const MT* __restrict__ val, const T* __restrict__ dinv,
+                                const T* __restrict__ b, T* __restrict__ xout, T w)
+{
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (size_t)n * KP) return;
+    const int row = (int)(e / KP), q = (int)(e % KP);
+    MgRow<T, MT> r;
+    r.load(n, width, row, col, val);
+    const T d = w * dinv[row], be = b[e];
+    const T s = r.dot(width, [&](int j) { return w * dinv[j] * b[(size_t)j * KP + q]; });
+    xout[e] = d * be + d * (be - s);
+}
+
+// The restriction of the residual, for up to MG_FUSE columns: eight lanes per
+// coarse row and column take the residuals of its (at most eight) fine rows,
+// which are then added in order.  A fine row's residual is formed in up to
+// two places (1.75 times the work), which costs less than the launch and
+// the pass over memory it saves: level 7, one column, 8.0 us as two launches.
+template <typename T, typename MT>
+__global__ void mg_residual_restrict(int nc, int nf, int KP, int width, const int* __restrict__ col,
+                                     const MT* __restrict__ val, const T* __restrict__ x,
+                                     const T* __restrict__ b, const int* __restrict__ rrp,
+                                     const int* __restrict__ ridx, const T* __restrict__ rw,
+                                     T* __restrict__ bc)
+{
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int q = (int)(e % KP), t = (int)(e / KP) & 7;
+    const size_t j = e / KP / 8;
+    int cnt = 0;
+    T v = T(0);
+    if (j < (size_t)nc) {
+        const int lo = rrp[j];
+        cnt = rrp[j + 1] - lo;
+        if (t < cnt) {
+            const int i = ridx[lo + t];
+            MgRow<T, MT> r;
+            r.load(nf, width, i, col, val);
+            const T s = r.dot(width, [&](int k) { return x[(size_t)k * KP + q]; });
+            v = rw[lo + t] * (b[(size_t)i * KP + q] - s);
+        }
+    }
+    const int lane = threadIdx.x & 63, first = lane - t * KP;
+    T s = T(0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const T u = s + __shfl(v, first + k * KP, 64);
+        s = k < cnt ? u : s;
+    }
+    if (t == 0 && j < (size_t)nc) bc[j * KP + q] = s;
+}
+
+// x_j with the coarse correction added (as mg_prolong_add adds it)
+template <typename T>
+__device__ __forceinline__ T mg_corrected(T xj, int a, int c, T xa, T xc)
+{
+    const T va = a >= 0 ? xa : T(0), vc = c >= 0 ? xc : T(0);
+    return xj + (c == -2 ? va : T(0.5) * (va + vc));
+}
+
+// The coarse correction and the Jacobi sweep after it in one launch, for up
+// to MG_FUSE columns: a neighbour's corrected value is formed where it is
+// gathered.
+template <typename T, typename MT>
+__global__ void mg_prolong_jacobi(int n, int KP, int width, const int* __restrict__ col,
+                                  const MT* __restrict__ val, const T* __restrict__ dinv,
+                                  const int* __restrict__ p0, const int* __restrict__ p1,
+                                  const T* __restrict__ xc, const T* __restrict__ x,
+                                  const T* __restrict__ b, T* __restrict__ xout, T w)
+{
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (size_t)n * KP) return;
+    const int row = (int)(e / KP), q = (int)(e % KP);
+    MgRow<T, MT> r;
+    r.load(n, width, row, col, val);
+    const auto at = [&](int j) {
+        const int a = p0[j], c = p1[j];
+        return mg_corrected(x[(size_t)j * KP + q], a, c, xc[(size_t)max(a, 0) * KP + q],
+                            xc[(size_t)max(c, 0) * KP + q]);
+    };
+    const T s = r.dot(width, at);
+    xout[e] = at(row) + w * dinv[row] * (b[e] - s);
+}
+
+// ---- the coarse levels in one launch ------------------------------------
+// One workgroup per column takes the V-cycle from level 3 down to the dense
+// inverse of level 2 and back: a sweep ends at a barrier instead of a launch,
+// the vectors are in LDS, and everything the workgroup reads (54 KB and the
+// inverse's 207 KB in FP64) is loaded into registers before the first sweep,
+// in one round trip.  Bound by that load: one CU takes some 27 GB/s from
+// beyond its L2.  So level 4 (215 KB) is not part of it: with it, and loads
+// where they are used, the launch took 43 us.
+constexpr int MGC_BS = 704;
+constexpr int MGC_N3 = 641, MGC_N2 = 161;  // rows of levels 3 and 2
+
+template <typename T, typename MT>
+struct MgcLevel {
+    int n, width;
+    const int* col;
+    const MT* val;
+    const T* dinv;
+    const int *p0, *p1, *rrp, *ridx;
+    const T* rw;
+};
+
+// Row threadIdx.x of a level's operator and prolongation, and row threadIdx.x
+// of its restriction (nc rows of at most eight entries).
+template <typename T, typename MT>
+struct MgcRows {
+    MgRow<T, MT> row;
+    T d, rw[8];
+    int n, width, nc, p0, p1, cnt, ri[8];
+    __device__ __forceinline__ void load(const MgcLevel<T, MT>& l, int nc_, T w)
+    {
+        n = l.n, width = l.width, nc = nc_;
+        const int i = min((int)threadIdx.x, n - 1), j = min((int)threadIdx.x, nc - 1);
+        const int lo = l.rrp[j];
+        cnt = l.rrp[j + 1] - lo;
+        row.load(n, width, i, l.col, l.val);
+        d = w * l.dinv[i];
+        p0 = l.p0[i], p1 = l.p1[i];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int o = lo + min(k, cnt - 1);
+            ri[k] = l.ridx[o];
+            rw[k] = l.rw[o];
+        }
+    }
+    __device__ __forceinline__ T dot(const T* x) const
+    {
+        return row.dot(width, [&](int j) { return x[j]; });
+    }
+    // two sweeps from zero, the residual (left in y) and its restriction to bc
+    __device__ __forceinline__ void down(T* x, T* y, const T* b, T* bc) const
+    {
+        const int i = threadIdx.x;
+        if (i < n) y[i] = d * b[i];
+        __syncthreads();
+        if (i < n) x[i] = y[i] + d * (b[i] - dot(y));
+        __syncthreads();
+        if (i < n) y[i] = b[i] - dot(x);
+        __syncthreads();
+        if (i < nc) {
+            T s = T(0);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const T u = s + rw[k] * y[ri[k]];
+                s = k < cnt ? u : s;
+            }
+            bc[i] = s;
+        }
+        __syncthreads();
+    }
+    // the coarse correction xc and two sweeps
+    __device__ __forceinline__ void up(T* x, T* y, const T* b, const T* xc) const
+    {
+        const int i = threadIdx.x;
+        if (i < n) x[i] = mg_corrected(x[i], p0, p1, xc[max(p0, 0)], xc[max(p1, 0)]);
+        __syncthreads();
+        if (i < n) y[i] = x[i] + d * (b[i] - dot(x));
+        __syncthreads();
+        if (i < n) x[i] = y[i] + d * (b[i] - dot(y));
+        __syncthreads();
+    }
+};
+
+// x = V-cycle(b) of level 3 over the dense inverse of level 2 (nc rows);
+// column blockIdx.x of n x KP arrays.
+template <typename T, typename MT>
+__global__ void __launch_bounds__(MGC_BS)
+mg_coarse(MgcLevel<T, MT> l3, int nc, const T* __restrict__ cinv, int KP,
+          const T* __restrict__ bin, T* __restrict__ xout, T w)
+{
+    __shared__ T x3[MGC_N3], y3[MGC_N3], b3[MGC_N3], x2[MGC_N2], b2[MGC_N2];
+    constexpr int W = MGC_BS / 64, RW = (MGC_N2 + W - 1) / W, CW = (MGC_N2 + 63) / 64;
+    const int q = blockIdx.x, t = threadIdx.x, lane = t & 63;
+    MgcRows<T, MT> m3;
+    m3.load(l3, nc, w);
+    // a wavefront takes every W-th row of the inverse, its lanes the columns
+    T inv[RW][CW];
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+        for (int k = 0; k < CW; ++k)
+            inv[r][k] = cinv[(size_t)min((t >> 6) + r * W, nc - 1) * nc + min(lane + 64 * k, nc - 1)];
+    if (t < l3.n) b3[t] = bin[(size_t)t * KP + q];
+    __syncthreads();
+    m3.down(x3, y3, b3, b2);
+    T bv[CW];
+#pragma unroll
+    for (int k = 0; k < CW; ++k) bv[k] = lane + 64 * k < nc ? b2[min(lane + 64 * k, nc - 1)] : T(0);
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        T a = T(0);
+#pragma unroll
+        for (int k = 0; k < CW; ++k) a += inv[r][k] * bv[k];
+        for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+        const int i = (t >> 6) + r * W;
+        if (lane == 0 && i < nc) x2[i] = a;
+    }
+    __syncthreads();
+    m3.up(x3, y3, b3, x2);
+    if (t < l3.n) xout[(size_t)t * KP + q] = x3[t];
 }
 
 __global__ void mg_to_f32(size_t n, const double* __restrict__ a, float* __restrict__ b)
@@ -314,6 +531,10 @@ int build_transfer(const SphereMesh& f, const SphereMesh& c, MgLevel& fl, int nc
             rw.push_back(e.second);
         }
         rrp[j + 1] = (int)ridx.size();
+        if (rows[j].empty() || rows[j].size() > 8) {
+            set_error("mg: a coarse row takes none or more than eight fine rows");
+            return PHG_ERR_ARG;
+        }
     }
     PHG_HIP(fl.p0.upload(p0.data(), nf));
     PHG_HIP(fl.p1.upload(p1.data(), nf));
@@ -376,7 +597,18 @@ struct MgT<float> {
     static float* cinv(phg_mg_s* M) { return M->cinvf.p; }
 };
 
-// z = V-cycle(v): v, z are n x KP (finest level); enqueued on s.
+template <typename T>
+MgcLevel<T, typename MgT<T>::MT> mgc_level(MgLevel& l)
+{
+    using B = MgT<T>;
+    const auto& E = B::E(l);
+    return {l.n, E.width, E.col.p, E.val.p, B::dinv(l), l.p0.p, l.p1.p, l.rrp.p, l.ridx.p, B::rw(l)};
+}
+
+// z = V-cycle(v): v, z are n x KP (finest level); enqueued on s.  Levels 3
+// and below are one launch; above, a level takes four launches for up to
+// MG_FUSE columns and six for more, where the passes are bound by memory and
+// the recomputation of the fused ones would show.
 template <typename T>
 void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
 {
@@ -384,41 +616,56 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
     using MT = typename B::MT;
     const T om = (T)MG_OMEGA;
     const int nlev = (int)M->lv.size();
+    if (nlev == 1) {  // the dense level alone
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_dense<T>), dim3((unsigned)M->nc), dim3(256), 0, s,
+                           M->nc, KP, B::cinv(M), v, z);
+        return;
+    }
+    const int kc = nlev - 2;  // level 3: with level 2 in one launch
+    const bool fuse = KP <= MG_FUSE && (KP & (KP - 1)) == 0;
     // descend: level 0 takes b = v (read directly), result to z
     const T* bk = v;
-    for (int k = 0; k < nlev - 1; ++k) {
+    for (int k = 0; k < kc; ++k) {
         MgLevel& l = *M->lv[k];
+        MgLevel& c = *M->lv[k + 1];
         const auto& E = B::E(l);
         const size_t w = (size_t)l.n * KP;
         T* xa = (k == 0) ? z : B::x0(l);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
-                           KP, E.width, E.col.p, E.val.p, B::dinv(l), (const T*)nullptr, bk,
-                           B::x1(l), om);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
-                           KP, E.width, E.col.p, E.val.p, B::dinv(l), B::x1(l), bk, xa, om);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
-                           KP, E.width, E.col.p, E.val.p, xa, bk, B::r(l));
-        MgLevel& c = *M->lv[k + 1];
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_restrict<T>), grid_for((size_t)c.n * KP), dim3(256),
-                           0, s, c.n, KP, l.rrp.p, l.ridx.p, B::rw(l), B::r(l), B::b(c));
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi_zero2<T, MT>), grid_for(w), dim3(256), 0, s,
+                           l.n, KP, E.width, E.col.p, E.val.p, B::dinv(l), bk, xa, om);
+        if (fuse) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual_restrict<T, MT>),
+                               grid_for((size_t)c.n * KP * 8), dim3(256), 0, s, c.n, l.n, KP, E.width,
+                               E.col.p, E.val.p, xa, bk, l.rrp.p, l.ridx.p, B::rw(l), B::b(c));
+        } else {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual<T, MT>), grid_for(w), dim3(256), 0, s,
+                               l.n, KP, E.width, E.col.p, E.val.p, xa, bk, B::r(l));
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_restrict<T>), grid_for((size_t)c.n * KP), dim3(256),
+                               0, s, c.n, KP, l.rrp.p, l.ridx.p, B::rw(l), B::r(l), B::b(c));
+        }
         bk = B::b(c);
     }
-    MgLevel& cl = *M->lv[nlev - 1];
-    T* xcoarse = (nlev == 1) ? z : B::x0(cl);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_dense<T>), dim3((unsigned)M->nc), dim3(256), 0, s, M->nc,
-                       KP, B::cinv(M), bk, xcoarse);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_coarse<T, MT>), dim3(KP), dim3(MGC_BS), 0, s,
+                       mgc_level<T>(*M->lv[kc]), M->nc, B::cinv(M), KP, bk,
+                       kc == 0 ? z : B::x0(*M->lv[kc]), om);
     // ascend
-    for (int k = nlev - 2; k >= 0; --k) {
+    for (int k = kc - 1; k >= 0; --k) {
         MgLevel& l = *M->lv[k];
         MgLevel& c = *M->lv[k + 1];
         const auto& E = B::E(l);
         const size_t w = (size_t)l.n * KP;
         const T* bl = (k == 0) ? v : B::b(l);
         T* xa = (k == 0) ? z : B::x0(l);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_add<T>), grid_for(w), dim3(256), 0, s, l.n, KP,
-                           l.p0.p, l.p1.p, B::x0(c), xa);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
-                           KP, E.width, E.col.p, E.val.p, B::dinv(l), xa, bl, B::x1(l), om);
+        if (fuse) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_jacobi<T, MT>), grid_for(w), dim3(256), 0,
+                               s, l.n, KP, E.width, E.col.p, E.val.p, B::dinv(l), l.p0.p, l.p1.p,
+                               B::x0(c), xa, bl, B::x1(l), om);
+        } else {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_add<T>), grid_for(w), dim3(256), 0, s, l.n,
+                               KP, l.p0.p, l.p1.p, B::x0(c), xa);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
+                               KP, E.width, E.col.p, E.val.p, B::dinv(l), xa, bl, B::x1(l), om);
+        }
         hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
                            KP, E.width, E.col.p, E.val.p, B::dinv(l), B::x1(l), bl, xa, om);
     }
