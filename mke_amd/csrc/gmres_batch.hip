@@ -34,6 +34,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 #include "ell.h"
 #include "persist.h"
@@ -45,7 +46,6 @@ constexpr int BB_BS = 256;
 constexpr int BB_MAXM = 32;
 constexpr int BB_MAXK = 64;
 constexpr int BB_RPT = 16;  // largest rows per thread of a launch shape
-constexpr int BB_LB = 4;   // basis vectors per load batch
 
 // A restart cycle runs its Arnoldi steps in chunks ending at steps 4, 8, 16,
 // 24 and 32; after each chunk but the last the host reads how many columns
@@ -158,79 +158,7 @@ __device__ __forceinline__ double readlane_d(double v, int lane)
 template <typename T>
 __device__ __forceinline__ double dd(T v) { return (double)v; }
 
-// Row of A times column q of X (n x KP), source scaled by s: FP64 without
-// fused multiply-add, or FP32 with fma over FP32/BF16 values.
-template <typename VT, typename MT>
-struct BRow;
-template <>
-struct BRow<double, double> {
-    __device__ __forceinline__ static double run(int n, int width, int row,
-                                                 const int* __restrict__ col,
-                                                 const double* __restrict__ val,
-                                                 const double* __restrict__ X, int KP, int q,
-                                                 double s)
-    {
-        if (width > ELL_MAXW) {  // long rows (block systems): the same sum, not unrolled
-            double r = 0.0;
-            for (int k = 0; k < width; ++k) {
-                const size_t o = (size_t)k * n + row;
-                r += val[o] * (X[(size_t)col[o] * KP + q] * s);
-            }
-            return r;
-        }
-        int c[ELL_MAXW];
-        double v[ELL_MAXW], xv[ELL_MAXW];
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) {
-            const size_t o = (size_t)k * n + row;
-            c[k] = k < width ? col[o] : 0;
-            v[k] = k < width ? val[o] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) xv[k] = k < width ? X[(size_t)c[k] * KP + q] : 0.0;
-        double r = 0.0;
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k)
-            if (k < width) r += v[k] * (xv[k] * s);
-        return r;
-    }
-};
-template <typename MT>
-struct BRow<float, MT> {
-    __device__ __forceinline__ static float run(int n, int width, int row,
-                                                const int* __restrict__ col,
-                                                const MT* __restrict__ val,
-                                                const float* __restrict__ X, int KP, int q,
-                                                float s)
-    {
-        if (width > ELL_MAXW) {
-            float r = 0.0f;
-            for (int k = 0; k < width; ++k) {
-                const size_t o = (size_t)k * n + row;
-                r = fmaf(ell_val_f32(val[o]), X[(size_t)col[o] * KP + q] * s, r);
-            }
-            return r;
-        }
-        int c[ELL_MAXW];
-        MT v[ELL_MAXW];
-        float xv[ELL_MAXW];
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) {
-            const size_t o = (size_t)k * n + row;
-            c[k] = k < width ? col[o] : 0;
-            v[k] = k < width ? val[o] : MT(0);
-        }
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) xv[k] = k < width ? X[(size_t)c[k] * KP + q] : 0.0f;
-        float r = 0.0f;
-#pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k)
-            if (k < width) r = fmaf(ell_val_f32(v[k]), xv[k] * s, r);
-        return r;
-    }
-};
-
-// One term of BRow's sum: r + val * (x * s) in FP64 (no fused multiply-add),
+// One term of a row's sum: r + val * (x * s) in FP64 (no fused multiply-add),
 // fmaf(val, x * s, r) in FP32.
 template <typename VT, typename MT>
 struct BTerm;
@@ -249,13 +177,80 @@ struct BTerm<float, MT> {
     }
 };
 
-// BRow of this thread's rows base + t * RB (t < RPT) of column q, and xo[t]
+// Row `row` of A times column q of X (row-major, ldx columns), X scaled by s.
+// For rows of at most ELL_MAXW entries all slots are loaded first (past the
+// width the last one again, in bounds), then all gathers.
+template <typename VT, typename MT>
+__device__ __forceinline__ VT brow(int n, int width, int row, const int* __restrict__ col,
+                                   const MT* __restrict__ val, const VT* __restrict__ X, int ldx,
+                                   int q, VT s)
+{
+    VT r = VT(0);
+    if (width >= 1 && width <= ELL_MAXW) {
+        int c[ELL_MAXW];
+        MT v[ELL_MAXW];
+        VT xv[ELL_MAXW];
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) {
+            const size_t o = ell_slot(k, width, n, row);
+            c[k] = col[o];
+            v[k] = val[o];
+        }
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) xv[k] = X[(size_t)c[k] * ldx + q];
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) {
+            const VT t = BTerm<VT, MT>::add(r, v[k], xv[k], s);
+            r = k < width ? t : r;
+        }
+    } else {
+        for (int k = 0; k < width; ++k) {
+            const size_t o = (size_t)k * n + row;
+            r = BTerm<VT, MT>::add(r, val[o], X[(size_t)col[o] * ldx + q], s);
+        }
+    }
+    return r;
+}
+
+// A thread's dots acc[i], i <= j (inactive threads: zeros), as block partials
+// part[((out0 + i) * KP + q) * G + block].  All threads of the block call it.
+template <int NV>
+__device__ __forceinline__ void put_partials(const double (&acc)[NV], int last, int KP, int out0,
+                                             double* __restrict__ part, int G)
+{
+    constexpr int LB = NV < 8 ? NV : 8;  // dots per round through LDS
+    __shared__ double sh[BB_BS / 64][LB][BB_MAXK];
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i0 = 0; i0 < NV; i0 += LB) {
+        if (i0 > last) break;
+#pragma unroll
+        for (int u = 0; u < LB; ++u) {
+            const double s = col_wave_sum(acc[i0 + u], KP);
+            if (lane < KP) sh[wid][u][lane] = s;
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < LB * KP; e += BB_BS) {
+            const int u = e / KP, qq = e % KP;
+            if (i0 + u <= last) {
+                double s = 0.0;
+#pragma unroll
+                for (int ww = 0; ww < BB_BS / 64; ++ww) s += sh[ww][u][qq];
+                part[((size_t)(out0 + i0 + u) * KP + qq) * G + lblock()] = s;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// brow of this thread's rows base + t * RB (t < RPT) of column q, and xo[t]
 // = X(row, q); w[t] = xo[t] = 0 for rows at or past n and inactive columns.
 // For rows of at most ELL_MAXW entries, RG rows at a time: every row's own
 // entry and column/value slots (ell_slot: past the width the last slot
 // again, in bounds) are loaded first, then every row's gathers, then the
-// sums in BRow's order; two memory round trips per group instead of three
-// per row.
+// sums in brow's order; two memory round trips per group instead of three
+// per row.  (Scalar loads of the slots, where 64 columns share a row, were
+// slower: 265 instead of 242 us at level 7, FP32.)
 template <typename VT, typename MT, int RPT, int RG>
 __device__ __forceinline__ void brows(int n, int width, int KP, int q, int base, int RB, bool act,
                                       const int* __restrict__ col, const MT* __restrict__ val,
@@ -304,112 +299,84 @@ __device__ __forceinline__ void brows(int n, int width, int KP, int q, int base,
             xo[t] = VT(0);
             if (act && row < n) {
                 xo[t] = X[(size_t)row * KP + q];
-                w[t] = BRow<VT, MT>::run(n, width, row, col, val, X, KP, q, s);
+                w[t] = brow<VT, MT>(n, width, row, col, val, X, KP, q, s);
             }
         }
     }
 }
 
-// Block partials of <V_i, w> for i < nd (i == own_i taken from `own`), or
-// of ||w||^2 when nd == 0, for this thread's rows; written to
-// part[((out0 + i) * KP + q) * G + block].  All threads of the block call it.
+// Partial dots of w with v_0..v_j (v_j from `own` where given) of a thread's
+// rows, V_LB vectors of all its rows at a time.  FP32 loads have no branch
+// between them (past the last vector that one again, unused: steps with few
+// vectors 55 instead of 67 us at level 7 x 64); FP64 ones stop at the last
+// vector (180 instead of 187 us there).  With a test of every row and column
+// before each load the steps with few vectors took 92 us.
+constexpr int V_LB = 4;
 template <typename VT, int RPT>
-__device__ __forceinline__ void bdots(int nd, int own_i, const VT* own, const VT* __restrict__ V,
-                                      size_t bs, int n, int KP, int q, int base, int RB,
-                                      bool act, const VT* w, double* __restrict__ part, int G,
-                                      int out0)
+__device__ __forceinline__ void bdots(int j, const VT* own, const VT* __restrict__ V, size_t bs,
+                                      int n, int KP, int q, int base, int RB, bool act,
+                                      const VT* w, double* __restrict__ part, int G)
 {
-    __shared__ double sh[BB_BS / 64][BB_LB][BB_MAXK];
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int nout = nd == 0 ? 1 : nd;
-    for (int i0 = 0; i0 < nout; i0 += BB_LB) {
-        double acc[BB_LB];
-        if (nd == 0) {
-            double a = 0.0;
+    const int last = own ? max(j - 1, 0) : j;
+    for (int i0 = 0; i0 <= j; i0 += V_LB) {
+        double acc[V_LB];
 #pragma unroll
-            for (int t = 0; t < RPT; ++t) {
-                const int row = base + t * RB;
-                if (act && row < n) a += dd(w[t]) * dd(w[t]);
-            }
-            acc[0] = a;
+        for (int u = 0; u < V_LB; ++u) acc[u] = 0.0;
+        if (act) {
+            VT vb[V_LB][RPT];
 #pragma unroll
-            for (int u = 1; u < BB_LB; ++u) acc[u] = 0.0;
-        } else {
-            VT vb[BB_LB][RPT];
+            for (int u = 0; u < V_LB; ++u)
 #pragma unroll
-            for (int u = 0; u < BB_LB; ++u) {
-                const int i = i0 + u;
+                for (int t = 0; t < RPT; ++t)
+                    vb[u][t] = sizeof(VT) == 4 || i0 + u <= last
+                                   ? V[(size_t)min(i0 + u, last) * bs +
+                                       (size_t)min(base + t * RB, n - 1) * KP + q]
+                                   : VT(0);
 #pragma unroll
-                for (int t = 0; t < RPT; ++t) {
-                    const int row = base + t * RB;
-                    vb[u][t] = (act && i < nd && i != own_i && row < n)
-                                   ? V[(size_t)i * bs + (size_t)row * KP + q] : VT(0);
-                }
-            }
+            for (int u = 0; u < V_LB; ++u)
 #pragma unroll
-            for (int u = 0; u < BB_LB; ++u) {
-                const int i = i0 + u;
-                double a = 0.0;
-#pragma unroll
-                for (int t = 0; t < RPT; ++t) {
-                    const int row = base + t * RB;
-                    if (act && i < nd && row < n) a += dd(w[t]) * dd(i == own_i ? own[t] : vb[u][t]);
-                }
-                acc[u] = a;
-            }
+                for (int t = 0; t < RPT; ++t)
+                    acc[u] += dd(w[t]) * dd(own && i0 + u == j ? own[t] : vb[u][t]);
         }
-#pragma unroll
-        for (int u = 0; u < BB_LB; ++u) {
-            const double s = col_wave_sum(acc[u], KP);
-            if (lane < KP) sh[wid][u][lane] = s;
-        }
-        __syncthreads();
-        for (int e = threadIdx.x; e < BB_LB * KP; e += BB_BS) {
-            const int u = e / KP, qq = e % KP;
-            if (i0 + u < nout) {
-                double s = 0.0;
-#pragma unroll
-                for (int ww = 0; ww < BB_BS / 64; ++ww) s += sh[ww][u][qq];
-                part[((size_t)(out0 + i0 + u) * KP + qq) * G + lblock()] = s;
-            }
-        }
-        __syncthreads();
+        put_partials<V_LB>(acc, j - i0, KP, i0, part, G);
     }
 }
 
 // ---------------------------------------------------------------- kernels --
+// The row kernels: a thread owns RPT (or R) rows base + t * RB of column q.
+//
 // Arnoldi step j: v_j = W_src / h (stored), W_dst = A v_j, partial dots of
-// W_dst with v_0..v_j (first CGS pass).
-template <typename VT, typename MT, int RPT>
+// W_dst with v_0..v_j (first CGS pass).  PC: W_dst = A z_j (X = z_j = M^-1 v_j,
+// the preconditioned vector), v_j has been stored.
+template <typename VT, typename MT, int RPT, bool PC>
 __global__ void __launch_bounds__(BB_BS)
 bk_step_spmm(int n, int KP, int K, int width, const int* __restrict__ col,
-             const MT* __restrict__ val, const VT* __restrict__ Wsrc, VT* __restrict__ V,
-             size_t bs, VT* __restrict__ Wdst, int j, double* __restrict__ part, int G,
+             const MT* __restrict__ val, const VT* __restrict__ X, VT* __restrict__ V, size_t bs,
+             VT* __restrict__ Wdst, int j, double* __restrict__ part, int G,
              const BCol* __restrict__ cols)
 {
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
     const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
     const bool act = q < K && cols[q].active;
-    double h = 1.0;
-    if (act) h = j == 0 ? cols[q].beta : cols[q].hn;
-    const VT inv = (VT)(1.0 / h);
-    VT* Vj = V + (size_t)j * bs;
-    VT w[RPT], vj[RPT], xo[RPT];
-    brows<VT, MT, RPT, (RPT < 4 ? RPT : 4)>(n, width, KP, q, base, RB, act, col, val, Wsrc, inv,
-                                            xo, w);
+    VT w[RPT], vj[RPT];
+    if (act) {
+        const double h = PC ? 1.0 : (j == 0 ? cols[q].beta : cols[q].hn);
+        const VT inv = (VT)(1.0 / h);
+        brows<VT, MT, RPT, (RPT < 4 ? RPT : 4)>(n, width, KP, q, base, RB, act, col, val, X, inv,
+                                                vj, w);
 #pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        vj[t] = VT(0);
-        if (act && row < n) {
-            const size_t o = (size_t)row * KP + q;
-            vj[t] = xo[t] * inv;
-            Vj[o] = vj[t];
-            Wdst[o] = w[t];
+        for (int t = 0; t < RPT; ++t) {
+            const int row = base + t * RB;
+            vj[t] = vj[t] * inv;
+            if (row < n) {
+                const size_t o = (size_t)row * KP + q;
+                if (!PC) V[(size_t)j * bs + o] = vj[t];
+                Wdst[o] = w[t];
+            }
         }
     }
-    bdots<VT, RPT>(j + 1, j, vj, V, bs, n, KP, q, base, RB, act, w, part, G, 0);
+    bdots<VT, RPT>(j, PC ? nullptr : vj, V, bs, n, KP, q, base, RB, act, w, part, G);
 }
 
 // Right-preconditioned step: v_j = W_src / h (stored) for the preconditioner.
@@ -424,30 +391,6 @@ bk_scale(int n, int KP, int K, const VT* __restrict__ Wsrc, VT* __restrict__ Vj,
     if (q >= K || !cols[q].active) return;
     const double h = j == 0 ? cols[q].beta : cols[q].hn;
     Vj[e] = Wsrc[e] * (VT)(1.0 / h);
-}
-
-// W_dst = A z_j (z_j = M^-1 v_j, the preconditioned vector) and the partial
-// dots of W_dst with v_0..v_j.
-template <typename VT, typename MT, int RPT>
-__global__ void __launch_bounds__(BB_BS)
-bk_step_spmm_pc(int n, int KP, int K, int width, const int* __restrict__ col,
-                const MT* __restrict__ val, const VT* __restrict__ Zj, const VT* __restrict__ V,
-                size_t bs, VT* __restrict__ Wdst, int j, double* __restrict__ part, int G,
-                const BCol* __restrict__ cols)
-{
-    const int q = threadIdx.x & (KP - 1);
-    const int RB = BB_BS / KP;
-    const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
-    const bool act = q < K && cols[q].active;
-    VT w[RPT], xo[RPT];
-    brows<VT, MT, RPT, (RPT < 4 ? RPT : 4)>(n, width, KP, q, base, RB, act, col, val, Zj, VT(1),
-                                            xo, w);
-#pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        if (act && row < n) Wdst[(size_t)row * KP + q] = w[t];
-    }
-    bdots<VT, RPT>(j + 1, -1, nullptr, V, bs, n, KP, q, base, RB, act, w, part, G, 0);
 }
 
 // Sums the partials of the nd dots of a pass, one wavefront per (i, column):
@@ -468,112 +411,94 @@ bk_reduce(int KP, int K, int nd, int j, int pass, const double* __restrict__ par
     }
 }
 
-// w -= sum_{i<=j} hc_i v_i, then the partial dots with v_0..v_j (next pass)
-// or the partial of ||w||^2 (final pass).
+// w -= sum_{i<=j} hc_i v_i, then with `norm` the partial of ||w||^2 as value
+// j + 1.  V_LB vectors of all a thread's rows at a time: level 7, 64 columns
+// FP32, 15.5 vectors on average, 148 us, 5.0 TB/s, what a copy reaches here
+// (row by row with all vectors of a row in flight 4.4 TB/s).
 template <typename VT, int RPT>
 __global__ void __launch_bounds__(BB_BS)
 bk_update(int n, int KP, int K, VT* __restrict__ W, const VT* __restrict__ V, size_t bs, int j,
-          int final_pass, double* __restrict__ part, int G, const BCol* __restrict__ cols)
+          int norm, double* __restrict__ part, int G, const BCol* __restrict__ cols)
 {
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
     const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
     const bool act = q < K && cols[q].active;
-    VT w[RPT];
+    double nrm[1] = {0.0};
+    if (act) {
+        VT w[RPT];
 #pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        w[t] = (act && row < n) ? W[(size_t)row * KP + q] : VT(0);
-    }
-    for (int i0 = 0; i0 <= j; i0 += BB_LB) {
-        VT vb[BB_LB][RPT];
-        VT hv[BB_LB];
+        for (int t = 0; t < RPT; ++t) w[t] = W[(size_t)min(base + t * RB, n - 1) * KP + q];
+        for (int i0 = 0; i0 <= j; i0 += V_LB) {
+            VT vb[V_LB][RPT], hv[V_LB];
 #pragma unroll
-        for (int u = 0; u < BB_LB; ++u) {
-            const int i = i0 + u;
-            hv[u] = (act && i <= j) ? (VT)cols[q].hc[i] : VT(0);
+            for (int u = 0; u < V_LB; ++u) {
+                hv[u] = i0 + u <= j ? (VT)cols[q].hc[i0 + u] : VT(0);
 #pragma unroll
-            for (int t = 0; t < RPT; ++t) {
-                const int row = base + t * RB;
-                vb[u][t] = (act && i <= j && row < n) ? V[(size_t)i * bs + (size_t)row * KP + q]
-                                                      : VT(0);
+                for (int t = 0; t < RPT; ++t)
+                    vb[u][t] = i0 + u <= j ? V[(size_t)(i0 + u) * bs +
+                                               (size_t)min(base + t * RB, n - 1) * KP + q]
+                                           : VT(0);
             }
+#pragma unroll
+            for (int u = 0; u < V_LB; ++u)
+#pragma unroll
+                for (int t = 0; t < RPT; ++t) w[t] = w[t] - hv[u] * vb[u][t];
         }
 #pragma unroll
-        for (int u = 0; u < BB_LB; ++u)
-#pragma unroll
-            for (int t = 0; t < RPT; ++t) w[t] = w[t] - hv[u] * vb[u][t];
+        for (int t = 0; t < RPT; ++t) {
+            const int row = base + t * RB;
+            if (row < n) {
+                W[(size_t)row * KP + q] = w[t];
+                nrm[0] += dd(w[t]) * dd(w[t]);
+            }
+        }
     }
-#pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        if (act && row < n) W[(size_t)row * KP + q] = w[t];
-    }
-    if (final_pass) bdots<VT, RPT>(0, -1, nullptr, V, bs, n, KP, q, base, RB, act, w, part, G, j + 1);
-    else bdots<VT, RPT>(j + 1, -1, nullptr, V, bs, n, KP, q, base, RB, act, w, part, G, 0);
+    if (norm) put_partials<1>(nrm, 0, KP, j + 1, part, G);
 }
 
-// First CGS2 pass fused with the dots of the second: w -= sum_{i<=j} hc_i v_i
-// row by row, with the row's v_0..v_j kept in registers for the partial
-// dots of the updated w with v_0..v_j.  The same operations in the same
-// order as bk_update (non-final pass) followed by its bdots, so the same
-// bits, with one read of the basis instead of two.
-template <typename VT, int RPT>
+// The first CGS2 pass fused with the dots of the second (UPD): w -= sum hc_i
+// v_i row by row, the row's v_0..v_j (j < NV, past j the last one again) kept in
+// registers for the partial dots of the updated w: one read of the basis
+// instead of two, the same bits.  Without UPD the dots alone.
+template <typename VT, int NV, bool UPD>
 __global__ void __launch_bounds__(BB_BS)
-bk_update_dots(int n, int KP, int K, VT* __restrict__ W, const VT* __restrict__ V, size_t bs,
+bk_update_dots(int n, int KP, int K, int R, VT* __restrict__ W, const VT* __restrict__ V, size_t bs,
                int j, double* __restrict__ part, int G, const BCol* __restrict__ cols)
 {
-    __shared__ VT shv[BB_MAXM][BB_MAXK];
-    __shared__ double sh[BB_BS / 64][BB_LB][BB_MAXK];
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
-    const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
+    const int base = lblock() * RB * R + (int)threadIdx.x / KP;
     const bool act = q < K && cols[q].active;
-    for (int e = threadIdx.x; e < BB_MAXM * KP; e += BB_BS) {
-        const int i = e / KP, qq = e % KP;
-        shv[i][qq] = (qq < K && i <= j && cols[qq].active) ? (VT)cols[qq].hc[i] : VT(0);
-    }
-    __syncthreads();
-    double acc[BB_MAXM];
+    double acc[NV];
 #pragma unroll
-    for (int i = 0; i < BB_MAXM; ++i) acc[i] = 0.0;
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        if (!act || row >= n) continue;
-        const size_t o = (size_t)row * KP + q;
-        VT vv[BB_MAXM];
+    for (int i = 0; i < NV; ++i) acc[i] = 0.0;
+    if (act) {
+        VT hv[NV];
 #pragma unroll
-        for (int i = 0; i < BB_MAXM; ++i) vv[i] = i <= j ? V[(size_t)i * bs + o] : VT(0);
-        VT w = W[o];
-#pragma unroll
-        for (int i = 0; i < BB_MAXM; ++i)
-            if (i <= j) w = w - shv[i][q] * vv[i];
-        W[o] = w;
-#pragma unroll
-        for (int i = 0; i < BB_MAXM; ++i)
-            if (i <= j) acc[i] += dd(w) * dd(vv[i]);
-    }
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int i0 = 0; i0 < BB_MAXM; i0 += BB_LB) {
-        if (i0 > j) break;
-#pragma unroll
-        for (int u = 0; u < BB_LB; ++u) {
-            const double s = col_wave_sum(acc[i0 + u], KP);
-            if (lane < KP) sh[wid][u][lane] = s;
+        for (int i = 0; i < NV; ++i) {
+            const VT h = (VT)cols[q].hc[min(i, j)];
+            hv[i] = UPD && i <= j ? h : VT(0);
         }
-        __syncthreads();
-        for (int e = threadIdx.x; e < BB_LB * KP; e += BB_BS) {
-            const int u = e / KP, qq = e % KP;
-            if (i0 + u <= j) {
-                double s = 0.0;
+#pragma unroll 1
+        for (int t = 0; t < R; ++t) {
+            const int row = base + t * RB;
+            if (row >= n) break;
+            const size_t o = (size_t)row * KP + q;
+            VT v[NV];
+            VT w = W[o];
 #pragma unroll
-                for (int ww = 0; ww < BB_BS / 64; ++ww) s += sh[ww][u][qq];
-                part[((size_t)(i0 + u) * KP + qq) * G + lblock()] = s;
+            for (int i = 0; i < NV; ++i) v[i] = V[(size_t)min(i, j) * bs + o];
+            if (UPD) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i) w = w - hv[i] * v[i];
+                W[o] = w;
             }
+#pragma unroll
+            for (int i = 0; i < NV; ++i) acc[i] += dd(w) * dd(v[i]);
         }
-        __syncthreads();
     }
+    put_partials<NV>(acc, j, KP, 0, part, G);
 }
 
 // Givens rotation of step j for each column (one wavefront per column) from
@@ -650,33 +575,47 @@ bk_solve_y(int K, BCol* __restrict__ cols)
 }
 
 // X += D (V y) per column (FP64 accumulation; D = dscale, or 1 when null: the
-// diagonal right preconditioner); X is n x K (the caller's layout).
-template <typename VT, int RPT>
+// diagonal right preconditioner); X is n x K (the caller's layout).  Eight
+// vectors' loads at a time.
+template <typename VT>
 __global__ void __launch_bounds__(BB_BS)
-bk_xupdate(int n, int KP, int K, const VT* __restrict__ V, size_t bs, const BIo* __restrict__ io,
-           const BCol* __restrict__ cols, const double* __restrict__ dscale)
+bk_xupdate(int n, int KP, int K, int R, const VT* __restrict__ V, size_t bs,
+           const BIo* __restrict__ io, const BCol* __restrict__ cols,
+           const double* __restrict__ dscale)
 {
+    __shared__ double ys[BB_MAXM][BB_MAXK];
+    for (int e = threadIdx.x; e < BB_MAXM * KP; e += BB_BS) {
+        const int i = e / KP, qq = e % KP;
+        ys[i][qq] = qq < K && i < cols[qq].k ? cols[qq].y[i] : 0.0;
+    }
+    __syncthreads();
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
-    const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
+    const int base = lblock() * RB * R + (int)threadIdx.x / KP;
     if (q >= K) return;
-    const BCol* c = cols + q;
-    const int k = c->k;
-    if (c->converged || k == 0) return;
+    const int k = cols[q].k;
+    if (cols[q].converged || k == 0) return;
     double* __restrict__ X = io->X;
-    for (int t = 0; t < RPT; ++t) {
+    for (int t = 0; t < R; ++t) {
         const int row = base + t * RB;
         if (row >= n) break;
+        const size_t o = (size_t)row * KP + q;
         double s = 0.0;
-        for (int i = 0; i < k; ++i) s += dd(V[(size_t)i * bs + (size_t)row * KP + q]) * c->y[i];
+        for (int i0 = 0; i0 < k; i0 += 8) {
+            VT v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = V[(size_t)min(i0 + u, k - 1) * bs + o];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += dd(v[u]) * ys[min(i0 + u, BB_MAXM - 1)][q];
+        }
         X[(size_t)row * K + q] += dscale ? dscale[row] * s : s;
     }
 }
 
 // r = b - A x (FP64), W0 = r in the Krylov type, partial ||r||^2 per column.
-template <typename VT, int RPT>
+template <typename VT>
 __global__ void __launch_bounds__(BB_BS)
-bk_residual(int n, int KP, int K, int width, const int* __restrict__ col,
+bk_residual(int n, int KP, int K, int R, int width, const int* __restrict__ col,
             const double* __restrict__ val, const BIo* __restrict__ io, VT* __restrict__ W0,
             double* __restrict__ part, int G, const BCol* __restrict__ cols)
 {
@@ -684,60 +623,39 @@ bk_residual(int n, int KP, int K, int width, const int* __restrict__ col,
     const double* __restrict__ X = io->X;
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
-    const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
-    const bool act = q < K && !cols[q].converged;
-    VT w[RPT];
-#pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        w[t] = VT(0);
-        if (act && row < n) {
-            double s = 0.0;
-            if (width > ELL_MAXW) {  // long rows: the same sum, not unrolled
-                for (int k = 0; k < width; ++k) {
-                    const size_t o = (size_t)k * n + row;
-                    s += val[o] * X[(size_t)col[o] * K + q];
-                }
-            } else {
-                int c[ELL_MAXW];
-                double v[ELL_MAXW], xv[ELL_MAXW];
-#pragma unroll
-                for (int k = 0; k < ELL_MAXW; ++k) {
-                    const size_t o = (size_t)k * n + row;
-                    c[k] = k < width ? col[o] : 0;
-                    v[k] = k < width ? val[o] : 0.0;
-                }
-#pragma unroll
-                for (int k = 0; k < ELL_MAXW; ++k)
-                    xv[k] = k < width ? X[(size_t)c[k] * K + q] : 0.0;
-#pragma unroll
-                for (int k = 0; k < ELL_MAXW; ++k)
-                    if (k < width) s += v[k] * xv[k];
-            }
-            const double r = B[(size_t)row * K + q] - s;
-            w[t] = (VT)r;
-            W0[(size_t)row * KP + q] = w[t];
+    const int base = lblock() * RB * R + (int)threadIdx.x / KP;
+    double a[1] = {0.0};
+    if (q < K && !cols[q].converged) {
+        for (int t = 0; t < R; ++t) {
+            const int row = base + t * RB;
+            if (row >= n) break;
+            const double s = brow<double, double>(n, width, row, col, val, X, K, q, 1.0);
+            const VT w = (VT)(B[(size_t)row * K + q] - s);
+            W0[(size_t)row * KP + q] = w;
+            a[0] += dd(w) * dd(w);
         }
     }
-    bdots<VT, RPT>(0, -1, nullptr, nullptr, 0, n, KP, q, base, RB, act, w, part, G, 0);
+    put_partials<1>(a, 0, KP, 0, part, G);
 }
 
 // ||b_q||^2 partials: the same reduction with B read as the vector.
-template <int RPT>
 __global__ void __launch_bounds__(BB_BS)
-bk_sumsq(int n, int KP, int K, const double* __restrict__ B, double* __restrict__ part, int G)
+bk_sumsq(int n, int KP, int K, int R, const double* __restrict__ B, double* __restrict__ part,
+         int G)
 {
     const int q = threadIdx.x & (KP - 1);
     const int RB = BB_BS / KP;
-    const int base = lblock() * RB * RPT + (int)threadIdx.x / KP;
-    const bool act = q < K;
-    double w[RPT];
-#pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int row = base + t * RB;
-        w[t] = (act && row < n) ? B[(size_t)row * K + q] : 0.0;
+    const int base = lblock() * RB * R + (int)threadIdx.x / KP;
+    double a[1] = {0.0};
+    if (q < K) {
+        for (int t = 0; t < R; ++t) {
+            const int row = base + t * RB;
+            if (row >= n) break;
+            const double b = B[(size_t)row * K + q];
+            a[0] += b * b;
+        }
     }
-    bdots<double, RPT>(0, -1, nullptr, nullptr, 0, n, KP, q, base, RB, act, w, part, G, 0);
+    put_partials<1>(a, 0, KP, 0, part, G);
 }
 
 __global__ void bk_set_bnorm(int KP, int K, const double* __restrict__ part, int G,
@@ -892,10 +810,61 @@ __global__ void bk_count_active(int K, const BCol* __restrict__ cols, int* __res
     if (lane == 0) out[0] = a;
 }
 
+// f(rows per thread as a constant)
+template <typename F>
+void by_rpt(int rpt, F f)
+{
+    switch (rpt) {
+    case 1: return f(std::integral_constant<int, 1>());
+    case 2: return f(std::integral_constant<int, 2>());
+    case 4: return f(std::integral_constant<int, 4>());
+    case 8: return f(std::integral_constant<int, 8>());
+    default: return f(std::integral_constant<int, BB_RPT>());
+    }
+}
+
+template <typename VT, typename MT, bool PC>
+void step(const Ell<MT>& E, BatchWork* w, int K, const VT* X, VT* dst, int j, hipStream_t s)
+{
+    const dim3 grid(w->G), block(BB_BS);
+    const size_t bs = (size_t)w->n * w->kp;
+    by_rpt(w->rpt, [&](auto r) {
+        constexpr int RPT = decltype(r)::value;
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_step_spmm<VT, MT, RPT, PC>), grid, block, 0, s, w->n,
+                           w->kp, K, E.width, E.col.p, E.val.p, X, (VT*)w->V.p, bs, dst, j,
+                           w->part.p, w->G, w->cols.p);
+    });
+}
+template <typename VT>
+void update(BatchWork* w, int K, VT* dst, int j, bool norm, hipStream_t s)
+{
+    by_rpt(w->rpt, [&](auto r) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_update<VT, decltype(r)::value>), dim3(w->G),
+                           dim3(BB_BS), 0, s, w->n, w->kp, K, dst, (const VT*)w->V.p,
+                           (size_t)w->n * w->kp, j, (int)norm, w->part.p, w->G, w->cols.p);
+    });
+}
+template <typename VT, bool UPD, int NV>
+void launch_update_dots(BatchWork* w, int K, VT* dst, int j, hipStream_t s)
+{
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_update_dots<VT, NV, UPD>), dim3(w->G), dim3(BB_BS), 0, s,
+                       w->n, w->kp, K, w->rpt, dst, (const VT*)w->V.p, (size_t)w->n * w->kp, j,
+                       w->part.p, w->G, w->cols.p);
+}
+template <typename VT, bool UPD>
+void update_dots(BatchWork* w, int K, VT* dst, int j, hipStream_t s)
+{
+    if (j < 4) launch_update_dots<VT, UPD, 4>(w, K, dst, j, s);
+    else if (j < 8) launch_update_dots<VT, UPD, 8>(w, K, dst, j, s);
+    else if (j < 16) launch_update_dots<VT, UPD, 16>(w, K, dst, j, s);
+    else if (j < 24) launch_update_dots<VT, UPD, 24>(w, K, dst, j, s);
+    else launch_update_dots<VT, UPD, 32>(w, K, dst, j, s);
+}
+
 // Arnoldi steps j0 .. j1-1 of a cycle of m steps (chunk c: steps up to
 // bb_chunk_end(c)); a chunk that is not the cycle's last ends by counting
 // the columns still running.
-template <typename VT, typename MT, int RPT>
+template <typename VT, typename MT>
 void enqueue_batch_steps(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, int j0, int j1,
                          int m, int passes, double rtol, double inner_rtol, int max_iters,
                          BatchPrecond* pc, hipStream_t s)
@@ -920,22 +889,22 @@ void enqueue_batch_steps(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K,
             hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_scale<VT>), dim3((unsigned)((bs + BB_BS - 1) / BB_BS)),
                                block, 0, s, n, KP, K, src, Vj, j, cols);
             precond_apply<VT>(pc, KP, Vj, Zj, s);
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_step_spmm_pc<VT, MT, RPT>), grid, block, 0, s, n, KP,
-                               K, E.width, E.col.p, E.val.p, Zj, V, bs, dst, j, part, G, cols);
+            step<VT, MT, true>(E, w, K, Zj, dst, j, s);
         } else {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_step_spmm<VT, MT, RPT>), grid, block, 0, s, n, KP, K,
-                               E.width, E.col.p, E.val.p, src, V, bs, dst, j, part, G, cols);
+            step<VT, MT, false>(E, w, K, src, dst, j, s);
         }
         for (int p = 0; p < passes; ++p) {
             const int nd = j + 1;
             hipLaunchKernelGGL(bk_reduce, dim3((nd * KP + 3) / 4), block, 0, s, KP, K, nd, j, p,
                                part, G, cols);
-            if (p < passes - 1 && fused_update_dots())
-                hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_update_dots<VT, RPT>), grid, block, 0, s, n,
-                                   KP, K, dst, V, bs, j, part, G, cols);
-            else
-                hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_update<VT, RPT>), grid, block, 0, s, n, KP,
-                                   K, dst, V, bs, j, p == passes - 1 ? 1 : 0, part, G, cols);
+            if (p == passes - 1) {
+                update<VT>(w, K, dst, j, true, s);
+            } else if (fused_update_dots()) {
+                update_dots<VT, true>(w, K, dst, j, s);
+            } else {
+                update<VT>(w, K, dst, j, false, s);
+                update_dots<VT, false>(w, K, dst, j, s);
+            }
         }
         hipLaunchKernelGGL(bk_givens, dim3(cb), block, 0, s, KP, K, j, m, part, G, cols, rtol,
                            inner_rtol, max_iters);
@@ -945,7 +914,7 @@ void enqueue_batch_steps(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K,
 
 // The end of a cycle: y, the x update, the true residual and the next
 // cycle's start (the host summary).
-template <typename VT, typename MT, int RPT>
+template <typename VT, typename MT>
 void enqueue_batch_finish(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, double rtol,
                           int max_iters, BatchPrecond* pc, hipStream_t s)
 {
@@ -958,18 +927,18 @@ void enqueue_batch_finish(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K
     const dim3 grid(G), block(BB_BS);
     const int cb = (K + 3) / 4;
     hipLaunchKernelGGL(bk_solve_y, dim3(cb), block, 0, s, K, cols);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_xupdate<VT, RPT>), grid, block, 0, s, n, KP, K,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_xupdate<VT>), grid, block, 0, s, n, KP, K, w->rpt,
                        pc ? (const VT*)w->Z.p : (const VT*)V, bs, w->io.p, cols,
                        (!pc && (const void*)E.val.p == (const void*)A->ell64d.val.p)
                            ? A->dinv.p : (const double*)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT, RPT>), grid, block, 0, s, n, KP, K,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT>), grid, block, 0, s, n, KP, K, w->rpt,
                        A->ell64.width, A->ell64.col.p, A->ell64.val.p, w->io.p, W0, part, G, cols);
     hipLaunchKernelGGL(bk_cycle_start, dim3(cb), block, 0, s, KP, K, part, G, cols, w->sum.p,
                        rtol, max_iters);
 }
 
-template <typename VT, typename MT, int RPT>
-int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const double* B, double* X,
+template <typename VT, typename MT>
+int batch_run(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const double* B, double* X,
               const phg_gmres_opts& o, phg_gmres_info* infos, BatchPrecond* pc, hipStream_t s)
 {
     const int n = w->n, KP = w->kp, G = w->G, m = o.restart;
@@ -987,10 +956,10 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
         const size_t tot = (size_t)n * K;
         hipLaunchKernelGGL(bk_fill0, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, tot, X);
     }
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_sumsq<RPT>), grid, block, 0, s, n, KP, K, B, part, G);
+    hipLaunchKernelGGL(bk_sumsq, grid, block, 0, s, n, KP, K, w->rpt, B, part, G);
     hipLaunchKernelGGL(bk_set_bnorm, dim3(cb), block, 0, s, KP, K, part, G, cols,
                        BIo{B, X}, w->io.p);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT, RPT>), grid, block, 0, s, n, KP, K,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT>), grid, block, 0, s, n, KP, K, w->rpt,
                        A->ell64.width, A->ell64.col.p, A->ell64.val.p, w->io.p, W0, part, G, cols);
     hipLaunchKernelGGL(bk_cycle_start, dim3(cb), block, 0, s, KP, K, part, G, cols, w->sum.p,
                        o.rtol, o.max_iters);
@@ -1019,11 +988,11 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
                 hipGraph_t g = nullptr;
                 PHG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
                 if (c < nch)
-                    enqueue_batch_steps<VT, MT, RPT>(A, E, w, K, chunk_lo(c), chunk_hi(c), m,
+                    enqueue_batch_steps<VT, MT>(A, E, w, K, chunk_lo(c), chunk_hi(c), m,
                                                      passes, o.rtol, inner, o.max_iters, pc,
                                                      cs);
                 else
-                    enqueue_batch_finish<VT, MT, RPT>(A, E, w, K, o.rtol, o.max_iters, pc, cs);
+                    enqueue_batch_finish<VT, MT>(A, E, w, K, o.rtol, o.max_iters, pc, cs);
                 PHG_HIP(hipStreamEndCapture(cs, &g));
                 hipError_t e = hipGraphInstantiate(&w->exec[c], g, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(g);
@@ -1050,7 +1019,7 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
             if (o.graph) {
                 PHG_HIP(hipGraphLaunch(w->exec[c], s));
             } else {
-                enqueue_batch_steps<VT, MT, RPT>(A, E, w, K, chunk_lo(c), chunk_hi(c), m, passes,
+                enqueue_batch_steps<VT, MT>(A, E, w, K, chunk_lo(c), chunk_hi(c), m, passes,
                                                  o.rtol, inner, o.max_iters, pc, s);
                 PHG_HIP(hipGetLastError());
             }
@@ -1063,7 +1032,7 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
         if (o.graph) {
             PHG_HIP(hipGraphLaunch(w->exec[nch], s));
         } else {
-            enqueue_batch_finish<VT, MT, RPT>(A, E, w, K, o.rtol, o.max_iters, pc, s);
+            enqueue_batch_finish<VT, MT>(A, E, w, K, o.rtol, o.max_iters, pc, s);
             PHG_HIP(hipGetLastError());
         }
     }
@@ -1081,19 +1050,6 @@ int batch_run_t(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const do
         }
     }
     return all ? PHG_OK : PHG_ERR_NOCONV;
-}
-
-template <typename VT, typename MT>
-int batch_run(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const double* B, double* X,
-              const phg_gmres_opts& o, phg_gmres_info* infos, BatchPrecond* pc, hipStream_t s)
-{
-    switch (w->rpt) {
-    case 1: return batch_run_t<VT, MT, 1>(A, E, w, K, B, X, o, infos, pc, s);
-    case 2: return batch_run_t<VT, MT, 2>(A, E, w, K, B, X, o, infos, pc, s);
-    case 4: return batch_run_t<VT, MT, 4>(A, E, w, K, B, X, o, infos, pc, s);
-    case 8: return batch_run_t<VT, MT, 8>(A, E, w, K, B, X, o, infos, pc, s);
-    default: return batch_run_t<VT, MT, BB_RPT>(A, E, w, K, B, X, o, infos, pc, s);
-    }
 }
 
 // ------------------------------------------------------- launch shapes --
