@@ -46,7 +46,8 @@ namespace phg {
 
 constexpr int GM_MAXM = 64;
 constexpr int GM_MAXN = 1 << 20; // most rows
-constexpr int GM_RED = 1024;  // threads of the reducing workgroup
+constexpr int GM_RED = 1024;      // threads of the reducing workgroup
+constexpr int GM_BS = KR_STRIDE;  // threads of the others
 
 struct GmresState {
     double R[GM_MAXM * GM_MAXM];  // rotated (upper triangular) columns
@@ -101,7 +102,7 @@ __device__ __forceinline__ void write_partials(const double (*sh)[GM_MAXM + 1], 
     if (t < nv || (norm && t == GM_MAXM)) {
         double r = 0.0;
 #pragma unroll
-        for (int q = 0; q < KR_BS / 64; ++q) r += sh[q][t];
+        for (int p = 0; p < GM_BS / 64; p += 4) r += krylov_half(sh[p][t], sh[p + 1][t], sh[p + 2][t], sh[p + 3][t]);
         part[(size_t)lblock() * S + v] = r;
     }
 }
@@ -140,21 +141,21 @@ __device__ __forceinline__ VT basis_at(const VT* V, size_t ldv, int i, int row)
     return *(const VT*)((const char*)V + o);
 }
 
-// A block owns R x KR_BS rows, a thread rows base + r * KR_BS, r < R.
+// A block owns R x GM_BS rows, a thread rows base + r * GM_BS, r < R.
 //
 // r = b - A x in FP64 (the refinement residual); W0 = r; partial ||r||^2.
 template <typename VT>
-__global__ void __launch_bounds__(KR_BS)
+__global__ void __launch_bounds__(GM_BS)
 k_residual(int n, int R, int width, const int* __restrict__ col, const double* __restrict__ val,
            VT* __restrict__ W0, int S, double* __restrict__ part, const GmresState* __restrict__ st)
 {
-    __shared__ double sh[KR_BS / 64][GM_MAXM + 1];
+    __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
     if (st->converged) return;
     const double *b = st->b, *x = st->x;
-    const int base = lblock() * KR_BS * R + threadIdx.x;
+    const int base = lblock() * GM_BS * R + threadIdx.x;
     double a = 0.0;
     for (int r = 0; r < R; ++r) {
-        const int row = base + r * KR_BS;
+        const int row = base + r * GM_BS;
         double xo, ax;
         krylov_rows<double, double, false, 1>(n, width, row, col, val, x, 1, 1.0, &xo, &ax);
         if (row >= n) break;
@@ -166,14 +167,14 @@ k_residual(int n, int R, int width, const int* __restrict__ col, const double* _
     write_partials(sh, 0, true, S, part);
 }
 
-__global__ void __launch_bounds__(KR_BS)
+__global__ void __launch_bounds__(GM_BS)
 k_sumsq(int n, int R, const double* __restrict__ b, int S, double* __restrict__ part)
 {
-    __shared__ double sh[KR_BS / 64][GM_MAXM + 1];
-    const int base = lblock() * KR_BS * R + threadIdx.x;
+    __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
+    const int base = lblock() * GM_BS * R + threadIdx.x;
     double a = 0.0;
     for (int r = 0; r < R; ++r) {
-        const int row = base + r * KR_BS;
+        const int row = base + r * GM_BS;
         if (row >= n) break;
         a = fma(b[row], b[row], a);
     }
@@ -186,21 +187,21 @@ k_sumsq(int n, int R, const double* __restrict__ b, int S, double* __restrict__ 
 // loaded without a branch (past j - 1 the last one again, not used), so that
 // all of them are in flight.
 template <typename VT, typename MT, int NV>
-__global__ void __launch_bounds__(KR_BS)
+__global__ void __launch_bounds__(GM_BS)
 k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __restrict__ val,
             const VT* __restrict__ Wsrc, VT* __restrict__ V, size_t ldv, VT* __restrict__ Wdst,
             int j, int S, double* __restrict__ part, const GmresState* __restrict__ st)
 {
-    __shared__ double sh[KR_BS / 64][GM_MAXM + 1];
+    __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
     if (!st->active) return;
     const VT inv = (VT)(1.0 / (j == 0 ? st->beta : st->hn));
-    const int base = lblock() * KR_BS * R + threadIdx.x;
+    const int base = lblock() * GM_BS * R + threadIdx.x;
     double acc[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) acc[i] = 0.0;
 #pragma unroll 1
     for (int r = 0; r < R; ++r) {
-        const int row = base + r * KR_BS;
+        const int row = base + r * GM_BS;
         if (row >= n) break;
         VT v[NV], vj, w;
 #pragma unroll
@@ -223,23 +224,23 @@ k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __re
 // coefficient of 0): with one, level 8's updates with 32 vectors took 95 us
 // instead of 30.
 template <typename VT, int NV, bool DOTS>
-__global__ void __launch_bounds__(KR_BS)
+__global__ void __launch_bounds__(GM_BS)
 k_update(int n, int R, VT* __restrict__ w, const VT* __restrict__ V, size_t ldv, int j, int norm,
          int S, double* __restrict__ part, const GmresState* __restrict__ st)
 {
-    __shared__ double sh[KR_BS / 64][GM_MAXM + 1];
+    __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
     __shared__ VT hs[NV];
     if (!st->active) return;
     if ((int)threadIdx.x < NV)
         hs[threadIdx.x] = (int)threadIdx.x <= j ? (VT)st->hc[threadIdx.x] : VT(0);
     __syncthreads();
-    const int base = lblock() * KR_BS * R + threadIdx.x;
+    const int base = lblock() * GM_BS * R + threadIdx.x;
     double acc[NV], nrm = 0.0;
 #pragma unroll
     for (int i = 0; i < NV; ++i) acc[i] = 0.0;
 #pragma unroll 1
     for (int r = 0; r < R; ++r) {
-        const int row = base + r * KR_BS;
+        const int row = base + r * GM_BS;
         if (row >= n) break;
         VT v[NV];
         VT wr = w[row];
@@ -263,12 +264,12 @@ k_update(int n, int R, VT* __restrict__ w, const VT* __restrict__ V, size_t ldv,
 // time, tier by tier: FIRST is the product and its dots, otherwise the update
 // (the basis read once for it and once for the dots).
 template <typename VT, typename MT, bool FIRST>
-__global__ void __launch_bounds__(KR_BS)
+__global__ void __launch_bounds__(GM_BS)
 k_long(int n, int R, int width, const int* __restrict__ col, const MT* __restrict__ val,
        const VT* __restrict__ Wsrc, VT* __restrict__ V, size_t ldv, VT* __restrict__ w, int j,
        int dots, int norm, int S, double* __restrict__ part, const GmresState* __restrict__ st)
 {
-    __shared__ double sh[KR_BS / 64][GM_MAXM + 1];
+    __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
     __shared__ VT hs[GM_MAXM];
     if (!st->active) return;
     const int lane = threadIdx.x & 63;
@@ -276,7 +277,7 @@ k_long(int n, int R, int width, const int* __restrict__ col, const MT* __restric
         hs[threadIdx.x] = (int)threadIdx.x <= j ? (VT)st->hc[threadIdx.x] : VT(0);
     if (FIRST) norm = 0;
     __syncthreads();
-    const int base = lblock() * KR_BS * R + threadIdx.x;
+    const int base = lblock() * GM_BS * R + threadIdx.x;
     double nrm = 0.0;
     for (int i0 = 0; i0 <= j; i0 += KR_T) {
         // the product or the whole update first, then the dots of this tier
@@ -284,7 +285,7 @@ k_long(int n, int R, int width, const int* __restrict__ col, const MT* __restric
 #pragma unroll
         for (int q = 0; q < KR_T; ++q) acc[q] = 0.0;
         for (int r = 0; r < R; ++r) {
-            const int row = base + r * KR_BS;
+            const int row = base + r * GM_BS;
             if (row >= n) break;
             VT wr;
             if (i0 == 0 && FIRST) {
@@ -437,7 +438,7 @@ k_solve_y(GmresState* __restrict__ st)
 
 // x += sum_i y_i v_i, accumulated in FP64.
 template <typename VT>
-__global__ void __launch_bounds__(KR_BS)
+__global__ void __launch_bounds__(GM_BS)
 k_xupdate(int n, const VT* __restrict__ V, size_t ldv, const GmresState* __restrict__ st)
 {
     __shared__ double ys[GM_MAXM];
@@ -446,7 +447,7 @@ k_xupdate(int n, const VT* __restrict__ V, size_t ldv, const GmresState* __restr
     if (k == 0) return;
     if ((int)threadIdx.x < k) ys[threadIdx.x] = st->y[threadIdx.x];
     __syncthreads();
-    const int row = lblock() * KR_BS + threadIdx.x;
+    const int row = lblock() * GM_BS + threadIdx.x;
     if (row >= n) return;
     double s = 0.0;
     int i = 0;
@@ -475,10 +476,11 @@ int prepare_work(phg_matrix_s* A, int prec, int m, int ortho, GmresWork** out)
     // The persistent form's rows per thread where it runs.  Above, as many as
     // leave about one workgroup per CU: the sums have few partials and the
     // workgroups end together (level 8, 5 rows on 257 workgroups: the
-    // reducing workgroup took 3.6 us instead of 6.9 with 641 partials).
-    const int R = n <= KR_ROWS * XCH_MAXG ? KR_RPT
-                                          : std::max(KR_RPT, (int)std::lround((double)n / (KR_BS * XCH_MAXG)));
-    const int G = (int)(((long)n + KR_BS * R - 1) / (KR_BS * R));
+    // reducing workgroup took 4.8 us instead of 6.9 with 641 partials).
+    const int R = n <= GM_BS * KR_RPT * KR_MAXG
+                      ? KR_RPT
+                      : std::max(KR_RPT, (int)std::lround((double)n / (GM_BS * KR_MAXG)));
+    const int G = (int)(((long)n + GM_BS * R - 1) / (GM_BS * R));
     if (n > GM_MAXN) {
         set_error("gmres: matrix too large for one device workspace");
         return PHG_ERR_ARG;
@@ -515,7 +517,7 @@ int prepare_passes(GmresWork* w)
 template <typename VT, typename MT, int NV>
 void step_nv(const Ell<MT>& E, GmresWork* w, const VT* src, VT* dst, int j, hipStream_t s)
 {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_step_spmv<VT, MT, NV>), dim3(w->G), dim3(KR_BS), 0, s, w->n,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_step_spmv<VT, MT, NV>), dim3(w->G), dim3(GM_BS), 0, s, w->n,
                        w->R, E.width, E.col.p, E.val.p, src, (VT*)w->V.p, w->ldv, dst, j, w->S,
                        w->part.p, w->st.p);
 }
@@ -523,7 +525,7 @@ template <typename VT, int NV>
 void update_nv(GmresWork* w, VT* dst, int j, bool dots, bool norm, hipStream_t s)
 {
     const VT* V = (const VT*)w->V.p;
-    const dim3 grid(w->G), block(KR_BS);
+    const dim3 grid(w->G), block(GM_BS);
     if (dots)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_update<VT, NV, true>), grid, block, 0, s, w->n, w->R,
                            dst, V, w->ldv, j, (int)norm, w->S, w->part.p, w->st.p);
@@ -540,7 +542,7 @@ void step(const Ell<MT>& E, GmresWork* w, const VT* src, VT* dst, int j, hipStre
     else if (j < 24) step_nv<VT, MT, 24>(E, w, src, dst, j, s);
     else if (j < 32) step_nv<VT, MT, 32>(E, w, src, dst, j, s);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_long<VT, MT, true>), dim3(w->G), dim3(KR_BS), 0, s,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_long<VT, MT, true>), dim3(w->G), dim3(GM_BS), 0, s,
                            w->n, w->R, E.width, E.col.p, E.val.p, src, (VT*)w->V.p, w->ldv, dst, j,
                            1, 0, w->S, w->part.p, w->st.p);
 }
@@ -553,7 +555,7 @@ void update(const Ell<MT>& E, GmresWork* w, VT* dst, int j, bool dots, bool norm
     else if (j < 24) update_nv<VT, 24>(w, dst, j, dots, norm, s);
     else if (j < 32) update_nv<VT, 32>(w, dst, j, dots, norm, s);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_long<VT, MT, false>), dim3(w->G), dim3(KR_BS), 0, s,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_long<VT, MT, false>), dim3(w->G), dim3(GM_BS), 0, s,
                            w->n, w->R, E.width, E.col.p, E.val.p, (const VT*)nullptr, (VT*)w->V.p,
                            w->ldv, dst, j, (int)dots, (int)norm, w->S, w->part.p, w->st.p);
 }
@@ -569,7 +571,7 @@ void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, bool 
     double* part = w->part.p;
     GmresState* st = w->st.p;
     const int mgs = cgs ? 0 : (sizeof(VT) == 4 ? 2 : 1);
-    const dim3 grid(G), block(KR_BS), one(1), red(GM_RED);
+    const dim3 grid(G), block(GM_BS), one(1), red(GM_RED);
     for (int j = 0; j < m; ++j) {
         VT* src = (j & 1) ? W1 : W0;
         VT* dst = (j & 1) ? W0 : W1;
@@ -587,7 +589,7 @@ void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, bool 
                            part, G, st);
     }
     hipLaunchKernelGGL(k_solve_y, one, dim3(64), 0, s, st);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_xupdate<VT>), dim3((n + KR_BS - 1) / KR_BS), block, 0, s,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_xupdate<VT>), dim3((n + GM_BS - 1) / GM_BS), block, 0, s,
                        n, V, ldv, st);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual<VT>), grid, block, 0, s, n, w->R, A->ell64.width,
                        A->ell64.col.p, A->ell64.val.p, W0, S, part, st);
@@ -604,7 +606,7 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
     VT* W0 = (VT*)w->W.p;
     double* part = w->part.p;
     GmresState* st = w->st.p;
-    const dim3 grid(G), block(KR_BS), one(1), red(GM_RED);
+    const dim3 grid(G), block(GM_BS), one(1), red(GM_RED);
     const bool cgs = o.ortho == PHG_CGS2;
 
     // parameters of the solve

@@ -12,10 +12,10 @@
 
 namespace phg {
 
-constexpr int KR_BS = 512;  // threads per workgroup
-constexpr int KR_RPT = 2;   // rows per thread
-constexpr int KR_ROWS = KR_BS * KR_RPT;
-constexpr int KR_T = 8;     // basis vectors per tier of dots
+constexpr int KR_RPT = 2;       // rows per thread
+constexpr int KR_STRIDE = 512;  // between a thread's rows
+constexpr int KR_T = 8;         // basis vectors per tier of dots
+constexpr int KR_MAXG = 256;    // most workgroups of a persistent launch
 
 // A double moved between lanes by a DPP pattern (both 32-bit halves).
 template <int CTRL>
@@ -147,7 +147,7 @@ struct RowTerm<float, MT> {
     }
 };
 
-// Rows of any width: base + r * KR_BS (r < RG) of A x, entry by entry.
+// Rows of any width: base + r * KR_STRIDE (r < RG) of A x, entry by entry.
 template <typename VT, typename MT, bool AGENT, int RG>
 __device__ __forceinline__ void krylov_rows_loop(int n, int width, int base,
                                                  const int* __restrict__ col,
@@ -156,7 +156,7 @@ __device__ __forceinline__ void krylov_rows_loop(int n, int width, int base,
 {
 #pragma unroll
     for (int q = 0; q < RG; ++q) {
-        const int rr = base + q * KR_BS;
+        const int rr = base + q * KR_STRIDE;
         xo[q] = VT(0);
         w[q] = VT(0);
         if (rr < n) {
@@ -171,7 +171,7 @@ __device__ __forceinline__ void krylov_rows_loop(int n, int width, int base,
     }
 }
 
-// Rows base + r * KR_BS (r < RG) of A x (x scaled by inv): xo[r] = x[row],
+// Rows base + r * KR_STRIDE (r < RG) of A x (x scaled by inv): xo[r] = x[row],
 // w[r] = the row's sum, both 0 at and past row n; x entry i at x[i * ldx].
 // For rows of at most ELL_MAXW entries every row's own entry and slots are
 // loaded first, then every gather, then the sums in slot order: two memory
@@ -187,7 +187,7 @@ __device__ __forceinline__ void krylov_rows(int n, int width, int base, const in
         VT xv[RG][ELL_MAXW];
 #pragma unroll
         for (int q = 0; q < RG; ++q) {
-            const int rr = min(base + q * KR_BS, n - 1);  // in bounds; unused past n
+            const int rr = min(base + q * KR_STRIDE, n - 1);  // in bounds; unused past n
             xo[q] = ld_x<AGENT>(x + (size_t)rr * ldx);
 #pragma unroll
             for (int k = 0; k < ELL_MAXW; ++k) {
@@ -208,7 +208,7 @@ __device__ __forceinline__ void krylov_rows(int n, int width, int base, const in
                 const VT t = RowTerm<VT, MT>::add(s, v[q][k], xv[q][k], inv);
                 s = k < width ? t : s;
             }
-            const bool in = base + q * KR_BS < n;
+            const bool in = base + q * KR_STRIDE < n;
             w[q] = in ? s : VT(0);
             xo[q] = in ? xo[q] : VT(0);
         }
@@ -231,9 +231,15 @@ __device__ __forceinline__ void dots_tier(const VT (&w)[KR_RPT], const VT (&v)[K
     }
 }
 
+// Wavefronts' sums 0..3 or 4..7 of a block of 1024 rows; the block's partial
+// is the sum of the two halves.
+__device__ __forceinline__ double krylov_half(double a, double b, double c, double d)
+{
+    return ((a + b) + c) + d;
+}
+
 // Block partials g = 0..G-1 are added as 32 running sums (g mod 32, in g
 // order), then the sums q and q + 16, then the sixteen results in order.
-constexpr int KR_GRP = KR_BS / 32;  // thread groups of 32 values
 __device__ __forceinline__ double krylov_join(const double (*s)[33], int i)
 {
     double r = s[0][i];
@@ -241,7 +247,6 @@ __device__ __forceinline__ double krylov_join(const double (*s)[33], int i)
     for (int q = 1; q < 16; ++q) r += s[q][i];
     return r;
 }
-static_assert(KR_GRP == 16, "the running sums are split over sixteen thread groups");
 
 // Modified Gram-Schmidt coefficients from the dots r_i = <v_i, w> (lane i)
 // and the basis vectors' products L(i, k) = <v_i, v_k>, k < i: subtracting

@@ -1,6 +1,10 @@
 // Restarted GMRES as persistent launches (persist.hip): the
 // workspace that a matrix keeps for it, and its entry.
 #pragma once
+#include <algorithm>
+#include <mutex>
+
+#include "krylov.h"
 #include "phg_internal.h"
 
 namespace phg {
@@ -28,7 +32,6 @@ struct PState {
     int iters, cycles, converged, active;
 };
 
-constexpr int XCH_MAXG = 256;       // most workgroups of a launch
 constexpr int PERSIST_NOT_HERE = 2;  // the shape does not run here: nothing was done
 
 struct PersistWork {
@@ -47,6 +50,16 @@ struct PersistWork {
     PersistWork& operator=(const PersistWork&) = delete;
     ~PersistWork();
 };
+
+std::mutex& persist_mutex(int dev);  // held while a device's launches run
+
+// Workgroups of n rows: of 512 threads 1024 rows each, of 256 threads (half
+// of those 1024 rows each) two where the rows past the last 1024 need both.
+inline int persist_workgroups(int n, int threads)
+{
+    const int pair = KR_STRIDE / threads, rows = KR_STRIDE * KR_RPT;
+    return n / rows * pair + std::min(pair, (n % rows + threads - 1) / threads);
+}
 
 // A x_q = b_q for the K columns of B and X (n x K, row-major), each column by
 // itself; o as gmres_batch_solve_pc takes it, also with PHG_MGS.  diag:

@@ -1,7 +1,7 @@
 // Restarted GMRES(m), m <= 32, as persistent launches: all workgroups of a
 // launch are resident, a column of the right-hand side belongs to G
-// workgroups of KR_ROWS rows each, and a restart cycle keeps everything that
-// it owns on the chip.  A thread holds its rows of every basis vector, of
+// workgroups of 512 or 1024 rows each, and a restart cycle keeps everything
+// that it owns on the chip.  A thread holds its rows of every basis vector, of
 // the work vector and of the matrix in registers; only the vector that the
 // next product gathers goes through memory, and the global sums of an
 // Arnoldi step go through an exchange (below) instead of kernel boundaries.
@@ -17,17 +17,8 @@
 // Columns are independent: each group of G workgroups runs its own cycles
 // and stops by itself, so the batched solves of small meshes (gmres_batch)
 // run here as one launch.
-#include <unistd.h>
-
-#include <chrono>
-#include <cstdlib>
-#include <cstring>
-#include <mutex>
-#include <thread>
-
-#include "krylov.h"
-#include "persist.h"
-#include "phg_internal.h"
+#define PS_BS 512
+#include "persist_run.h"
 
 namespace phg {
 
@@ -99,688 +90,37 @@ PersistWork::~PersistWork()
     if (host) (void)hipHostFree(host);
 }
 
-namespace {
-
-typedef unsigned long long xch_t;
-constexpr xch_t XCH_EMPTY = 0x7FF4DEADBEEF0001ull;  // a signalling-NaN pattern no partial takes
-constexpr long XCH_SPIN = 1L << 22;                  // polls before a wait gives up
-// (PHG_XCH_SPIN overrides it: the failure-path test forces a give-up with
-// a limit of a few polls; every workgroup still exits normally)
-// polls of a launch's first exchange (some 0.1 s), and launches until it succeeds
-constexpr long XCH_START = 1L << 17;
-constexpr int XCH_TRIES = 64;
-enum { ABORT_WAIT = 1, ABORT_START = 2 };  // bits of the host's abort word
-constexpr int XCH_RING = 4;   // rows of a column's ring
-constexpr int XCH_V = 32;     // values of a slot
-constexpr int PS_M = 32;      // largest restart
-
-// ------------------------------------------------------------- exchange --
-// Exchange e of a column: every workgroup stores up to 32 block partials
-// into its slot (32 words) of row e mod 4 with agent-scope stores, and every
-// workgroup reads all G slots until none holds XCH_EMPTY, then adds them in
-// krylov_join's order.  All of a thread's loads are issued before the first
-// test, with no branch between them: 2.65 us among 161 workgroups, 32 values
-// as fast as one; with a bounds test before each load the same exchange took
-// 8.7 us.  A slot is one coalesced 256-byte store and load.  A row has one
-// of a few lengths (hop_slots), so that the loads have fixed offsets; the
-// slots past the last workgroup hold 0.
-//
-// A row is used again four exchanges later.  When a workgroup has finished
-// exchange e - 1, every workgroup has stored into row e - 1 and has
-// therefore finished reading row e - 2: each clears its own slot of row
-// e - 2 then.  The clearing is complete before it stores into row e + 1 (the
-// wait at the start of an exchange), and whoever polls row e + 2 has seen
-// that store.  The rows of the ring start out clear: a launch uses one of two
-// rings and clears its slots of the other one.
-//
-// Vectors that other workgroups gather (the next Arnoldi vector, x before the
-// residual) are written with agent-scope stores that complete (s_waitcnt
-// vmcnt(0)) before the partial that announces them is stored, and are
-// gathered with agent-scope loads; no cache-wide write-back or invalidation
-// is needed.  Every wait is bounded: after `spin` polls a workgroup raises
-// the abort flag and leaves, and the others leave at their next look at it.
-//
-// The first exchange of a launch shows that its workgroups are resident
-// together: each stays until it has seen the others' slots.  If something
-// else holds the CUs (another process's launch, half of it waiting for this
-// one's other half), that exchange ends after start_spin polls, and the host
-// launches again: x and the state of the columns are written only after
-// later exchanges, so nothing is lost.  Within a process launches take turns
-// (launch_mutex).  A cooperative launch would give the same guarantee but is
-// refused to every process of a GPU except the first that asks.
-struct Hop {
-    xch_t* ring;
-    int G, bid, e;  // G: slots of a row (padded workgroup count)
-    long spin, start_spin;
-    int *abort_dev, *abort_host;
-};
-
-inline int hop_slots(int G)
-{
-    return G <= 16 ? 16 : G <= 48 ? 48 : G <= 96 ? 96 : G <= 176 ? 176 : 256;
-}
-
-struct HopLds {
-    double w[KR_BS / 64][33];  // partials of the wavefronts
-    double g[KR_GRP][33];      // sums of the thread groups
-    int bad, cont;
-};
-
-template <int NQ>
-__device__ __forceinline__ bool hop_poll(const Hop& h, const xch_t* row, int val, double* sum)
-{
-    const long spin = h.e == 0 ? h.start_spin : h.spin;
-    const unsigned off = ((threadIdx.x >> 5) * XCH_V + val) * (unsigned)sizeof(xch_t);
-    xch_t u[NQ];
-    bool ok = false, left = false;
-    for (long it = 0; it < spin; ++it) {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q)
-            u[q] = ld_agent((const xch_t*)((const char*)(row + KR_GRP * q * XCH_V) + off));
-        bool all = true;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) all = all & (u[q] != XCH_EMPTY);
-        if (__all(all)) {
-            ok = true;
-            break;
-        }
-        if ((it & 63) == 63 && ld_agent(h.abort_dev)) {
-            left = true;
-            break;
-        }
-    }
-    if (!ok && !left) {
-        st_agent(h.abort_dev, 1);
-        __hip_atomic_fetch_or(h.abort_host, h.e == 0 ? ABORT_START : ABORT_WAIT, __ATOMIC_RELAXED,
-                              __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    double a[2] = {0.0, 0.0};
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        a[q & 1] += __longlong_as_double((long long)u[q]);
-    *sum = a[0] + a[1];
-    return ok;
-}
-
-enum { HOP_OK = 0, HOP_STOP = 1, HOP_FAIL = 2 };
-
-// The exchange of values 0..nv-1 and, with `last`, of value 31, from the
-// wavefronts' partials in l->w; lane i of every wavefront returns the total
-// of value i & 31.  With `check`, HOP_STOP when l->cont (written before) is
-// 0: every workgroup of the column decides the same.
-__device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool check, HopLds* l, double* tot)
-{
-    const int t = threadIdx.x, i = t & 31;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's stores are complete
-    __syncthreads();
-    if (check && !l->cont) return HOP_STOP;
-    xch_t* row = h.ring + (size_t)(h.e & (XCH_RING - 1)) * h.G * XCH_V;
-    const bool mine = i < nv || (last && i == 31);
-    if (t < 32 && mine) {
-        double r = 0.0;
-#pragma unroll
-        for (int q = 0; q < KR_BS / 64; ++q) r += l->w[q][i];
-        st_agent(row + (size_t)h.bid * XCH_V + i, (xch_t)__double_as_longlong(r));
-    }
-    if (t >= 64 && t < 96)
-        st_agent(h.ring + ((size_t)((h.e + 2) & (XCH_RING - 1)) * h.G + h.bid) * XCH_V + i, XCH_EMPTY);
-    const int val = mine ? i : (nv > 0 ? 0 : 31);
-    double sum = 0.0;
-    bool ok;
-    if (h.G == 16) ok = hop_poll<1>(h, row, val, &sum);
-    else if (h.G == 48) ok = hop_poll<3>(h, row, val, &sum);
-    else if (h.G == 96) ok = hop_poll<6>(h, row, val, &sum);
-    else if (h.G == 176) ok = hop_poll<11>(h, row, val, &sum);
-    else ok = hop_poll<16>(h, row, val, &sum);
-    l->g[t >> 5][i] = sum;
-    if (!ok) l->bad = 1;
-    __syncthreads();
-    *tot = krylov_join(l->g, i);
-    ++h.e;
-    return l->bad ? HOP_FAIL : HOP_OK;
-}
-
-// --------------------------------------------------------------- kernel --
-template <typename VT, typename MT>
-struct PArgs {
-    int n, ld, G, Gp, m, width, width64;
-    const int* col;
-    const MT* val;
-    const int* col64;
-    const double* val64;
-    const double* dscale;  // x += dscale * (V y), or null
-    const double* B;       // row-major, ld columns; column q at q
-    double* X;
-    VT* W;                 // a vector of ldw per column
-    size_t ldw;
-    xch_t *ring, *other;   // XCH_RING rows of Gp slots per column
-    PState *st, *host;
-    int *abort_dev, *abort_host;
-    long spin, start_spin;
-    double rtol, inner_rtol;
-    int max_iters, max_cycles, first, use_x0, stall;
-};
-
-// ||.||^2 of a thread's rows, as the block partial of value `i`
-template <typename T>
-__device__ __forceinline__ void put_norm(const T (&w)[KR_RPT], int i, HopLds* l)
-{
-    double a = 0.0;
-#pragma unroll
-    for (int r = 0; r < KR_RPT; ++r) a = fma(to_d(w[r]), to_d(w[r]), a);
-    a = wave_sum(a);
-    if ((threadIdx.x & 63) == 0) l->w[threadIdx.x >> 6][i] = a;
-}
-
-// A thread's rows of the basis, in tiers of KR_T vectors: the first ones in
-// LDS (16 FP64 vectors or all 32 FP32 ones of 1024 rows are 128 of the 160
-// KB), the others in registers.  All 32 in registers spilled 409 of them.
-template <typename VT>
-struct Basis {
-    static constexpr int TIERS = PS_M / KR_T;
-    static constexpr int LDS_TIERS = sizeof(VT) == 8 ? TIERS / 2 : TIERS;
-    static constexpr int REG_TIERS = TIERS > LDS_TIERS ? TIERS - LDS_TIERS : 1;
-    VT* lds;  // [vector][row of the workgroup], this thread's first row
-    VT reg[REG_TIERS][KR_T][KR_RPT];
-
-    __device__ __forceinline__ VT at(int t, int i, int r) const
-    {
-        return t < LDS_TIERS ? lds[(t * KR_T + i) * KR_ROWS + r * KR_BS]
-                             : reg[t < LDS_TIERS ? 0 : t - LDS_TIERS][i][r];
-    }
-    // zeros: tiers are read whole, and what is not a basis vector yet must be
-    // finite there (a vector w / ||w|| with ||w|| = 0 is put as zeros too)
-    __device__ __forceinline__ void clear()
-    {
-#pragma unroll
-        for (int i = 0; i < LDS_TIERS * KR_T; ++i)
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) lds[i * KR_ROWS + r * KR_BS] = VT(0);
-#pragma unroll
-        for (int u = 0; u < REG_TIERS; ++u)
-#pragma unroll
-            for (int i = 0; i < KR_T; ++i)
-#pragma unroll
-                for (int r = 0; r < KR_RPT; ++r) reg[u][i][r] = VT(0);
-    }
-    __device__ __forceinline__ void put(int j, const VT (&v)[KR_RPT])
-    {
-        if (j < LDS_TIERS * KR_T) {
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) lds[j * KR_ROWS + r * KR_BS] = v[r];
-        } else {
-#pragma unroll
-            for (int u = 0; u < TIERS - LDS_TIERS; ++u) {
-                if (u + LDS_TIERS != j / KR_T) continue;
-#pragma unroll
-                for (int i = 0; i < KR_T; ++i)
-#pragma unroll
-                    for (int r = 0; r < KR_RPT; ++r)
-                        reg[u][i][r] = i == j % KR_T ? v[r] : reg[u][i][r];
-            }
-        }
-    }
-};
-
-// partials of the dots of w with v_0..v_j
-template <typename VT>
-__device__ __forceinline__ void put_dots(int j, const VT (&w)[KR_RPT], const Basis<VT>& V,
-                                         HopLds* l)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int t = 0; t < Basis<VT>::TIERS; ++t) {
-        if (t * KR_T > j) break;
-        VT v[KR_T][KR_RPT];
-        double p[KR_T];
-#pragma unroll
-        for (int i = 0; i < KR_T; ++i)
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) v[i][r] = V.at(t, i, r);
-        dots_tier<VT>(w, v, p);
-        const double s = reduce8(p);
-        const int i = t * KR_T + reduce8_value(lane);
-        if ((lane & 7) == 0 && i <= j) l->w[threadIdx.x >> 6][i] = s;
-    }
-}
-
-// w -= sum_{i<=j} h_i v_i (lane i of the wavefront holds h_i)
-template <typename VT>
-__device__ __forceinline__ void take_off(int j, double h, VT (&w)[KR_RPT], const Basis<VT>& V)
-{
-#pragma unroll
-    for (int t = 0; t < Basis<VT>::TIERS; ++t) {
-        if (t * KR_T > j) break;
-        VT v[KR_T][KR_RPT];
-#pragma unroll
-        for (int i = 0; i < KR_T; ++i)
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) v[i][r] = V.at(t, i, r);
-#pragma unroll
-        for (int i = 0; i < KR_T; ++i) {
-            // entries past j (finite: see put) take no part
-            const VT hv = t * KR_T + i <= j ? (VT)readlane_d(h, t * KR_T + i) : VT(0);
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) w[r] = kfma(-hv, v[i][r], w[r]);
-        }
-    }
-}
-
-template <typename VT, typename MT, int ORTHO>
-__global__ void __launch_bounds__(KR_BS)
-k_persist(PArgs<VT, MT> a)
-{
-    __shared__ VT sV[Basis<VT>::LDS_TIERS * KR_T * KR_ROWS];
-    __shared__ HopLds l;
-    __shared__ double sL[PS_M * 33];  // <v_i, v_k>, k < i
-    __shared__ double sR[PS_M * 33];
-    __shared__ double s_cs[2 * PS_M], s_g[PS_M], s_carry[PS_M + 1], s_y[PS_M];
-    __shared__ double s_h[PS_M + 8];  // Hessenberg column of the last step
-    const int t = threadIdx.x, lane = t & 63, li = lane & 31;
-    const int q = (int)blockIdx.x / a.G, bid = (int)blockIdx.x % a.G;
-    const int n = a.n, ld = a.ld, m = a.m;
-    Hop h{a.ring + (size_t)q * XCH_RING * a.Gp * XCH_V, a.Gp, bid, 0, a.spin, a.start_spin,
-          a.abort_dev, a.abort_host};
-    if (t < XCH_RING * XCH_V)
-        st_agent(a.other + (size_t)q * XCH_RING * a.Gp * XCH_V +
-                     ((size_t)(t >> 5) * a.Gp + bid) * XCH_V + (t & 31), XCH_EMPTY);
-    if (t == 0) l.bad = 0;
-    const int base = bid * KR_ROWS + t;
-    const double* B = a.B + q;
-    double* X = a.X + q;
-    VT* W = a.W + (size_t)q * a.ldw;
-
-    VT w[KR_RPT];
-    double bnorm = 1.0, beta = 0.0, rel = 0.0, tot = 0.0;
-    int iters = 0, cycles = 0, converged = 0, active = 0;
-    if (a.first) {
-        // x, ||b|| and the first residual; with x = 0 that is b
-        double b[KR_RPT], r0[KR_RPT], xo[KR_RPT], ax[KR_RPT];
-#pragma unroll
-        for (int r = 0; r < KR_RPT; ++r) {
-            const int rr = base + r * KR_BS;
-            b[r] = rr < n ? B[(size_t)rr * ld] : 0.0;
-            r0[r] = b[r];
-        }
-        if (a.use_x0) {
-            krylov_rows<double, double, false, KR_RPT>(n, a.width64, base, a.col64, a.val64, X, ld,
-                                                       1.0, xo, ax);
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) r0[r] = b[r] - ax[r];
-        }
-#pragma unroll
-        for (int r = 0; r < KR_RPT; ++r) {
-            const int rr = base + r * KR_BS;
-            if (rr < n && !a.use_x0) st_agent(X + (size_t)rr * ld, 0.0);
-            w[r] = (VT)r0[r];
-            if (rr < n) st_agent(W + rr, w[r]);
-        }
-        put_norm(b, 0, &l);
-        put_norm(r0, 1, &l);
-        if (hop(h, 2, false, false, &l, &tot) != HOP_OK) return;
-        bnorm = sqrt(readlane_d(tot, 0));
-        if (!(bnorm > 0.0)) bnorm = 1.0;
-        beta = sqrt(readlane_d(tot, 1));
-        rel = beta / bnorm;
-        if (rel <= a.rtol || beta == 0.0) converged = 1;
-        else active = iters < a.max_iters && (!a.stall || isfinite(beta));
-        if (active) ++cycles;
-    } else {
-        const PState s = a.st[q];
-        bnorm = s.bnorm, beta = s.beta, rel = s.rel;
-        iters = s.iters, cycles = s.cycles, converged = s.converged, active = s.active;
-#pragma unroll
-        for (int r = 0; r < KR_RPT; ++r) {
-            const int rr = base + r * KR_BS;
-            w[r] = rr < n ? W[rr] : VT(0);
-        }
-    }
-
-    // the thread's matrix rows (past a row's width its last slot again, past
-    // row n row n - 1: every load is in bounds), and its rows of the basis
-    const bool pre = a.width >= 1 && a.width <= ELL_MAXW;
-    unsigned sc[KR_RPT][ELL_MAXW];  // byte offsets into W
-    MT sv[KR_RPT][ELL_MAXW];
-    if (pre && active) {
-#pragma unroll
-        for (int r = 0; r < KR_RPT; ++r) {
-            const int rr = min(base + r * KR_BS, n - 1);
-#pragma unroll
-            for (int k = 0; k < ELL_MAXW; ++k) {
-                const size_t o = ell_slot(k, a.width, n, rr);
-                sc[r][k] = (unsigned)a.col[o] * (unsigned)sizeof(VT);
-                sv[r][k] = a.val[o];
-            }
-        }
-    }
-    Basis<VT> V;
-    V.lds = sV + t;
-    V.clear();
-
-    for (int run = 0; active && run < a.max_cycles; ++run) {
-        const int iters0 = iters;
-        const double stop = fmax(a.rtol * bnorm, a.inner_rtol * beta);
-        if (t == 0) s_carry[0] = beta;
-        double hn = beta;
-        int j = 0, rc = HOP_OK;
-        for (;; ++j) {
-            // v_j = w / hn; w = A v_j, whose gathers are in flight while the
-            // first wavefront rotates the column of step j - 1
-            const VT inv = (VT)(1.0 / hn);
-            VT vj[KR_RPT], xv[KR_RPT][ELL_MAXW];
-            if (j < m) {
-#pragma unroll
-                for (int r = 0; r < KR_RPT; ++r) vj[r] = hn > 0.0 ? w[r] * inv : VT(0);
-                if (pre) {
-#pragma unroll
-                    for (int r = 0; r < KR_RPT; ++r)
-#pragma unroll
-                        for (int k = 0; k < ELL_MAXW; ++k) xv[r][k] = ld_agent((const VT*)((const char*)W + sc[r][k]));
-                }
-            }
-            if (j > 0 && t < 64) {
-                const GivensOut g = krylov_givens(j - 1, m, s_h, hn, stop, iters0, a.max_iters,
-                                                  s_cs, s_g, s_carry, sR, 33);
-                if (lane == 0) l.cont = g.cont;
-            }
-            if (j == m) break;
-            if (pre) {
-#pragma unroll
-                for (int r = 0; r < KR_RPT; ++r) {
-                    VT s = VT(0);
-#pragma unroll
-                    for (int k = 0; k < ELL_MAXW; ++k) {
-                        const VT u = RowTerm<VT, MT>::add(s, sv[r][k], xv[r][k], inv);
-                        s = k < a.width ? u : s;
-                    }
-                    w[r] = base + r * KR_BS < n ? s : VT(0);
-                }
-            } else {
-                VT xo[KR_RPT];
-                krylov_rows_loop<VT, MT, true, KR_RPT>(n, a.width, opaque(base), a.col, a.val, W,
-                                                       1, inv, xo, w);
-            }
-            V.put(j, vj);
-            put_dots<VT>(j, w, V, &l);
-            rc = hop(h, j + 1, false, j > 0, &l, &tot);
-            if (rc != HOP_OK) break;
-            double hcol = tot;
-            if (ORTHO == PHG_MGS) hcol = mgs_solve<PS_M>(tot, j, sL, 33, li);
-            take_off<VT>(j, hcol, w, V);
-            if (ORTHO == PHG_CGS2) {
-                put_dots<VT>(j, w, V, &l);
-                rc = hop(h, j + 1, false, false, &l, &tot);
-                if (rc != HOP_OK) break;
-                take_off<VT>(j, tot, w, V);
-                hcol += tot;
-            }
-            if (t < PS_M) s_h[t] = hcol;
-#pragma unroll
-            for (int r = 0; r < KR_RPT; ++r) {
-                const int rr = base + r * KR_BS;
-                if (rr < n) st_agent(W + rr, w[r]);
-            }
-            const bool more = ORTHO == PHG_MGS && j + 1 < m;
-            put_norm(w, 31, &l);
-            if (more) put_dots<VT>(j, w, V, &l);
-            rc = hop(h, more ? j + 1 : 0, true, false, &l, &tot);
-            if (rc != HOP_OK) break;
-            hn = sqrt(readlane_d(tot, 31));
-            if (more && t <= j) sL[(j + 1) * 33 + t] = tot * to_d((VT)(1.0 / hn));
-        }
-        if (rc == HOP_FAIL) return;
-        // j steps are complete: y = R^-1 g, x += V y
-        iters = iters0 + j;
-        __syncthreads();
-        if (t < 64) {
-            const double y = krylov_solve_y(j, sR, 33, s_g);
-            if (lane < PS_M) s_y[lane] = y;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < KR_RPT; ++r) {
-            const int rr = opaque(base) + r * KR_BS;
-            double s = 0.0;  // y is 0 past step j
-#pragma unroll
-            for (int i = 0; i < PS_M; ++i) s = fma(to_d(V.at(i / KR_T, i % KR_T, r)), s_y[i], s);
-            if (rr < n) {
-                if (a.dscale) s = a.dscale[rr] * s;
-                double* x = X + (size_t)rr * ld;
-                st_agent(x, ld_agent(x) + s);
-            }
-        }
-        if (lane == 0) l.w[t >> 6][0] = 0.0;
-        if (hop(h, 1, false, false, &l, &tot) != HOP_OK) return;
-        // r = b - A x in FP64, the next cycle's vector
-        double res[KR_RPT], xo[KR_RPT];
-        const int rb = opaque(base);
-        krylov_rows<double, double, true, KR_RPT>(n, a.width64, rb, a.col64, a.val64, X, ld, 1.0,
-                                                  xo, res);
-#pragma unroll
-        for (int r = 0; r < KR_RPT; ++r) {
-            const int rr = rb + r * KR_BS;
-            res[r] = rr < n ? B[(size_t)rr * ld] - res[r] : 0.0;
-            w[r] = (VT)res[r];
-            if (rr < n) st_agent(W + rr, w[r]);
-        }
-        put_norm(res, 0, &l);
-        if (hop(h, 1, false, false, &l, &tot) != HOP_OK) return;
-        const double now = sqrt(readlane_d(tot, 0));
-        const bool stalled = a.stall && iters > iters0 && now > 0.99 * beta;
-        beta = now;
-        rel = beta / bnorm;
-        if (rel <= a.rtol || beta == 0.0) {
-            converged = 1;
-            active = 0;
-        } else if (iters >= a.max_iters || stalled || (a.stall && !isfinite(beta))) {
-            active = 0;
-        } else {
-            ++cycles;
-        }
-    }
-    if (bid == 0 && t == 0) {
-        PState s;
-        s.bnorm = bnorm, s.beta = beta, s.rel = rel;
-        s.iters = iters, s.cycles = cycles, s.converged = converged, s.active = active;
-        a.st[q] = s;
-        a.host[q] = s;
-    }
-}
-
-// Clears both rings (slots past the last workgroup: 0) and the abort flag.
-__global__ void k_ring_reset(xch_t* ring, size_t count, int G, int Gp, int* abort_dev)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) ring[i] = (int)(i / XCH_V % Gp) < G ? XCH_EMPTY : 0;
-    if (i == 0) *abort_dev = 0;
-}
-
 // Launches of one device take turns: two that each hold half of the CUs would
 // wait for each other until they give up.
-std::mutex& launch_mutex(int dev)
+std::mutex& persist_mutex(int dev)
 {
     static std::mutex m[64];
     return m[dev & 63];
 }
 
-// Workgroups of the kernel that the device holds at once, per template
-// instance, computed once (thread-safe static initialisation).
-template <typename VT, typename MT, int ORTHO>
-int capacity()
-{
-    static const int n = [] {
-        int dev = 0, cus = 0, per = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per, (const void*)k_persist<VT, MT, ORTHO>, KR_BS, 0) != hipSuccess)
-            return 0;
-        return cus * per;
-    }();
-    return n;
-}
-
-// Columns q0 .. q0 + K - 1 of the ld in B and X.
-template <typename VT, typename MT, int ORTHO>
-int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int ld, const double* B,
-           double* X, const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles,
-           int first, hipStream_t s)
-{
-    const int n = A->n_rows, G = (n + KR_ROWS - 1) / KR_ROWS, Gp = hop_slots(G);
-    const size_t ldw = ((size_t)n + 63) / 64 * 64, slots = (size_t)K * XCH_RING * Gp * XCH_V;
-    if (w->ring_k != K || w->ring_g != G) {
-        // another shape than the last launch's, or after a give-up
-        hipLaunchKernelGGL(k_ring_reset, dim3((unsigned)((2 * slots + 255) / 256)), dim3(256), 0, s,
-                           w->xch.p(), 2 * slots, G, Gp, w->abort_dev.p);
-        PHG_HIP(hipGetLastError());
-        w->ring_k = K;
-        w->ring_g = G;
-    }
-    PArgs<VT, MT> a;
-    a.n = n, a.ld = ld, a.G = G, a.Gp = Gp, a.m = o.restart, a.width = E.width;
-    a.width64 = A->ell64.width;
-    a.col = E.col.p, a.val = E.val.p, a.col64 = A->ell64.col.p, a.val64 = A->ell64.val.p;
-    a.dscale = dscale, a.B = B + q0, a.X = X + q0, a.W = (VT*)w->W.p + (size_t)q0 * ldw, a.ldw = ldw;
-    a.ring = w->xch.p() + (w->parity ? slots : 0);
-    a.other = w->xch.p() + (w->parity ? 0 : slots);
-    w->parity ^= 1;
-    a.st = w->st.p + q0, a.host = w->host + q0;
-    a.abort_dev = w->abort_dev.p, a.abort_host = (int*)(w->host + w->host_k);
-    a.spin = XCH_SPIN;
-    if (const char* e = getenv("PHG_XCH_SPIN")) a.spin = std::max(1L, atol(e));
-    a.start_spin = std::min(a.spin, XCH_START);
-    a.rtol = o.rtol;
-    a.inner_rtol = o.precision == PHG_F64 ? 0.0 : o.inner_rtol;
-    a.max_iters = o.max_iters, a.max_cycles = max_cycles, a.use_x0 = o.use_x0;
-    a.stall = stall, a.first = first;
-    for (int q = q0; q < q0 + K; ++q) w->host[q].active = -1;  // until the kernel writes it
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_persist<VT, MT, ORTHO>), dim3(G * K), dim3(KR_BS), 0, s, a);
-    PHG_HIP(hipGetLastError());
-    return PHG_OK;
-}
-
-template <typename VT, typename MT, int ORTHO>
-int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
-        const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles, int max_rounds,
-        int* launches, double* ms, hipStream_t s)
-{
-    const int n = A->n_rows, G = (n + KR_ROWS - 1) / KR_ROWS;
-    // columns of a launch, and launches for all columns, of equal size
-    const int fit = std::min(capacity<VT, MT, ORTHO>(), XCH_MAXG) / G;
-    if (fit < 1) return PERSIST_NOT_HERE;
-    const int rounds = (K + fit - 1) / fit, per = (K + rounds - 1) / rounds;
-    if (rounds > max_rounds) return PERSIST_NOT_HERE;
-    const size_t ldw = ((size_t)n + 63) / 64 * 64;
-    const size_t slots = (size_t)per * XCH_RING * hop_slots(G) * XCH_V;
-    const size_t bytes = (size_t)K * ldw * sizeof(VT);
-    if (w->W.n < bytes) PHG_HIP(w->W.alloc(bytes));
-    if (w->host_k < K) {
-        if (w->host) (void)hipHostFree(w->host);
-        w->host = nullptr;
-        w->host_k = 0;
-        PHG_HIP(w->st.alloc(K));
-        // K states, then the abort word
-        PHG_HIP(hipHostMalloc((void**)&w->host, sizeof(PState) * (K + 1), hipHostMallocDefault));
-        w->host_k = K;
-    }
-    if (!w->abort_dev.p) PHG_HIP(w->abort_dev.alloc(1));
-    if (w->ring_slots < slots) {
-        w->ring_slots = 0;
-        PHG_HIP(w->xch.alloc(2 * slots));
-        w->ring_slots = slots;
-        w->ring_k = 0;
-    }
-    if (ms && !w->ev[0]) {
-        PHG_HIP(hipEventCreate(&w->ev[0]));
-        PHG_HIP(hipEventCreate(&w->ev[1]));
-    }
-    int dev = 0;
-    PHG_HIP(hipGetDevice(&dev));
-    std::unique_lock<std::mutex> turn(launch_mutex(dev), std::try_to_lock);
-    if (!turn.owns_lock()) {
-        // another thread's solve runs: wait for this stream's earlier work
-        // first, so that nobody waits for that while it is this one's turn
-        PHG_HIP(hipStreamSynchronize(s));
-        turn.lock();
-    }
-    volatile int* abort_host = (int*)(w->host + w->host_k);
-    int tries = 0;
-    for (int first = 1;; first = 0) {
-        for (int q = 0; q < K; ++q)
-            if (first) w->host[q].active = 1;
-        // the columns still running, and one by one those of a launch that
-        // did not start
-        for (bool again = false;; again = true) {
-            *abort_host = 0;
-            if (ms) PHG_HIP(hipEventRecord(w->ev[0], s));
-            const int step = again ? 1 : per;
-            for (int q0 = 0; q0 < K; q0 += step) {
-                const int kq = std::min(step, K - q0);
-                bool any = false;
-                for (int q = q0; q < q0 + kq; ++q)
-                    any = any || (again ? w->host[q].active == -1 : w->host[q].active == 1);
-                if (!any) continue;
-                const int rc = launch<VT, MT, ORTHO>(A, E, w, q0, kq, K, B, X, o, dscale, stall,
-                                                     max_cycles, first, s);
-                if (rc) return rc;
-                if (launches) ++*launches;
-            }
-            if (ms) PHG_HIP(hipEventRecord(w->ev[1], s));
-            const hipError_t e = hipStreamSynchronize(s);
-            if (e != hipSuccess) w->ring_k = 0;
-            PHG_HIP(e);
-            if (ms) {
-                float t = 0.0f;
-                PHG_HIP(hipEventElapsedTime(&t, w->ev[0], w->ev[1]));
-                *ms += t;
-            }
-            if (!*abort_host) break;
-            w->ring_k = 0;
-            if ((*abort_host & ABORT_WAIT) || ++tries >= XCH_TRIES) {
-                set_error("gmres: a workgroup of the persistent solve timed out waiting for the "
-                          "others");
-                return PHG_ERR_HIP;
-            }
-            // two processes that collided do not try again at the same moment
-            std::this_thread::sleep_for(std::chrono::microseconds(100 * (1 + (getpid() * 7 + tries) % 32)));
-        }
-        bool any = false;
-        for (int q = 0; q < K; ++q) any = any || w->host[q].active;
-        if (!any) break;
-    }
-    return PHG_OK;
-}
-
-template <typename VT, typename MT, typename... Rest>
-int run_ortho(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
-              const phg_gmres_opts& o, Rest... rest)
-{
-    switch (o.ortho) {
-    case PHG_MGS: return run<VT, MT, PHG_MGS>(A, E, w, K, B, X, o, rest...);
-    case PHG_CGS2: return run<VT, MT, PHG_CGS2>(A, E, w, K, B, X, o, rest...);
-    default: return run<VT, MT, PHG_CGS1>(A, E, w, K, B, X, o, rest...);
-    }
-}
-
-}  // namespace
-
 void persist_destroy(PersistWork* w) { delete w; }
 
+int persist_solve_small(phg_matrix_s* A, PersistWork* w, int K, const double* B, double* X,
+                        const phg_gmres_opts& o, bool diag, bool stall, int max_cycles,
+                        int max_rounds, int* launches, double* ms, hipStream_t s);
+
+// Workgroups of 256 threads wherever all columns fit the device with them: a
+// SIMD then runs one wavefront instead of two, and a step is instructions
+// beside its exchanges; the results are the same bits.  Measured with 512 and
+// with 256 threads: level 4 FP64 MGS 371 and 305 us a solve, 7 columns of
+// 9,991 rows FP64 CGS2 1.03 and 0.85 ms, 36,503 rows FP32 CGS2 1.89 and
+// 1.88 ms.  Columns that would need more launches than with 512 threads are
+// faster with those.
 int persist_solve(phg_matrix_s* A, PersistWork* w, int K, const double* B, double* X,
                   const phg_gmres_opts& o, bool diag, bool stall, int max_cycles, int max_rounds,
                   int* launches, double* ms, hipStream_t s)
 {
-    if (o.restart > PS_M || A->n_rows > KR_ROWS * XCH_MAXG) return PERSIST_NOT_HERE;
-    const double* none = nullptr;
-    if (o.precision == PHG_F64)
-        return run_ortho<double, double>(A, diag ? A->ell64d : A->ell64, w, K, B, X, o,
-                                         diag ? (const double*)A->dinv.p : none, stall, max_cycles,
-                                         max_rounds, launches, ms, s);
-    if (o.precision == PHG_F32)
-        return run_ortho<float, float>(A, A->ell32, w, K, B, X, o, none, stall, max_cycles,
-                                       max_rounds, launches, ms, s);
-    return run_ortho<float, uint16_t>(A, A->ell16, w, K, B, X, o, none, stall, max_cycles,
-                                      max_rounds, launches, ms, s);
+    if ((long)persist_workgroups(A->n_rows, 256) * K <= KR_MAXG) {
+        const int rc = persist_solve_small(A, w, K, B, X, o, diag, stall, max_cycles, max_rounds,
+                                           launches, ms, s);
+        if (rc != PERSIST_NOT_HERE) return rc;
+    }
+    return solve(A, w, K, B, X, o, diag, stall, max_cycles, max_rounds, launches, ms, s);
 }
 
 }  // namespace phg

@@ -145,3 +145,27 @@ def test_batch_persistent_and_launches(n, K, opts):
         for i, q in enumerate(some):
             assert torch.equal(Z[:, i], X[:, q]), q
     A.close()
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 512, 513, 768, 769, 1280, 1281, 23553, 24833, 49000,
+                               90113, 131072, 131073])
+@pytest.mark.parametrize("precision", [P.F64, P.F32])
+def test_half_workgroups_same_bits(n, precision):
+    """Workgroups of 256 threads (up to 131,072 rows) at their edges: halves
+    of a 1024-row block that are missing, partly filled or full, and the row
+    lengths of the exchange.  Same bits as the launches, whose blocks are
+    always whole."""
+    _check(n, 7, ortho=P.MGS, precision=precision, restart=30)
+
+
+@pytest.mark.parametrize("n,K", [(2304, 64), (2305, 64), (33000, 4)])
+def test_half_and_whole_workgroups_same_column(n, K):
+    """K columns take workgroups of 512 threads, two of them 256."""
+    csr = _line(n, 7, n)
+    A = P.Matrix.from_csr(n, n, *csr)
+    B = torch.as_tensor(np.random.default_rng(n).standard_normal((n, K)), device=DEV)
+    X, its, done = _batch(A, B, None, 1, ortho=P.CGS2)
+    Z, some, _ = _batch(A, B[:, [0, K - 1]].contiguous(), None, 1, ortho=P.CGS2)
+    assert all(done) and some == [its[0], its[-1]]
+    assert torch.equal(Z, X[:, [0, K - 1]])
+    A.close()
