@@ -465,9 +465,9 @@ def l7_system(stream):
 
 
 def solve_only_leg(steps, warmup, stream, only=None):
-    """The level-7 single right-hand-side forms alone: FP64 MGS as a
-    persistent cooperative cycle and as a kernel per MGS pass, FP64 CGS2,
-    mixed FP32 MGS (persistent) and CGS2."""
+    """The level-7 single right-hand-side forms alone: FP64 MGS with
+    persistent restart cycles and with launches per pass, FP64 CGS2, mixed
+    FP32 MGS and CGS2."""
     import torch
 
     import mke_amd as P
@@ -943,11 +943,11 @@ def main():
                     cold_avg_launch_us=round(cold_ms * 1e3, 3))
     if cyc is not None:
         out["roofline"] = {
-            "bound": "hbm", "kernel": "k_mgs_cycle<double,double> (one GMRES(30) restart cycle, "
-                                      "MGS; latency-bound chain of dependent global sums)",
+            "bound": "hbm", "kernel": "k_persist<double,double> (one GMRES(30) restart cycle, MGS, "
+                                      "the basis on the chip; two exchanges of global sums a step)",
             "achieved": cyc["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(cyc["achieved"] / HBM_PEAK_GBS, 4),
-            "traffic": traffic_from_profiles("k_mgs_cycle_L7_traffic.json"),
+            "traffic": traffic_from_profiles("k_persist_L7_traffic.json"),
             "bytes_per_launch": cyc["bytes_per_launch"], "avg_launch_us": cyc["avg_launch_us"],
             "launches_per_solve": cyc["launches_per_solve"],
             "whole_solve": whole, "spmv": spmv}

@@ -143,14 +143,18 @@ enum { HOP_OK = 0, HOP_STOP = 1, HOP_FAIL = 2 };
 
 // The exchange of values 0..nv-1 and, with `last`, of value 31, from the
 // wavefronts' partials in l->w; lane i of every wavefront returns the total
-// of value i & 31.  With `check`, HOP_STOP when l->cont (written before) is
-// 0: every workgroup of the column decides the same.
-__device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool check, HopLds* l, double* tot)
+// of value i & 31.  The last wavefront runs `meanwhile` once the partials are
+// on their way, and polls after it.  HOP_STOP when l->cont is 0, with `early`
+// before the exchange, with `check` after it (meanwhile may write it): every
+// workgroup of the column decides the same.
+template <typename F>
+__device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool early, bool check, HopLds* l,
+                                   double* tot, F meanwhile)
 {
     const int t = threadIdx.x, i = t & 31;
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's stores are complete
     __syncthreads();
-    if (check && !l->cont) return HOP_STOP;
+    if (early && !l->cont) return HOP_STOP;
     xch_t* row = h.ring + (size_t)(h.e & (XCH_RING - 1)) * h.G * XCH_V;
     const bool mine = i < nv || (last && i == 31);
     if (t < 32 && mine) {
@@ -162,6 +166,7 @@ __device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool check, HopLds
     }
     if (t >= 64 && t < 96)
         st_agent(h.ring + ((size_t)((h.e + 2) & (XCH_RING - 1)) * h.G + h.slot) * XCH_V + i, XCH_EMPTY);
+    if (t >= BS - 64) meanwhile();
     const int val = mine ? i : (nv > 0 ? 0 : 31);
     double sum[16 / GRP];
     bool ok;
@@ -176,7 +181,11 @@ __device__ __forceinline__ int hop(Hop& h, int nv, bool last, bool check, HopLds
     __syncthreads();
     *tot = krylov_join(l->g, i);
     ++h.e;
-    return l->bad ? HOP_FAIL : HOP_OK;
+    return l->bad ? HOP_FAIL : check && !l->cont ? HOP_STOP : HOP_OK;
+}
+__device__ __forceinline__ int hop(Hop& h, int nv, bool last, HopLds* l, double* tot)
+{
+    return hop(h, nv, last, false, false, l, tot, [] {});
 }
 
 // --------------------------------------------------------------- kernel --
@@ -319,6 +328,9 @@ k_persist(PArgs<VT, MT> a)
     __shared__ double s_h[PS_M + 8];  // Hessenberg column of the last step
     const int t = threadIdx.x, lane = t & 63, li = lane & 31;
     const int q = (int)blockIdx.x / a.G, bid = (int)blockIdx.x % a.G;
+    // (512 threads with FP64 vectors spill 160 registers with it: 10.1 ms
+    // instead of 5.0 at level 7)
+    constexpr bool LATE = BS == 256 || sizeof(VT) == 4;
     const int n = a.n, ld = a.ld, m = a.m, slot = slot_of(bid, a.Gp);
     Hop h{a.ring + (size_t)q * XCH_RING * a.Gp * XCH_V, a.Gp, slot, 0, a.spin, a.start_spin,
           a.abort_dev, a.abort_host};
@@ -358,7 +370,7 @@ k_persist(PArgs<VT, MT> a)
         }
         put_norm(b, 0, &l);
         put_norm(r0, 1, &l);
-        if (hop(h, 2, false, false, &l, &tot) != HOP_OK) return;
+        if (hop(h, 2, false, &l, &tot) != HOP_OK) return;
         bnorm = sqrt(readlane_d(tot, 0));
         if (!(bnorm > 0.0)) bnorm = 1.0;
         beta = sqrt(readlane_d(tot, 1));
@@ -405,8 +417,10 @@ k_persist(PArgs<VT, MT> a)
         double hn = beta;
         int j = 0, rc = HOP_OK;
         for (;; ++j) {
-            // v_j = w / hn; w = A v_j, whose gathers are in flight while the
-            // first wavefront rotates the column of step j - 1
+            // v_j = w / hn; w = A v_j.  The column of step j - 1 is rotated
+            // while the dots are exchanged (level 4 FP64 MGS 305 -> 292 us a
+            // solve, 36,503 rows FP32 CGS2 1.88 -> 1.73 ms), or by the first
+            // wavefront while the gathers are in flight
             const VT inv = (VT)(1.0 / hn);
             VT vj[KR_RPT], xv[KR_RPT][ELL_MAXW];
             if (j < m) {
@@ -419,12 +433,16 @@ k_persist(PArgs<VT, MT> a)
                         for (int k = 0; k < ELL_MAXW; ++k) xv[r][k] = ld_agent((const VT*)((const char*)W + sc[r][k]));
                 }
             }
-            if (j > 0 && t < 64) {
+            const auto rotate = [&] {
+                if (j == 0) return;
                 const GivensOut g = krylov_givens(j - 1, m, s_h, hn, stop, iters0, a.max_iters,
                                                   s_cs, s_g, s_carry, sR, 33);
                 if (lane == 0) l.cont = g.cont;
+            };
+            if (j == m || !LATE) {
+                if (t < 64) rotate();
+                if (j == m) break;
             }
-            if (j == m) break;
             if (pre) {
 #pragma unroll
                 for (int r = 0; r < KR_RPT; ++r) {
@@ -441,14 +459,16 @@ k_persist(PArgs<VT, MT> a)
             }
             V.put(j, vj);
             put_dots<VT>(j, w, V, &l);
-            rc = hop(h, j + 1, false, j > 0, &l, &tot);
+            rc = hop(h, j + 1, false, !LATE && j > 0, LATE && j > 0, &l, &tot, [&] {
+                if (LATE) rotate();
+            });
             if (rc != HOP_OK) break;
             double hcol = tot;
             if (ORTHO == PHG_MGS) hcol = mgs_solve<PS_M>(tot, j, sL, 33, li);
             take_off<VT>(j, hcol, w, V);
             if (ORTHO == PHG_CGS2) {
                 put_dots<VT>(j, w, V, &l);
-                rc = hop(h, j + 1, false, false, &l, &tot);
+                rc = hop(h, j + 1, false, &l, &tot);
                 if (rc != HOP_OK) break;
                 take_off<VT>(j, tot, w, V);
                 hcol += tot;
@@ -462,7 +482,7 @@ k_persist(PArgs<VT, MT> a)
             const bool more = ORTHO == PHG_MGS && j + 1 < m;
             put_norm(w, 31, &l);
             if (more) put_dots<VT>(j, w, V, &l);
-            rc = hop(h, more ? j + 1 : 0, true, false, &l, &tot);
+            rc = hop(h, more ? j + 1 : 0, true, &l, &tot);
             if (rc != HOP_OK) break;
             hn = sqrt(readlane_d(tot, 31));
             if (more && t <= j) sL[(j + 1) * 33 + t] = tot * to_d((VT)(1.0 / hn));
@@ -489,7 +509,7 @@ k_persist(PArgs<VT, MT> a)
             }
         }
         if (lane == 0) l.w[t >> 6][0] = 0.0;
-        if (hop(h, 1, false, false, &l, &tot) != HOP_OK) return;
+        if (hop(h, 1, false, &l, &tot) != HOP_OK) return;
         // r = b - A x in FP64, the next cycle's vector
         double res[KR_RPT], xo[KR_RPT];
         const int rb = opaque(base);
@@ -503,7 +523,7 @@ k_persist(PArgs<VT, MT> a)
             if (rr < n) st_agent(W + rr, w[r]);
         }
         put_norm(res, 0, &l);
-        if (hop(h, 1, false, false, &l, &tot) != HOP_OK) return;
+        if (hop(h, 1, false, &l, &tot) != HOP_OK) return;
         const double now = sqrt(readlane_d(tot, 0));
         const bool stalled = a.stall && iters > iters0 && now > 0.99 * beta;
         beta = now;
