@@ -20,14 +20,15 @@
 //
 // Up to 262,144 rows and m <= 32 a restart cycle is one persistent launch
 // (persist.hip).  Here are the driver and the form with a launch per pass, for
-// larger matrices and restarts.  Its kernels per Arnoldi step: the SpMV with the first
-// pass's dots, the update with the dots of the next pass or of the next
+// larger matrices and restarts.  Its kernels per Arnoldi step: the SpMV with
+// the first pass's dots, the update with the dots of the next pass or of the next
 // basis vector and the norm (twice for CGS2), and after each of them one
 // workgroup that adds the block partials and does the step's small dense
 // work.  Every pass reads the basis once: the update keeps a row's basis
-// entries in registers for the dots of the updated row.  Level 8 (641
+// entries in registers for the dots of the updated row.  Level 8 (257
 // workgroups): 1217 steps in 63 ms, against 125 ms with a pass per basis
-// vector.  A restart cycle is captured once in a hipGraph and replayed;
+// vector; 52 us a step, of which reading the basis and the matrix takes 51
+// at a copy's rate.  A restart cycle is captured once in a hipGraph and replayed;
 // kernels of a finished cycle return at once.
 //
 // Reductions are deterministic: every block writes one partial per dot, and
@@ -318,7 +319,8 @@ k_long(int n, int R, int width, const int* __restrict__ col, const MT* __restric
 // Adds the block partials of a pass and does the step's small dense work, in
 // one workgroup: 32 running sums per value (block g to sum g mod 32), added
 // in the persistent form's order.  The loads of a value's sum are the
-// kernel's time: 20 per thread at level 8's 641 blocks, eight in flight.
+// kernel's time: 8 per thread at level 8's 257 blocks, all in flight, 4.8 us
+// (641 blocks, 20 per thread: 6.9 us).
 enum { RED_BNORM, RED_START, RED_FIRST, RED_AGAIN, RED_NORM };
 __global__ void __launch_bounds__(GM_RED)
 k_reduce(int what, int mgs, int j, int nv, int norm, int S, const double* __restrict__ part, int G,
