@@ -86,6 +86,43 @@ struct phg_mg_s {
 
 namespace {
 
+// C consecutive columns of a row
+template <typename T, int C>
+struct alignas(C * sizeof(T)) MgVec {
+    T a[C];
+};
+// A thread's row and first column of an array with 2^lk C columns.
+template <int C>
+struct MgAt {
+    size_t row;
+    int lk, q;
+    __device__ __forceinline__ explicit MgAt(int lk_) : lk(lk_)
+    {
+        const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+        row = e >> lk;
+        q = ((int)e & ((1 << lk) - 1)) * C;
+    }
+    __device__ __forceinline__ size_t at(int j) const { return ((size_t)j << lk) * C + q; }
+    template <typename T>
+    __device__ __forceinline__ MgVec<T, C> get(const T* x, int j) const
+    {
+        return *(const MgVec<T, C>*)(x + at(j));
+    }
+    template <typename T>
+    __device__ __forceinline__ void put(T* x, int j, MgVec<T, C> v) const
+    {
+        *(MgVec<T, C>*)(x + at(j)) = v;
+    }
+};
+
+// x_j with the coarse correction added
+template <typename T>
+__device__ __forceinline__ T mg_corrected(T xj, int a, int c, T xa, T xc)
+{
+    const T va = a >= 0 ? xa : T(0), vc = c >= 0 ? xc : T(0);
+    return xj + (c == -2 ? va : T(0.5) * (va + vc));
+}
+
 // An ELL row's columns and values, loaded without a branch (past the width
 // the last slot again), and its product with x in slot order.
 template <typename T, typename MT>
@@ -102,114 +139,144 @@ struct MgRow {
             v[k] = (T)val[o];
         }
     }
-    // x(k): the entry that slot k multiplies
-    template <typename F>
-    __device__ __forceinline__ T dot(int width, F x) const
+    // x(k): the entries that slot k multiplies
+    template <int C, typename F>
+    __device__ __forceinline__ MgVec<T, C> dot(int width, F x) const
     {
-        T xv[ELL_MAXW];
+        MgVec<T, C> xv[ELL_MAXW], s{};
 #pragma unroll
         for (int k = 0; k < ELL_MAXW; ++k) xv[k] = x(c[k]);
-        T s = T(0);
 #pragma unroll
-        for (int k = 0; k < ELL_MAXW; ++k) {
-            const T t = s + v[k] * xv[k];
-            s = k < width ? t : s;
-        }
+        for (int k = 0; k < ELL_MAXW; ++k)
+#pragma unroll
+            for (int u = 0; u < C; ++u) {
+                const T t = s.a[u] + v[k] * xv[k].a[u];
+                s.a[u] = k < width ? t : s.a[u];
+            }
         return s;
     }
 };
 
 // The V-cycle kernels in the vector type T (double, or float for the
-// mixed-precision form) over matrix values MT.
-template <typename T, typename MT>
-__global__ void mg_jacobi(int n, int KP, int width, const int* __restrict__ col,
+// mixed-precision form) over matrix values MT.  A thread takes C consecutive
+// columns of a row (mg_apply_c), 16 bytes where a row has that many: with one
+// column a wavefront loads a row's 14 matrix words for 64 products each, and
+// the loads and their addresses bound it.  KP, the columns of an array, is a
+// power of two; lk = log2(KP / C).
+template <typename T, typename MT, int C>
+__global__ void mg_jacobi(int n, int lk, int width, const int* __restrict__ col,
                           const MT* __restrict__ val, const T* __restrict__ dinv,
                           const T* __restrict__ xin, const T* __restrict__ b, T* __restrict__ xout,
                           T w)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)n * KP) return;
-    const int row = (int)(e / KP), q = (int)(e % KP);
+    const MgAt<C> e(lk);
+    if (e.row >= (size_t)n) return;
+    const int row = (int)e.row;
     MgRow<T, MT> r;
     r.load(n, width, row, col, val);
-    const T s = r.dot(width, [&](int j) { return xin[(size_t)j * KP + q]; });
-    xout[e] = xin[e] + w * dinv[row] * (b[e] - s);
+    const MgVec<T, C> s = r.template dot<C>(width, [&](int j) { return e.get(xin, j); });
+    MgVec<T, C> x = e.get(xin, row);
+    const MgVec<T, C> be = e.get(b, row);
+    const T d = w * dinv[row];
+#pragma unroll
+    for (int u = 0; u < C; ++u) x.a[u] = x.a[u] + d * (be.a[u] - s.a[u]);
+    e.put(xout, row, x);
 }
 
-template <typename T, typename MT>
-__global__ void mg_residual(int n, int KP, int width, const int* __restrict__ col,
+template <typename T, typename MT, int C>
+__global__ void mg_residual(int n, int lk, int width, const int* __restrict__ col,
                             const MT* __restrict__ val, const T* __restrict__ x,
                             const T* __restrict__ b, T* __restrict__ r)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)n * KP) return;
-    const int row = (int)(e / KP), q = (int)(e % KP);
-    MgRow<T, MT> a;
-    a.load(n, width, row, col, val);
-    r[e] = b[e] - a.dot(width, [&](int j) { return x[(size_t)j * KP + q]; });
+    const MgAt<C> e(lk);
+    if (e.row >= (size_t)n) return;
+    const int row = (int)e.row;
+    MgRow<T, MT> m;
+    m.load(n, width, row, col, val);
+    const MgVec<T, C> s = m.template dot<C>(width, [&](int j) { return e.get(x, j); });
+    MgVec<T, C> be = e.get(b, row);
+#pragma unroll
+    for (int u = 0; u < C; ++u) be.a[u] = be.a[u] - s.a[u];
+    e.put(r, row, be);
 }
 
-template <typename T>
-__global__ void mg_restrict(int nc, int KP, const int* __restrict__ rrp,
+template <typename T, int C>
+__global__ void mg_restrict(int nc, int lk, const int* __restrict__ rrp,
                             const int* __restrict__ ridx, const T* __restrict__ rw,
                             const T* __restrict__ rf, T* __restrict__ bc)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)nc * KP) return;
-    const int j = (int)(e / KP), q = (int)(e % KP);
-    T s = T(0);
-    for (int t = rrp[j]; t < rrp[j + 1]; ++t) s += rw[t] * rf[(size_t)ridx[t] * KP + q];
-    bc[e] = s;
+    const MgAt<C> e(lk);
+    if (e.row >= (size_t)nc) return;
+    const int j = (int)e.row;
+    MgVec<T, C> s{};
+    for (int t = rrp[j]; t < rrp[j + 1]; ++t) {
+        const MgVec<T, C> v = e.get(rf, ridx[t]);
+#pragma unroll
+        for (int u = 0; u < C; ++u) s.a[u] += rw[t] * v.a[u];
+    }
+    e.put(bc, j, s);
 }
 
-template <typename T>
-__global__ void mg_prolong_add(int nf, int KP, const int* __restrict__ p0,
+template <typename T, int C>
+__global__ void mg_prolong_add(int nf, int lk, const int* __restrict__ p0,
                                const int* __restrict__ p1, const T* __restrict__ xc,
                                T* __restrict__ xf)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)nf * KP) return;
-    const int i = (int)(e / KP), q = (int)(e % KP);
+    const MgAt<C> e(lk);
+    if (e.row >= (size_t)nf) return;
+    const int i = (int)e.row;
     const int a = p0[i], c = p1[i];
-    T v;
-    if (c == -2) v = a >= 0 ? xc[(size_t)a * KP + q] : T(0);  // the vertex itself
-    else v = T(0.5) * ((a >= 0 ? xc[(size_t)a * KP + q] : T(0)) + (c >= 0 ? xc[(size_t)c * KP + q] : T(0)));
-    xf[e] += v;
+    const MgVec<T, C> va = e.get(xc, max(a, 0)), vc = e.get(xc, max(c, 0));
+    MgVec<T, C> x = e.get(xf, i);
+#pragma unroll
+    for (int u = 0; u < C; ++u) x.a[u] = mg_corrected(x.a[u], a, c, va.a[u], vc.a[u]);
+    e.put(xf, i, x);
 }
 
 // Both Jacobi sweeps from x = 0 in one launch: the first one's value of a
 // neighbour is w d b, formed where it is gathered (the same operations as
-// two launches of mg_jacobi: the same bits).
-template <typename T, typename MT>
-__global__ void mg_jacobi_zero2(int n, int KP, int width, const int* __restrict__ col,
+// two launches of mg_jacobi: the same bits).  Bound by its launch: one
+// column FP64, levels 4 to 7 on average, 3.8 us instead of two of 3.3.
+template <typename T, typename MT, int C>
+__global__ void mg_jacobi_zero2(int n, int lk, int width, const int* __restrict__ col,
                                 const MT* __restrict__ val, const T* __restrict__ dinv,
                                 const T* __restrict__ b, T* __restrict__ xout, T w)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)n * KP) return;
-    const int row = (int)(e / KP), q = (int)(e % KP);
+    const MgAt<C> e(lk);
+    if (e.row >= (size_t)n) return;
+    const int row = (int)e.row;
     MgRow<T, MT> r;
     r.load(n, width, row, col, val);
-    const T d = w * dinv[row], be = b[e];
-    const T s = r.dot(width, [&](int j) { return w * dinv[j] * b[(size_t)j * KP + q]; });
-    xout[e] = d * be + d * (be - s);
+    const T d = w * dinv[row];
+    MgVec<T, C> be = e.get(b, row);
+    const MgVec<T, C> s = r.template dot<C>(width, [&](int j) {
+        MgVec<T, C> x = e.get(b, j);
+        const T dj = w * dinv[j];
+#pragma unroll
+        for (int u = 0; u < C; ++u) x.a[u] = dj * x.a[u];
+        return x;
+    });
+#pragma unroll
+    for (int u = 0; u < C; ++u) be.a[u] = d * be.a[u] + d * (be.a[u] - s.a[u]);
+    e.put(xout, row, be);
 }
 
 // The restriction of the residual, for up to MG_FUSE columns: eight lanes per
 // coarse row and column take the residuals of its (at most eight) fine rows,
 // which are then added in order.  A fine row's residual is formed in up to
 // two places (1.75 times the work), which costs less than the launch and
-// the pass over memory it saves: level 7, one column, 8.0 us as two launches.
+// the pass over memory it saves: one column FP64, levels 4 to 7 on average,
+// 5.7 us instead of 2.9 and 4.7 in two launches.
 template <typename T, typename MT>
-__global__ void mg_residual_restrict(int nc, int nf, int KP, int width, const int* __restrict__ col,
+__global__ void mg_residual_restrict(int nc, int nf, int lk, int width, const int* __restrict__ col,
                                      const MT* __restrict__ val, const T* __restrict__ x,
                                      const T* __restrict__ b, const int* __restrict__ rrp,
                                      const int* __restrict__ ridx, const T* __restrict__ rw,
                                      T* __restrict__ bc)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int q = (int)(e % KP), t = (int)(e / KP) & 7;
-    const size_t j = e / KP / 8;
+    const MgAt<1> e(lk);
+    const int KP = 1 << lk, t = (int)e.row & 7;
+    const size_t j = e.row >> 3;
     int cnt = 0;
     T v = T(0);
     if (j < (size_t)nc) {
@@ -219,8 +286,8 @@ __global__ void mg_residual_restrict(int nc, int nf, int KP, int width, const in
             const int i = ridx[lo + t];
             MgRow<T, MT> r;
             r.load(nf, width, i, col, val);
-            const T s = r.dot(width, [&](int k) { return x[(size_t)k * KP + q]; });
-            v = rw[lo + t] * (b[(size_t)i * KP + q] - s);
+            const T s = r.template dot<1>(width, [&](int k) { return e.get(x, k); }).a[0];
+            v = rw[lo + t] * (e.get(b, i).a[0] - s);
         }
     }
     const int lane = threadIdx.x & 63, first = lane - t * KP;
@@ -230,39 +297,32 @@ __global__ void mg_residual_restrict(int nc, int nf, int KP, int width, const in
         const T u = s + __shfl(v, first + k * KP, 64);
         s = k < cnt ? u : s;
     }
-    if (t == 0 && j < (size_t)nc) bc[j * KP + q] = s;
-}
-
-// x_j with the coarse correction added (as mg_prolong_add adds it)
-template <typename T>
-__device__ __forceinline__ T mg_corrected(T xj, int a, int c, T xa, T xc)
-{
-    const T va = a >= 0 ? xa : T(0), vc = c >= 0 ? xc : T(0);
-    return xj + (c == -2 ? va : T(0.5) * (va + vc));
+    if (t == 0 && j < (size_t)nc) bc[e.at((int)j)] = s;
 }
 
 // The coarse correction and the Jacobi sweep after it in one launch, for up
 // to MG_FUSE columns: a neighbour's corrected value is formed where it is
-// gathered.
+// gathered.  One column FP64, levels 4 to 7 on average, 5.9 us instead of 3.1
+// and 3.3 in two launches and the gap between them.
 template <typename T, typename MT>
-__global__ void mg_prolong_jacobi(int n, int KP, int width, const int* __restrict__ col,
+__global__ void mg_prolong_jacobi(int n, int lk, int width, const int* __restrict__ col,
                                   const MT* __restrict__ val, const T* __restrict__ dinv,
                                   const int* __restrict__ p0, const int* __restrict__ p1,
                                   const T* __restrict__ xc, const T* __restrict__ x,
                                   const T* __restrict__ b, T* __restrict__ xout, T w)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)n * KP) return;
-    const int row = (int)(e / KP), q = (int)(e % KP);
+    const MgAt<1> e(lk);
+    if (e.row >= (size_t)n) return;
+    const int row = (int)e.row;
     MgRow<T, MT> r;
     r.load(n, width, row, col, val);
     const auto at = [&](int j) {
         const int a = p0[j], c = p1[j];
-        return mg_corrected(x[(size_t)j * KP + q], a, c, xc[(size_t)max(a, 0) * KP + q],
-                            xc[(size_t)max(c, 0) * KP + q]);
+        return MgVec<T, 1>{{mg_corrected(e.get(x, j).a[0], a, c, e.get(xc, max(a, 0)).a[0],
+                                         e.get(xc, max(c, 0)).a[0])}};
     };
-    const T s = r.dot(width, at);
-    xout[e] = at(row) + w * dinv[row] * (b[e] - s);
+    const T s = r.template dot<1>(width, at).a[0];
+    xout[e.at(row)] = at(row).a[0] + w * dinv[row] * (e.get(b, row).a[0] - s);
 }
 
 // ---- the coarse levels in one launch ------------------------------------
@@ -311,7 +371,7 @@ struct MgcRows {
     }
     __device__ __forceinline__ T dot(const T* x) const
     {
-        return row.dot(width, [&](int j) { return x[j]; });
+        return row.template dot<1>(width, [&](int j) { return MgVec<T, 1>{{x[j]}}; }).a[0];
     }
     // two sweeps from zero, the residual (left in y) and its restriction to bc
     __device__ __forceinline__ void down(T* x, T* y, const T* b, T* bc) const
@@ -348,7 +408,8 @@ struct MgcRows {
 };
 
 // x = V-cycle(b) of level 3 over the dense inverse of level 2 (nc rows);
-// column blockIdx.x of n x KP arrays.
+// column blockIdx.x of n x KP arrays.  FP64 19.9 us, FP32 11, instead of
+// eight launches (level 3's seven of 3 us and the dense product's 6.2).
 template <typename T, typename MT>
 __global__ void __launch_bounds__(MGC_BS)
 mg_coarse(MgcLevel<T, MT> l3, int nc, const T* __restrict__ cinv, int KP,
@@ -609,7 +670,7 @@ MgcLevel<T, typename MgT<T>::MT> mgc_level(MgLevel& l)
 // and below are one launch; above, a level takes four launches for up to
 // MG_FUSE columns and six for more, where the passes are bound by memory and
 // the recomputation of the fused ones would show.
-template <typename T>
+template <typename T, int C>
 void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
 {
     using B = MgT<T>;
@@ -622,26 +683,28 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
         return;
     }
     const int kc = nlev - 2;  // level 3: with level 2 in one launch
-    const bool fuse = KP <= MG_FUSE && (KP & (KP - 1)) == 0;
+    const bool fuse = KP <= MG_FUSE;
+    const int l1 = __builtin_ctz((unsigned)KP), lk = l1 - __builtin_ctz((unsigned)C);
     // descend: level 0 takes b = v (read directly), result to z
     const T* bk = v;
     for (int k = 0; k < kc; ++k) {
         MgLevel& l = *M->lv[k];
         MgLevel& c = *M->lv[k + 1];
         const auto& E = B::E(l);
-        const size_t w = (size_t)l.n * KP;
+        const size_t w = (size_t)l.n * KP / C;
         T* xa = (k == 0) ? z : B::x0(l);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi_zero2<T, MT>), grid_for(w), dim3(256), 0, s,
-                           l.n, KP, E.width, E.col.p, E.val.p, B::dinv(l), bk, xa, om);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi_zero2<T, MT, C>), grid_for(w), dim3(256), 0, s,
+                           l.n, lk, E.width, E.col.p, E.val.p, B::dinv(l), bk, xa, om);
         if (fuse) {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual_restrict<T, MT>),
-                               grid_for((size_t)c.n * KP * 8), dim3(256), 0, s, c.n, l.n, KP, E.width,
+                               grid_for((size_t)c.n * KP * 8), dim3(256), 0, s, c.n, l.n, l1, E.width,
                                E.col.p, E.val.p, xa, bk, l.rrp.p, l.ridx.p, B::rw(l), B::b(c));
         } else {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual<T, MT>), grid_for(w), dim3(256), 0, s,
-                               l.n, KP, E.width, E.col.p, E.val.p, xa, bk, B::r(l));
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_restrict<T>), grid_for((size_t)c.n * KP), dim3(256),
-                               0, s, c.n, KP, l.rrp.p, l.ridx.p, B::rw(l), B::r(l), B::b(c));
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual<T, MT, C>), grid_for(w), dim3(256), 0, s,
+                               l.n, lk, E.width, E.col.p, E.val.p, xa, bk, B::r(l));
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_restrict<T, C>), grid_for((size_t)c.n * KP / C),
+                               dim3(256), 0, s, c.n, lk, l.rrp.p, l.ridx.p, B::rw(l), B::r(l),
+                               B::b(c));
         }
         bk = B::b(c);
     }
@@ -653,32 +716,45 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
         MgLevel& l = *M->lv[k];
         MgLevel& c = *M->lv[k + 1];
         const auto& E = B::E(l);
-        const size_t w = (size_t)l.n * KP;
+        const size_t w = (size_t)l.n * KP / C;
         const T* bl = (k == 0) ? v : B::b(l);
         T* xa = (k == 0) ? z : B::x0(l);
         if (fuse) {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_jacobi<T, MT>), grid_for(w), dim3(256), 0,
-                               s, l.n, KP, E.width, E.col.p, E.val.p, B::dinv(l), l.p0.p, l.p1.p,
+                               s, l.n, lk, E.width, E.col.p, E.val.p, B::dinv(l), l.p0.p, l.p1.p,
                                B::x0(c), xa, bl, B::x1(l), om);
         } else {
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_add<T>), grid_for(w), dim3(256), 0, s, l.n,
-                               KP, l.p0.p, l.p1.p, B::x0(c), xa);
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
-                               KP, E.width, E.col.p, E.val.p, B::dinv(l), xa, bl, B::x1(l), om);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_add<T, C>), grid_for(w), dim3(256), 0, s,
+                               l.n, lk, l.p0.p, l.p1.p, B::x0(c), xa);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT, C>), grid_for(w), dim3(256), 0, s, l.n,
+                               lk, E.width, E.col.p, E.val.p, B::dinv(l), xa, bl, B::x1(l), om);
         }
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT>), grid_for(w), dim3(256), 0, s, l.n,
-                           KP, E.width, E.col.p, E.val.p, B::dinv(l), B::x1(l), bl, xa, om);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi<T, MT, C>), grid_for(w), dim3(256), 0, s, l.n,
+                           lk, E.width, E.col.p, E.val.p, B::dinv(l), B::x1(l), bl, xa, om);
     }
+}
+
+// Columns per thread: 16 bytes of a row where the fused passes (which are
+// launch bound) don't run: a solve of 64 FP32 columns at level 7 9.76 ms with
+// one column per thread, 7.70 ms with four.  Every array of a level starts on
+// 16 bytes and its rows of at least 16 columns are a multiple of them.
+template <typename T>
+void mg_apply_c(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
+{
+    constexpr int C = 16 / sizeof(T);
+    const bool wide = KP > MG_FUSE && ((size_t)v | (size_t)z) % 16 == 0;
+    if (wide) mg_apply_t<T, C>(M, KP, v, z, s);
+    else mg_apply_t<T, 1>(M, KP, v, z, s);
 }
 
 void mg_apply(phg_mg_s* M, int KP, const double* v, double* z, hipStream_t s)
 {
-    mg_apply_t<double>(M, KP, v, z, s);
+    mg_apply_c<double>(M, KP, v, z, s);
 }
 
 void mg_apply_f32(phg_mg_s* M, int KP, const float* v, float* z, hipStream_t s)
 {
-    mg_apply_t<float>(M, KP, v, z, s);
+    mg_apply_c<float>(M, KP, v, z, s);
 }
 
 // FP32 copies of every level's operator values, inverse diagonal and
