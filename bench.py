@@ -668,7 +668,7 @@ def main():
         "n=%d nnz=%d" % (t_asm * 1e3, t_asm2 * 1e3, n, nnz))
 
     # ---- timed region: plain FP64 GMRES(30), MGS (the reference form), each
-    #      restart cycle one cooperative kernel (HIP events around each) ----
+    #      restart cycle one persistent launch (HIP events around each) ----
     wall, lat, p50, p99, infos = time_solves(A, b, x, args.steps, args.warmup, stream,
                                              restart=30, rtol=1e-10, ortho=P.MGS)
     ok = all(i["converged"] and i["rel_residual"] <= 1e-10 for i in infos)
