@@ -139,7 +139,23 @@ struct MgRow {
             v[k] = (T)val[o];
         }
     }
-    // x(k): the entries that slot k multiplies
+    // x(k): the entry that slot k multiplies
+    template <typename F>
+    __device__ __forceinline__ T dot1(int width, F x) const
+    {
+        T xv[ELL_MAXW];
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) xv[k] = x(c[k]);
+        T s = T(0);
+#pragma unroll
+        for (int k = 0; k < ELL_MAXW; ++k) {
+            const T t = s + v[k] * xv[k];
+            s = k < width ? t : s;
+        }
+        return s;
+    }
+    // the same for C columns (in place of dot1 too it spilled four more
+    // registers of mg_coarse: a V-cycle of one column took 6 us more)
     template <int C, typename F>
     __device__ __forceinline__ MgVec<T, C> dot(int width, F x) const
     {
@@ -286,8 +302,8 @@ __global__ void mg_residual_restrict(int nc, int nf, int lk, int width, const in
             const int i = ridx[lo + t];
             MgRow<T, MT> r;
             r.load(nf, width, i, col, val);
-            const T s = r.template dot<1>(width, [&](int k) { return e.get(x, k); }).a[0];
-            v = rw[lo + t] * (e.get(b, i).a[0] - s);
+            const T s = r.dot1(width, [&](int k) { return x[e.at(k)]; });
+            v = rw[lo + t] * (b[e.at(i)] - s);
         }
     }
     const int lane = threadIdx.x & 63, first = lane - t * KP;
@@ -318,11 +334,10 @@ __global__ void mg_prolong_jacobi(int n, int lk, int width, const int* __restric
     r.load(n, width, row, col, val);
     const auto at = [&](int j) {
         const int a = p0[j], c = p1[j];
-        return MgVec<T, 1>{{mg_corrected(e.get(x, j).a[0], a, c, e.get(xc, max(a, 0)).a[0],
-                                         e.get(xc, max(c, 0)).a[0])}};
+        return mg_corrected(x[e.at(j)], a, c, xc[e.at(max(a, 0))], xc[e.at(max(c, 0))]);
     };
-    const T s = r.template dot<1>(width, at).a[0];
-    xout[e.at(row)] = at(row).a[0] + w * dinv[row] * (e.get(b, row).a[0] - s);
+    const T s = r.dot1(width, at);
+    xout[e.at(row)] = at(row) + w * dinv[row] * (b[e.at(row)] - s);
 }
 
 // ---- the coarse levels in one launch ------------------------------------
@@ -371,7 +386,7 @@ struct MgcRows {
     }
     __device__ __forceinline__ T dot(const T* x) const
     {
-        return row.template dot<1>(width, [&](int j) { return MgVec<T, 1>{{x[j]}}; }).a[0];
+        return row.dot1(width, [&](int j) { return x[j]; });
     }
     // two sweeps from zero, the residual (left in y) and its restriction to bc
     __device__ __forceinline__ void down(T* x, T* y, const T* b, T* bc) const
