@@ -37,7 +37,7 @@ constexpr int PERSIST_NOT_HERE = 2;  // the shape does not run here: nothing was
 struct PersistWork {
     DevBuf<char> W;              // the vector that the products gather, per column
     DevBuf<PState> st;           // per column
-    DevBuf<int> abort_dev;
+    DevBuf<int> abort_dev;       // per column
     PState* host = nullptr;      // pinned: host_k states, then the abort flag
     int host_k = 0;
     XchRows xch;                 // two rings of ring_slots words

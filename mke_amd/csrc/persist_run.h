@@ -70,19 +70,27 @@ constexpr int PS_M = 32;      // largest restart
 // is needed.  Every wait is bounded: after `spin` polls a workgroup raises
 // the abort flag and leaves, and the others leave at their next look at it.
 //
-// The first exchange of a launch shows that its workgroups are resident
+// The first exchange of a launch shows that a column's workgroups are resident
 // together: each stays until it has seen the others' slots.  If something
 // else holds the CUs (another process's launch, half of it waiting for this
 // one's other half), that exchange ends after start_spin polls, and the host
-// launches again: x and the state of the columns are written only after
-// later exchanges, so nothing is lost.  Within a process launches take turns
-// (persist_mutex).  A cooperative launch would give the same guarantee but is
-// refused to every process of a GPU except the first that asks.
+// launches the column again.  A workgroup that gives up has stored its slot,
+// and its CU may go to the one that was missing, so others may still pass the
+// first exchange; none passes the second, which the one that gave up never
+// stores.  So nothing that a repeated launch reads (W, the state, x when it is
+// a start vector) is written before the second exchange: a launch that
+// continues a solve begins with an exchange of no values, whose 1.7 to 2.7 us
+// are 1 to 2 % of a cycle.  The abort flag is the column's own: the other
+// columns of the launch, which may be far along, go on.  Within a process
+// launches take turns (persist_mutex).  A cooperative launch would give the
+// same guarantee but is refused to every process of a GPU except the first
+// that asks.
 struct Hop {
     xch_t* ring;
     int G, slot, e;  // G: slots of a row (padded workgroup count)
     long spin, start_spin;
-    int *abort_dev, *abort_host;
+    int* abort_dev;   // the column's
+    int* abort_host;  // the solve's
 };
 
 inline int hop_slots(int G)
@@ -203,7 +211,7 @@ struct PArgs {
     size_t ldw;
     xch_t *ring, *other;   // XCH_RING rows of Gp slots per column
     PState *st, *host;
-    int *abort_dev, *abort_host;
+    int *abort_dev, *abort_host;  // a word per column; one for the host
     long spin, start_spin;
     double rtol, inner_rtol;
     int max_iters, max_cycles, first, use_x0, stall;
@@ -333,7 +341,7 @@ k_persist(PArgs<VT, MT> a)
     constexpr bool LATE = BS == 256 || sizeof(VT) == 4;
     const int n = a.n, ld = a.ld, m = a.m, slot = slot_of(bid, a.Gp);
     Hop h{a.ring + (size_t)q * XCH_RING * a.Gp * XCH_V, a.Gp, slot, 0, a.spin, a.start_spin,
-          a.abort_dev, a.abort_host};
+          a.abort_dev + q, a.abort_host};
     if (t < XCH_RING * XCH_V)
         st_agent(a.other + (size_t)q * XCH_RING * a.Gp * XCH_V +
                      ((size_t)(t >> 5) * a.Gp + slot) * XCH_V + (t & 31), XCH_EMPTY);
@@ -370,14 +378,6 @@ k_persist(PArgs<VT, MT> a)
         }
         put_norm(b, 0, &l);
         put_norm(r0, 1, &l);
-        if (hop(h, 2, false, &l, &tot) != HOP_OK) return;
-        bnorm = sqrt(readlane_d(tot, 0));
-        if (!(bnorm > 0.0)) bnorm = 1.0;
-        beta = sqrt(readlane_d(tot, 1));
-        rel = beta / bnorm;
-        if (rel <= a.rtol || beta == 0.0) converged = 1;
-        else active = iters < a.max_iters && (!a.stall || isfinite(beta));
-        if (active) ++cycles;
     } else {
         const PState s = a.st[q];
         bnorm = s.bnorm, beta = s.beta, rel = s.rel;
@@ -387,6 +387,17 @@ k_persist(PArgs<VT, MT> a)
             const int rr = base + r * KR_STRIDE;
             w[r] = rr < n ? W[rr] : VT(0);
         }
+        if (lane < 2) l.w[t >> 6][lane] = 0.0;
+    }
+    if ((a.first || active) && hop(h, 2, false, &l, &tot) != HOP_OK) return;
+    if (a.first) {
+        bnorm = sqrt(readlane_d(tot, 0));
+        if (!(bnorm > 0.0)) bnorm = 1.0;
+        beta = sqrt(readlane_d(tot, 1));
+        rel = beta / bnorm;
+        if (rel <= a.rtol || beta == 0.0) converged = 1;
+        else active = iters < a.max_iters && (!a.stall || isfinite(beta));
+        if (active) ++cycles;
     }
 
     // the thread's matrix rows (past a row's width its last slot with the
@@ -553,12 +564,13 @@ __device__ inline bool slot_used(int slot, int G, int Gp)
     return p * PAIR + half < G;
 }
 
-// Clears both rings (slots past the last workgroup: 0) and the abort flag.
-__global__ void k_ring_reset(xch_t* ring, size_t count, int G, int Gp, int* abort_dev)
+// Clears both rings (slots past the last workgroup: 0) and the nab columns'
+// abort flags (nab at most a ring's slots).
+__global__ void k_ring_reset(xch_t* ring, size_t count, int G, int Gp, int* abort_dev, int nab)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < count) ring[i] = slot_used((int)(i / XCH_V % Gp), G, Gp) ? XCH_EMPTY : 0;
-    if (i == 0) *abort_dev = 0;
+    if (i < (size_t)nab) abort_dev[i] = 0;
 }
 
 // Workgroups of the kernel that the device holds at once, per template
@@ -589,7 +601,7 @@ int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int
     if (w->ring_k != K || w->ring_g != G) {
         // another shape than the last launch's, or after a give-up
         hipLaunchKernelGGL(k_ring_reset, dim3((unsigned)((2 * slots + 255) / 256)), dim3(256), 0, s,
-                           w->xch.p(), 2 * slots, G, Gp, w->abort_dev.p);
+                           w->xch.p(), 2 * slots, G, Gp, w->abort_dev.p, w->host_k);
         PHG_HIP(hipGetLastError());
         w->ring_k = K;
         w->ring_g = G;
@@ -603,7 +615,7 @@ int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int
     a.other = w->xch.p() + (w->parity ? 0 : slots);
     w->parity ^= 1;
     a.st = w->st.p + q0, a.host = w->host + q0;
-    a.abort_dev = w->abort_dev.p, a.abort_host = (int*)(w->host + w->host_k);
+    a.abort_dev = w->abort_dev.p + q0, a.abort_host = (int*)(w->host + w->host_k);
     a.spin = XCH_SPIN;
     if (const char* e = getenv("PHG_XCH_SPIN")) a.spin = std::max(1L, atol(e));
     a.start_spin = std::min(a.spin, XCH_START);
@@ -637,11 +649,12 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
         w->host = nullptr;
         w->host_k = 0;
         PHG_HIP(w->st.alloc(K));
+        PHG_HIP(w->abort_dev.alloc(K));
+        w->ring_k = 0;  // they are cleared with the rings
         // K states, then the abort word
         PHG_HIP(hipHostMalloc((void**)&w->host, sizeof(PState) * (K + 1), hipHostMallocDefault));
         w->host_k = K;
     }
-    if (!w->abort_dev.p) PHG_HIP(w->abort_dev.alloc(1));
     if (w->ring_slots < slots) {
         w->ring_slots = 0;
         PHG_HIP(w->xch.alloc(2 * slots));
