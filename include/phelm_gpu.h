@@ -206,8 +206,10 @@ typedef struct {
                         partials through device memory (restart <= 32, up to
                         262,144 rows); 0 launches kernels for each pass
                         (captured in a hipGraph).  Both give the same bits;
-                        1 falls back to 0 for other shapes and where the
-                        device cannot keep every workgroup resident.
+                        1 falls back to 0 for other shapes, where the
+                        device cannot keep every workgroup resident, and
+                        from the cycle on for which it does not (16
+                        launches that do not start: other work holds it).
                         phg_gmres_batch: 1 runs the columns that way where
                         it is the faster form for (rows, nrhs, restart,
                         precision, ortho), 0 never; the two add their dot

@@ -369,11 +369,6 @@ k_reduce(int what, int mgs, int j, int nv, int norm, int S, const double* __rest
         if (lane == 0) {
             const double bn = sqrt(last);
             st->bnorm = bn > 0.0 ? bn : 1.0;
-            st->iters = 0;
-            st->cycles = 0;
-            st->converged = 0;
-            st->active = 0;
-            st->k = 0;
         }
     } else if (what == RED_START) {
         if (lane == 0) {
@@ -598,9 +593,10 @@ void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, bool 
     hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, mgs, 0, 0, 1, S, part, G, st);
 }
 
+// iters, cycles: what a solve that is continued from x has done.
 template <typename VT, typename MT>
 int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* b, double* x,
-                 const phg_gmres_opts& o, phg_gmres_info* info, hipStream_t s)
+                 const phg_gmres_opts& o, int iters, int cycles, phg_gmres_info* info, hipStream_t s)
 {
     int rc = prepare_passes(w);
     if (rc) return rc;
@@ -618,6 +614,8 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
     init.rtol = o.rtol;
     init.inner_rtol = (o.precision == PHG_F64) ? 0.0 : o.inner_rtol;
     init.max_iters = o.max_iters;
+    init.iters = iters;
+    init.cycles = cycles;
     init.b = b;
     init.x = x;
     PHG_HIP(hipMemcpyAsync(st, &init, sizeof init, hipMemcpyHostToDevice, s));
@@ -718,13 +716,22 @@ int gmres_solve(phg_matrix_s* A, const double* b, double* x, const phg_gmres_opt
     if (rc) return rc;
 
     rc = PERSIST_NOT_HERE;
+    int iters = 0, cycles = 0;
     if (o.persistent) {
         // one launch per restart cycle
         int launches = 0;
         double ms = 0.0;
         rc = persist_solve(A, &w->persist, 1, b, x, o, false, false, 1, 1, &launches, &ms, s);
+        const PState* st = w->persist.host;
+        if (rc == PERSIST_NO_START) {
+            // the launches per pass need no CUs at the same time; they give
+            // the same bits from here
+            if (st->cycles > 0) o.use_x0 = 1;
+            iters = st->iters, cycles = std::max(0, st->cycles - 1);
+            if (info) info->cycle_launches = launches, info->cycle_ms = ms;
+        }
         if (rc == PHG_OK) {
-            const PState& h = w->persist.host[0];
+            const PState& h = *st;
             if (info) {
                 info->iterations = h.iters;
                 info->restarts = h.cycles;
@@ -736,13 +743,13 @@ int gmres_solve(phg_matrix_s* A, const double* b, double* x, const phg_gmres_opt
             rc = h.converged ? PHG_OK : PHG_ERR_NOCONV;
         }
     }
-    if (rc == PERSIST_NOT_HERE) {
+    if (rc == PERSIST_NOT_HERE || rc == PERSIST_NO_START) {
         if (o.precision == PHG_F64)
-            rc = gmres_passes<double, double>(A, A->ell64, w, b, x, o, info, s);
+            rc = gmres_passes<double, double>(A, A->ell64, w, b, x, o, iters, cycles, info, s);
         else if (o.precision == PHG_F32)
-            rc = gmres_passes<float, float>(A, A->ell32, w, b, x, o, info, s);
+            rc = gmres_passes<float, float>(A, A->ell32, w, b, x, o, iters, cycles, info, s);
         else
-            rc = gmres_passes<float, uint16_t>(A, A->ell16, w, b, x, o, info, s);
+            rc = gmres_passes<float, uint16_t>(A, A->ell16, w, b, x, o, iters, cycles, info, s);
     }
     if (info) info->refinements = o.precision == PHG_F64 ? 0 : info->restarts;
     return rc;

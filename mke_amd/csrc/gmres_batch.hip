@@ -658,8 +658,10 @@ bk_sumsq(int n, int KP, int K, int R, const double* __restrict__ B, double* __re
     put_partials<1>(a, 0, KP, 0, part, G);
 }
 
+// from: the columns of a solve that is continued from X (persist.h), or null.
 __global__ void bk_set_bnorm(int KP, int K, const double* __restrict__ part, int G,
-                             BCol* __restrict__ cols, BIo arrays, BIo* __restrict__ io)
+                             BCol* __restrict__ cols, BIo arrays, BIo* __restrict__ io,
+                             const PState* __restrict__ from)
 {
     if (lblock() == 0 && threadIdx.x == 0) *io = arrays;
     const int q = lblock() * (BB_BS / 64) + ((int)threadIdx.x >> 6);
@@ -669,9 +671,10 @@ __global__ void bk_set_bnorm(int KP, int K, const double* __restrict__ part, int
         BCol* c = cols + q;
         const double bn = sqrt(s);
         c->bnorm = bn > 0.0 ? bn : 1.0;
-        c->iters = 0;
-        c->cycles = 0;
-        c->converged = 0;
+        c->iters = from ? from[q].iters : 0;
+        c->iters0 = c->iters;
+        c->cycles = from ? max(0, from[q].cycles - 1) : 0;  // before the next one
+        c->converged = from && !from[q].active;  // complete: left alone
         c->active = 0;
         c->k = 0;
     }
@@ -718,10 +721,12 @@ __global__ void bk_cycle_start(int KP, int K, const double* __restrict__ part, i
     sum[q] = o;
 }
 
-__global__ void bk_fill0(size_t n, double* __restrict__ x)
+// x = 0, of a continued solve only the columns that have not begun
+__global__ void bk_fill0(size_t n, int K, double* __restrict__ x, const PState* __restrict__ from)
 {
     const size_t i = (size_t)lblock() * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0;
+    if (i >= n) return;
+    if (!from || (from[i % K].active && from[i % K].cycles == 0)) x[i] = 0.0;
 }
 
 // ---------------------------------------------------------------- driver --
@@ -939,7 +944,8 @@ void enqueue_batch_finish(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K
 
 template <typename VT, typename MT>
 int batch_run(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const double* B, double* X,
-              const phg_gmres_opts& o, phg_gmres_info* infos, BatchPrecond* pc, hipStream_t s)
+              const phg_gmres_opts& o, phg_gmres_info* infos, BatchPrecond* pc,
+              const PersistWork* from, hipStream_t s)
 {
     const int n = w->n, KP = w->kp, G = w->G, m = o.restart;
     const size_t bs = (size_t)n * KP;
@@ -952,13 +958,19 @@ int batch_run(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const doub
     const double inner = o.precision == PHG_F64 ? 0.0 : o.inner_rtol;
     (void)bs;
 
+    const PState* state = nullptr;
+    if (from) {
+        state = from->st.p;
+        PHG_HIP(hipMemcpyAsync(from->st.p, from->host, sizeof(PState) * K, hipMemcpyHostToDevice, s));
+    }
     if (!o.use_x0) {
         const size_t tot = (size_t)n * K;
-        hipLaunchKernelGGL(bk_fill0, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, tot, X);
+        hipLaunchKernelGGL(bk_fill0, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, tot, K, X,
+                           state);
     }
     hipLaunchKernelGGL(bk_sumsq, grid, block, 0, s, n, KP, K, w->rpt, B, part, G);
     hipLaunchKernelGGL(bk_set_bnorm, dim3(cb), block, 0, s, KP, K, part, G, cols,
-                       BIo{B, X}, w->io.p);
+                       BIo{B, X}, w->io.p, state);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(bk_residual<VT>), grid, block, 0, s, n, KP, K, w->rpt,
                        A->ell64.width, A->ell64.col.p, A->ell64.val.p, w->io.p, W0, part, G, cols);
     hipLaunchKernelGGL(bk_cycle_start, dim3(cb), block, 0, s, KP, K, part, G, cols, w->sum.p,
@@ -1038,7 +1050,11 @@ int batch_run(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const doub
     }
     bool all = true;
     for (int q = 0; q < K; ++q) {
-        const BSum& h = w->host[q];
+        BSum h = w->host[q];
+        if (from && !from->host[q].active) {
+            const PState& p = from->host[q];
+            h.rel = p.rel, h.converged = p.converged, h.iters = p.iters, h.cycles = p.cycles;
+        }
         all = all && h.converged;
         if (infos) {
             memset(&infos[q], 0, sizeof infos[q]);
@@ -1109,7 +1125,8 @@ int persistent_rounds(int n, int kp, int m, bool f64, bool twice)
 }
 
 // The columns as persistent launches, where that is the faster form;
-// PERSIST_NOT_HERE otherwise.
+// PERSIST_NOT_HERE otherwise, PERSIST_NO_START where the launches go on with
+// what w->host has.
 int batch_persistent(phg_matrix_s* A, int K, const double* B, double* X, const phg_gmres_opts& o,
                      phg_gmres_info* infos, hipStream_t s)
 {
@@ -1205,12 +1222,14 @@ int gmres_batch_solve_pc(phg_matrix_s* A, int K, const double* B, double* X,
     else if (o.precision == PHG_F32) rc = ensure_ell32(A, s);
     else if (o.precision == PHG_BF16) rc = ensure_ell16(A, s);
     if (rc) return rc;
+    const int slot = o.precision == PHG_F64 ? 0 : 1;
+    const PersistWork* from = nullptr;
     if (!pc && o.persistent) {
         rc = batch_persistent(A, K, B, X, o, infos, s);
-        if (rc != PERSIST_NOT_HERE) return rc;
+        if (rc == PERSIST_NO_START) from = A->pbatch[slot];
+        else if (rc != PERSIST_NOT_HERE) return rc;
     }
     BatchWork* w = nullptr;
-    const int slot = o.precision == PHG_F64 ? 0 : 1;
     // the autotuner times the plain form, so a preconditioned solve keeps the
     // untuned default shape: its speed and bits do not depend on which
     // tunings ran earlier in the process
@@ -1220,10 +1239,11 @@ int gmres_batch_solve_pc(phg_matrix_s* A, int K, const double* B, double* X,
     if (rc) return rc;
     // diag: right preconditioning by D^-1: solve (A D^-1) y = b, x = D^-1 y
     if (o.precision == PHG_F64)
-        return batch_run<double, double>(A, diag ? A->ell64d : A->ell64, w, K, B, X, o, infos, pc, s);
+        return batch_run<double, double>(A, diag ? A->ell64d : A->ell64, w, K, B, X, o, infos, pc,
+                                         from, s);
     if (o.precision == PHG_F32)
-        return batch_run<float, float>(A, A->ell32, w, K, B, X, o, infos, pc, s);
-    return batch_run<float, uint16_t>(A, A->ell16, w, K, B, X, o, infos, pc, s);
+        return batch_run<float, float>(A, A->ell32, w, K, B, X, o, infos, pc, from, s);
+    return batch_run<float, uint16_t>(A, A->ell16, w, K, B, X, o, infos, pc, from, s);
 }
 
 int batch_shape_get(int n, int K, int prec)

@@ -33,6 +33,11 @@ struct PState {
 };
 
 constexpr int PERSIST_NOT_HERE = 2;  // the shape does not run here: nothing was done
+// Launches found no CUs for their workgroups: to be continued elsewhere.
+// w->host[q]: a column with active = 1 and cycles = 0 has not begun (x as it
+// was if it is a start vector, else undefined), with cycles > 0 it continues
+// from x with cycle number `cycles`; one with active = 0 is complete.
+constexpr int PERSIST_NO_START = 3;
 
 struct PersistWork {
     DevBuf<char> W;              // the vector that the products gather, per column

@@ -34,11 +34,14 @@ __host__ __device__ inline int slot_of(int bid, int Gp) { return bid / PAIR + bi
 typedef unsigned long long xch_t;
 constexpr xch_t XCH_EMPTY = 0x7FF4DEADBEEF0001ull;  // a signalling-NaN pattern no partial takes
 constexpr long XCH_SPIN = 1L << 22;                  // polls before a wait gives up
-// (PHG_XCH_SPIN overrides it: the failure-path test forces a give-up with
-// a limit of a few polls; every workgroup still exits normally)
-// polls of a launch's first exchange (some 0.1 s), and launches until it succeeds
+// polls of a launch's first exchange (some 0.1 s), and launches until it
+// succeeds or the solve goes on without them: 1.6 s for another process's
+// work to end
 constexpr long XCH_START = 1L << 17;
-constexpr int XCH_TRIES = 64;
+constexpr int XCH_TRIES = 16;
+// (PHG_XCH_SPIN and PHG_XCH_START override the two limits: the tests of the
+// failure paths force a give-up with a few polls; every workgroup still exits
+// normally)
 enum { ABORT_WAIT = 1, ABORT_START = 2 };  // bits of the host's abort word
 constexpr int XCH_RING = 4;   // rows of a column's ring
 constexpr int XCH_V = 32;     // values of a slot
@@ -590,6 +593,12 @@ int capacity()
     return n;
 }
 
+inline long poll_limit(const char* name, long limit)
+{
+    const char* e = getenv(name);
+    return e ? std::max(1L, atol(e)) : limit;
+}
+
 // Columns q0 .. q0 + K - 1 of the ld in B and X.
 template <typename VT, typename MT, int ORTHO>
 int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int ld, const double* B,
@@ -616,9 +625,8 @@ int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int
     w->parity ^= 1;
     a.st = w->st.p + q0, a.host = w->host + q0;
     a.abort_dev = w->abort_dev.p + q0, a.abort_host = (int*)(w->host + w->host_k);
-    a.spin = XCH_SPIN;
-    if (const char* e = getenv("PHG_XCH_SPIN")) a.spin = std::max(1L, atol(e));
-    a.start_spin = std::min(a.spin, XCH_START);
+    a.spin = poll_limit("PHG_XCH_SPIN", XCH_SPIN);
+    a.start_spin = poll_limit("PHG_XCH_START", XCH_START);
     a.rtol = o.rtol;
     a.inner_rtol = o.precision == PHG_F64 ? 0.0 : o.inner_rtol;
     a.max_iters = o.max_iters, a.max_cycles = max_cycles, a.use_x0 = o.use_x0;
@@ -678,7 +686,7 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
     int tries = 0;
     for (int first = 1;; first = 0) {
         for (int q = 0; q < K; ++q)
-            if (first) w->host[q].active = 1;
+            if (first) w->host[q] = PState{0.0, 0.0, 0.0, 0, 0, 0, 1};
         // the columns still running, and one by one those of a launch that
         // did not start
         for (bool again = false;; again = true) {
@@ -707,13 +715,20 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
             }
             if (!*abort_host) break;
             w->ring_k = 0;
-            if ((*abort_host & ABORT_WAIT) || ++tries >= XCH_TRIES) {
+            if (*abort_host & ABORT_WAIT) {
                 set_error("gmres: a workgroup of the persistent solve timed out waiting for the "
                           "others");
                 return PHG_ERR_HIP;
             }
+            if (++tries >= XCH_TRIES) {
+                for (int q = 0; q < K; ++q)
+                    if (w->host[q].active == -1) w->host[q].active = 1;
+                return PERSIST_NO_START;
+            }
             // two processes that collided do not try again at the same moment
+            turn.unlock();
             std::this_thread::sleep_for(std::chrono::microseconds(100 * (1 + (getpid() * 7 + tries) % 32)));
+            turn.lock();
         }
         bool any = false;
         for (int q = 0; q < K; ++q) any = any || w->host[q].active;

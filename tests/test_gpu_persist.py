@@ -169,3 +169,52 @@ def test_half_and_whole_workgroups_same_column(n, K):
     assert all(done) and some == [its[0], its[-1]]
     assert torch.equal(Z, X[:, [0, K - 1]])
     A.close()
+
+
+@pytest.mark.parametrize("polls", [1, 2, 4, 8, 16, 32])
+def test_launches_that_do_not_start(polls, monkeypatch):
+    """A limit of a few polls on a launch's first exchange makes launches give
+    up, some or all of them: they are repeated, and the solve goes on as
+    launches per pass when they keep failing.  The same bits and counts each
+    time, with and without a start vector; batched columns reach their
+    residual (the launches add their dots in other groups)."""
+    print("start limit %d" % polls, flush=True)
+    rng = np.random.default_rng(polls)
+    for n, kw in ((700, dict(ortho=P.MGS)), (40000, dict(ortho=P.CGS2)),
+                  (90000, dict(ortho=P.MGS, precision=P.F32)), (200000, dict(ortho=P.MGS))):
+        csr = _line(n, 7, n)
+        A = P.Matrix.from_csr(n, n, *csr)
+        b = torch.as_tensor(rng.standard_normal(n), device=DEV)
+        for x0 in (None, torch.as_tensor(rng.standard_normal(n), device=DEV)):
+            got = []
+            for limit in (None, polls):
+                if limit:
+                    monkeypatch.setenv("PHG_XCH_START", str(limit))
+                x = torch.full_like(b, 7.0) if x0 is None else x0.clone()
+                info = A.solve(x, b, rtol=1e-10, restart=4, use_x0=x0 is not None, **kw)
+                monkeypatch.delenv("PHG_XCH_START", raising=False)
+                got.append((x, info))
+            (x, ref), (y, info) = got
+            assert ref["restarts"] > 2 and ref["cycle_launches"] == ref["restarts"]
+            keys = ("iterations", "restarts", "refinements", "rel_residual", "converged")
+            assert all(info[k] == ref[k] for k in keys) and torch.equal(x, y), (n, info, ref)
+            if polls == 1 and n == 200000:  # no workgroup but the last sees all slots at once
+                assert info["cycle_launches"] == 16
+        A.close()
+    for n, K in ((1000, 40), (30000, 7)):
+        csr = _line(n, 7, n)
+        A = P.Matrix.from_csr(n, n, *csr)
+        Bh = rng.standard_normal((n, K))
+        Bh[:, -1] = 0.0
+        B = torch.as_tensor(Bh, device=DEV)
+        for x0 in (None, torch.as_tensor(rng.standard_normal((n, K)), device=DEV)):
+            _, ref, _ = _batch(A, B, x0, 1, ortho=P.CGS2, restart=4)
+            monkeypatch.setenv("PHG_XCH_START", str(polls))
+            X, its, done = _batch(A, B, x0, 1, ortho=P.CGS2, restart=4)
+            monkeypatch.delenv("PHG_XCH_START")
+            assert all(done) and max(abs(a - c) for a, c in zip(its, ref)) <= 1, (its, ref)
+            for q in range(K):
+                x = np.ascontiguousarray(X[:, q].cpu().numpy())
+                scale = np.linalg.norm(Bh[:, q]) or 1.0
+                assert np.linalg.norm(Bh[:, q] - O.spmv(*csr, x)) <= 1.001e-10 * scale, q
+        A.close()
