@@ -2,9 +2,9 @@
 // workspace that a matrix keeps for it, and its entry.
 #pragma once
 #include <algorithm>
-#include <mutex>
 
 #include "krylov.h"
+#include "persist_turns.h"
 #include "phg_internal.h"
 
 namespace phg {
@@ -56,7 +56,7 @@ struct PersistWork {
     ~PersistWork();
 };
 
-std::mutex& persist_mutex(int dev);  // held while a device's launches run
+PersistTurns& persist_turns(int dev);  // of the device's launches
 
 // Workgroups of n rows: of 512 threads 1024 rows each, of 256 threads (half
 // of those 1024 rows each) two where the rows past the last 1024 need both.

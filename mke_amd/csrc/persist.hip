@@ -21,6 +21,9 @@
 // Columns are independent: each group of G workgroups runs its own cycles
 // and stops by itself, so the batched solves of small meshes (gmres_batch)
 // run here as one launch.
+#include <map>
+#include <mutex>
+
 #define PS_BS 512
 #include "persist_run.h"
 
@@ -94,12 +97,18 @@ PersistWork::~PersistWork()
     if (host) (void)hipHostFree(host);
 }
 
-// Launches of one device take turns: two that each hold half of the CUs would
-// wait for each other until they give up.
-std::mutex& persist_mutex(int dev)
+PersistTurns& persist_turns(int dev)
 {
-    static std::mutex m[64];
-    return m[dev & 63];
+    static std::mutex mu;
+    static std::map<int, PersistTurns>* m = new std::map<int, PersistTurns>();  // kept until exit
+    std::lock_guard<std::mutex> l(mu);
+    auto it = m->find(dev);
+    if (it == m->end()) {
+        int cus = 0;
+        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        it = m->try_emplace(dev, cus).first;
+    }
+    return it->second;
 }
 
 void persist_destroy(PersistWork* w) { delete w; }

@@ -7,7 +7,6 @@
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
 #include <thread>
 
 #include "krylov.h"
@@ -84,8 +83,8 @@ constexpr int PS_M = 32;      // largest restart
 // a start vector) is written before the second exchange: a launch that
 // continues a solve begins with an exchange of no values, whose 1.7 to 2.7 us
 // are 1 to 2 % of a cycle.  The abort flag is the column's own: the other
-// columns of the launch, which may be far along, go on.  Within a process
-// launches take turns (persist_mutex).  A cooperative launch would give the
+// columns of the launch, which may be far along, go on.  Within a process only
+// launches that fit the device together run at the same time (persist_turns.h).  A cooperative launch would give the
 // same guarantee but is refused to every process of a GPU except the first
 // that asks.
 struct Hop {
@@ -637,6 +636,36 @@ int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int
     return PHG_OK;
 }
 
+// The launches that a stream runs from begin to end, one after the other, of
+// at most so many workgroups each.
+struct Turn {
+    PersistTurns& turns;
+    int workgroups;
+    bool in = false;
+    Turn(PersistTurns& t, int w) : turns(t), workgroups(w) {}
+    Turn(const Turn&) = delete;
+    Turn& operator=(const Turn&) = delete;
+    ~Turn() { end(); }
+    hipError_t begin(hipStream_t s)
+    {
+        hipError_t e = hipSuccess;
+        if (!turns.try_enter(workgroups)) {
+            // other threads' launches run: wait for this stream's earlier work
+            // first, so that nobody waits for that while it is this one's turn
+            e = hipStreamSynchronize(s);
+            if (e != hipSuccess) return e;
+            turns.enter(workgroups);
+        }
+        in = true;
+        return e;
+    }
+    void end()
+    {
+        if (in) turns.leave(workgroups);
+        in = false;
+    }
+};
+
 template <typename VT, typename MT, int ORTHO>
 int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
         const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles, int max_rounds,
@@ -675,13 +704,7 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
     }
     int dev = 0;
     PHG_HIP(hipGetDevice(&dev));
-    std::unique_lock<std::mutex> turn(persist_mutex(dev), std::try_to_lock);
-    if (!turn.owns_lock()) {
-        // another thread's solve runs: wait for this stream's earlier work
-        // first, so that nobody waits for that while it is this one's turn
-        PHG_HIP(hipStreamSynchronize(s));
-        turn.lock();
-    }
+    PersistTurns& turns = persist_turns(dev);
     volatile int* abort_host = (int*)(w->host + w->host_k);
     int tries = 0;
     for (int first = 1;; first = 0) {
@@ -691,8 +714,10 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
         // did not start
         for (bool again = false;; again = true) {
             *abort_host = 0;
-            if (ms) PHG_HIP(hipEventRecord(w->ev[0], s));
             const int step = again ? 1 : per;
+            Turn turn(turns, G * step);
+            PHG_HIP(turn.begin(s));
+            if (ms) PHG_HIP(hipEventRecord(w->ev[0], s));
             for (int q0 = 0; q0 < K; q0 += step) {
                 const int kq = std::min(step, K - q0);
                 bool any = false;
@@ -701,13 +726,17 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
                 if (!any) continue;
                 const int rc = launch<VT, MT, ORTHO>(A, E, w, q0, kq, K, B, X, o, dscale, stall,
                                                      max_cycles, first, s);
-                if (rc) return rc;
+                if (rc) {
+                    (void)hipStreamSynchronize(s);  // those before it, in this turn
+                    return rc;
+                }
                 if (launches) ++*launches;
             }
             if (ms) PHG_HIP(hipEventRecord(w->ev[1], s));
             const hipError_t e = hipStreamSynchronize(s);
             if (e != hipSuccess) w->ring_k = 0;
             PHG_HIP(e);
+            turn.end();
             if (ms) {
                 float t = 0.0f;
                 PHG_HIP(hipEventElapsedTime(&t, w->ev[0], w->ev[1]));
@@ -726,9 +755,7 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
                 return PERSIST_NO_START;
             }
             // two processes that collided do not try again at the same moment
-            turn.unlock();
             std::this_thread::sleep_for(std::chrono::microseconds(100 * (1 + (getpid() * 7 + tries) % 32)));
-            turn.lock();
         }
         bool any = false;
         for (int q = 0; q < K; ++q) any = any || w->host[q].active;

@@ -218,3 +218,42 @@ def test_launches_that_do_not_start(polls, monkeypatch):
                 scale = np.linalg.norm(Bh[:, q]) or 1.0
                 assert np.linalg.norm(Bh[:, q] - O.spmv(*csr, x)) <= 1.001e-10 * scale, q
         A.close()
+
+
+def test_threads_solve_at_once():
+    """Solves of several threads, each with a matrix and a stream of its own,
+    small ones that run beside each other and ones that need the whole
+    device: the bits of the same solve alone."""
+    import threading
+    print("threads", flush=True)
+    sizes = [(3000, 1), (3000, 1), (20000, 2), (200000, 1), (60000, 4), (700, 30)]
+    jobs = []
+    for i, (n, K) in enumerate(sizes):
+        A = P.Matrix.from_csr(n, n, *_line(n, 7, n + i))
+        B = torch.as_tensor(np.random.default_rng(i).standard_normal((n, K)), device=DEV)
+        X = torch.zeros_like(B)
+        A.solve_batch(X, B, rtol=1e-10)
+        jobs.append((A, B, X))
+    torch.cuda.synchronize()
+    bad, gate = [], threading.Barrier(len(jobs))
+
+    def work(i):
+        A, B, X = jobs[i]
+        try:
+            stream = torch.cuda.Stream()
+            gate.wait(60)
+            with torch.cuda.stream(stream):
+                for _ in range(40):
+                    Y = torch.zeros_like(B)
+                    A.solve_batch(Y, B, rtol=1e-10, stream=stream)
+                    if not torch.equal(X, Y):
+                        bad.append(i)
+        except Exception as e:  # reported below: an assertion here would be lost
+            bad.append((i, e))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad

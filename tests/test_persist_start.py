@@ -9,8 +9,12 @@ its column are all there, and so on; the first thing that a repeated launch
 would read is written after exchange `quiet` - 1.  While a slot of exchange 0 is
 missing a workgroup may give up: it sets the abort flag and leaves its CU to
 the next.  A workgroup that waits may see the flag and leave."""
+import os
+import subprocess
+
 import pytest
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HOPS = 3
 
 
@@ -87,3 +91,77 @@ def test_column_goes_on_beside_one_that_gives_up():
 
     assert not stopped(outcomes(2, (2, 3), 4, False))
     assert stopped(outcomes(2, (2, 3), 4, True))
+
+
+TURNS = r"""
+#include <atomic>
+#include <chrono>
+#include <cstdio>
+#include <thread>
+#include <vector>
+#include "persist_turns.h"
+using phg::PersistTurns;
+
+// threads that each hold a turn until `together` of them do at once, or 2 s
+static bool meet(PersistTurns& t, std::vector<int> workgroups, int together)
+{
+    std::atomic<int> in{0}, most{0};
+    std::vector<std::thread> threads;
+    for (int w : workgroups)
+        threads.emplace_back([&, w] {
+            t.enter(w);
+            const int now = ++in;
+            for (int m = most; now > m && !most.compare_exchange_weak(m, now);) {}
+            for (int k = 0; k < 2000 && most < together; ++k)
+                std::this_thread::sleep_for(std::chrono::milliseconds(1));
+            --in;
+            t.leave(w);
+        });
+    for (auto& th : threads) th.join();
+    return most >= together;
+}
+
+int main()
+{
+    PersistTurns t(256);
+    // as many small ones as have a shader engine's CUs to themselves
+    if (!meet(t, {22, 22}, 2) || !meet(t, {161, 64}, 2)) return 1;
+    if (!meet(t, {1, 9, 32, 7, 11, 22, 3, 5}, 8)) return 2;
+    // 33 workgroups put two on an engine: 4 x 2 + 1 are more than its 8 CUs
+    for (int w : {33, 33, 64, 50})
+        if (!t.try_enter(w)) return 3;
+    if (t.try_enter(1)) return 4;
+    for (int w : {33, 33, 64, 50}) t.leave(w);
+    // a whole device's launch alone, also on a device with fewer CUs
+    if (!t.try_enter(256) || t.try_enter(1)) return 5;
+    t.leave(256);
+    PersistTurns small(32);
+    if (!small.try_enter(64) || small.try_enter(1)) return 6;
+    small.leave(64);
+    // who waits is not passed: a small launch comes after the big one that
+    // came before it
+    if (!t.try_enter(22)) return 7;
+    std::atomic<int> order{0};
+    int big = 0;
+    std::thread first([&] { t.enter(256); big = ++order; t.leave(256); });
+    std::this_thread::sleep_for(std::chrono::milliseconds(100));
+    if (t.try_enter(22)) return 8;
+    t.leave(22);
+    first.join();
+    if (big != 1 || !t.try_enter(22)) return 9;
+    t.leave(22);
+    std::puts("ok");
+    return 0;
+}
+"""
+
+
+def test_turns_of_a_process(tmp_path):
+    """Launches of several threads run at the same time where they are sure to
+    be resident together, and only there (csrc/persist_turns.h)."""
+    src, exe = tmp_path / "turns.cpp", tmp_path / "turns"
+    src.write_text(TURNS)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I",
+                    os.path.join(ROOT, "mke_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", r
