@@ -222,10 +222,11 @@ typedef struct {
     int refinements;      /* outer refinement steps (mixed forms)         */
     double rel_residual;  /* true FP64 ||b - A x|| / ||b|| at exit          */
     int converged;
-    int cycle_launches;   /* persistent cycles: kernels launched, and      */
+    int cycle_launches;   /* persistent cycles: kernels launched (in a batch
+                             for all its columns), and                  */
     double cycle_ms;      /* their summed duration (HIP events recorded on
-                             the solve's stream around each launch); 0
-                             for the other forms                        */
+                             the solve's stream around each launch; not
+                             taken in a batch); 0 for the other forms   */
 } phg_gmres_info;
 
 void phg_gmres_default_opts(phg_gmres_opts *o);
@@ -263,8 +264,12 @@ int phg_block_gmres(phg_matrix_t A, int nrhs, const double *d_B, double *d_X,
 /* d_B, d_X: n_rows x nrhs FP64, row-major (entry (i, q) at i * nrhs + q).
  * opts->restart <= 32, opts->ortho PHG_CGS2 or PHG_CGS1, opts->precision
  * PHG_F64 or mixed (PHG_F32 / PHG_BF16 inner Krylov, FP64 refinement).
- * A column's result does not depend on the other columns of the call (the
- * form that runs, opts->persistent, follows from the sizes alone).
+ * A column's result does not depend on the other columns of the call.  Its
+ * last bits may depend on how many there are: the form that runs
+ * (opts->persistent) follows from the sizes, nrhs among them, and the launches
+ * group their sums by nrhs rounded up to a power of two.  Other work on the
+ * device can change them too, where it keeps the persistent form from starting
+ * (opts->persistent = 0: always the launches).
  * infos: nrhs host entries (may be NULL).  Returns PHG_ERR_NOCONV unless
  * every column converged. */
 int phg_gmres_batch(phg_matrix_t A, int nrhs, const double *d_B, double *d_X,
@@ -275,7 +280,7 @@ int phg_gmres_batch(phg_matrix_t A, int nrhs, const double *d_B, double *d_X,
  * (1, 2, 4, 8 or 16) of one column; the value is kept per process for each
  * (n_rows, nrhs rounded up to a power of two, precision) shape and fixes the
  * grouping of every dot product's block partials, so results are bitwise
- * reproducible for a fixed value.  Untuned shapes take the largest value
+ * reproducible for a fixed value (the persistent form does not use it).  Untuned shapes take the largest value
  * (at most 8) that still gives >= 1024 workgroups; preconditioned solves
  * (phg_gmres_batch_mg) always take that default, whatever is tuned or pinned
  * for the plain form.  phg_gmres_batch_tune times one

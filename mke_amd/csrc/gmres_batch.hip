@@ -23,7 +23,9 @@
 //
 // Reductions are deterministic and do not depend on the column's position
 // or on the other columns: a column's result is bit-identical whatever else
-// is in the batch, provided KP is the same.  A restart cycle is captured in
+// is in the batch, provided K is the same.  In the persistent form below it is the
+// same bits for every K, in the launches for every K of one KP; which form
+// runs depends on K too.  A restart cycle is captured in
 // one hipGraph and replayed; the host reads a K-entry summary per cycle.
 //
 // Where the columns' rows fit the chip in few enough launches, the solve runs
@@ -1057,12 +1059,14 @@ int batch_run(phg_matrix_s* A, const Ell<MT>& E, BatchWork* w, int K, const doub
         }
         all = all && h.converged;
         if (infos) {
+            const int launches = from ? infos[q].cycle_launches : 0;
             memset(&infos[q], 0, sizeof infos[q]);
             infos[q].iterations = h.iters;
             infos[q].restarts = h.cycles;
             infos[q].refinements = o.precision == PHG_F64 ? 0 : h.cycles;
             infos[q].rel_residual = h.rel;
             infos[q].converged = h.converged;
+            infos[q].cycle_launches = launches;
         }
     }
     return all ? PHG_OK : PHG_ERR_NOCONV;
@@ -1109,8 +1113,11 @@ void set_shape_rpt(int n, int kp, int prec, int rpt)
 // kernels here: 26 us for the four launches of a step with one Gram-Schmidt
 // pass, 43 us for the six with two, and the vectors they read and write at
 // 4.2 TB/s.  A persistent launch: 6.8 to 12 us, and 0.01 us per workgroup of
-// a column.  Measured at levels 4 to 7 with 1 to 64 columns the model is
-// within 15 % of either; per step, here and persistent: level 5 x 8 columns
+// a column.  Of 92 shapes measured in both forms at levels 4 to 7 with 1 to 64
+// columns the model picks the faster one in all; its times are off by up to
+// 22 % (launches) and 29 % (persistent, 7 us steps of one column).  It takes
+// K as it is, not KP: 24 mass columns at level 6 are faster in four persistent
+// launches, 32 as launches.  Per step, here and persistent: level 5 x 8 columns
 // FP64 CGS2 48 and 12 us, level 6 x 64 303 and 144, level 7 x 1 56 and 14,
 // level 7 x 16 277 and 234; level 7 x 16 FP32 CGS1 103 and 145; mass solves
 // (restart 8, CGS1) level 6 x 24 61 and 52, level 6 x 64 101 and 143.
@@ -1136,8 +1143,11 @@ int batch_persistent(phg_matrix_s* A, int K, const double* B, double* X, const p
     if (!w) w = new PersistWork();
     // a launch ends after some 4,000 Arnoldi steps (50 ms) for the host to look
     const int max_cycles = std::max(1, 4096 / o.restart);
+    int launches = 0;
     const int rc = persist_solve(A, w, K, B, X, o, o.precision == PHG_F64 && o.diag_scale, true,
-                                 max_cycles, rounds, nullptr, nullptr, s);
+                                 max_cycles, rounds, &launches, nullptr, s);
+    if (rc == PERSIST_NO_START && infos)
+        for (int q = 0; q < K; ++q) infos[q].cycle_launches = launches;
     if (rc) return rc;
     bool all = true;
     for (int q = 0; q < K; ++q) {
@@ -1150,6 +1160,7 @@ int batch_persistent(phg_matrix_s* A, int K, const double* B, double* X, const p
             infos[q].refinements = o.precision == PHG_F64 ? 0 : h.cycles;
             infos[q].rel_residual = h.rel;
             infos[q].converged = h.converged;
+            infos[q].cycle_launches = launches;
         }
     }
     return all ? PHG_OK : PHG_ERR_NOCONV;

@@ -3,8 +3,8 @@ of the GPU SphereJacobian (phg_jacobian_*), through the C ABI.
 
 Bars: each column's true FP64 residual <= rtol (checked on the host with the
 oracle's SpMV) and its forward error against a tight oracle solve; a
-column's result is bit-identical whatever else is in the batch (same padded
-width); GPU calc2 against the oracle restatement (direct mass solves) within
+column's result is bit-identical whatever else is in the batch (same width
+and form); GPU calc2 against the oracle restatement (direct mass solves) within
 1e-11 of max |J| (the GPU mass solves stop at 1e-13)."""
 import numpy as np
 import pytest

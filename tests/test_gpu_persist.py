@@ -53,6 +53,8 @@ def _check(n, width, **kw):
     rel = np.linalg.norm(bh - O.spmv(*csr, x.cpu().numpy())) / np.linalg.norm(bh)
     assert info["converged"] and rel <= 1.001e-10, (info, rel)
     assert info["iterations"] == ref["iterations"] and torch.equal(x, y), (info, ref)
+    here = n <= 262144 and kw.get("restart", 30) <= 32
+    assert info["cycle_launches"] == (info["restarts"] if here else 0) and not ref["cycle_launches"]
     A.close()
 
 
@@ -93,8 +95,9 @@ def test_start_vector_and_zero_right_side():
     A.close()
 
 
-def _batch(A, B, x0=None, persistent=1, **kw):
-    """phg_gmres_batch with opts.persistent given."""
+def _batch(A, B, x0=None, persistent=1, runs=None, **kw):
+    """phg_gmres_batch with opts.persistent given; runs: whether the persistent
+    form is the one that does."""
     import ctypes as C
     from mke_amd.phelm import GmresInfo, GmresOpts, check
     o = GmresOpts()
@@ -107,6 +110,8 @@ def _batch(A, B, x0=None, persistent=1, **kw):
     infos = (GmresInfo * B.shape[1])()
     check(P.lib().phg_gmres_batch(A.h, B.shape[1], B.data_ptr(), X.data_ptr(), C.byref(o), infos,
                                   None), "phg_gmres_batch")
+    runs = persistent if runs is None else runs
+    assert all((i.cycle_launches > 0) == bool(runs) for i in infos)
     return X, [i.iterations for i in infos], [i.converged for i in infos]
 
 
@@ -257,3 +262,76 @@ def test_threads_solve_at_once():
     for t in threads:
         t.join()
     assert not bad, bad
+
+
+@pytest.mark.parametrize("n,opts,inside,outside", [
+    (163841, dict(ortho=P.CGS1, precision=P.F32), 12, 13),
+    (40961, dict(ortho=P.CGS1, restart=8, diag_scale=1), 24, 32)])
+def test_batch_widths_of_both_forms(n, opts, inside, outside):
+    """Numbers of columns with the same padded width on either side of the
+    line between the forms: a column's bits are the same for every number on
+    one side, and across the line the residual is."""
+    csr = _line(n, 7, n)
+    A = P.Matrix.from_csr(n, n, *csr)
+    Bh = np.random.default_rng(n).standard_normal((n, outside + 1))
+    B = torch.as_tensor(Bh, device=DEV)
+
+    def run(k, runs):
+        X, its, done = _batch(A, B[:, :k].contiguous(), None, 1, runs=runs, **opts)
+        assert all(done)
+        x = np.ascontiguousarray(X[:, 1].cpu().numpy())
+        assert np.linalg.norm(Bh[:, 1] - O.spmv(*csr, x)) <= 1.001e-10 * np.linalg.norm(Bh[:, 1])
+        return X[:, :2], its[:2]
+
+    few, most, over = run(2, True), run(inside, True), run(outside, False)
+    assert torch.equal(few[0], most[0]) and few[1] == most[1]
+    if outside < 16:
+        assert torch.equal(over[0], run(outside + 1, False)[0])
+    assert max(abs(a - b) for a, b in zip(most[1], over[1])) <= 1
+
+
+def test_batch_of_more_than_one_launch():
+    """A launch ends after 4,096 Arnoldi steps of a column; slow columns take
+    several, beside columns that stop in the first."""
+    nx = 140
+    i = np.arange(nx * nx)
+    x, y = i % nx, i // nx
+    cols = np.stack([i - nx, i - 1, i, i + 1, i + nx], 1)
+    there = np.stack([y > 0, x > 0, x >= 0, x < nx - 1, y < nx - 1], 1)
+    vals = np.full(cols.shape, -1.0)
+    vals[:, 2] = 4.0 + 1e-4
+    csr = (np.concatenate([[0], np.cumsum(there.sum(1))]).astype(np.int32),
+           cols[there].astype(np.int32), vals[there])
+    n = nx * nx
+    A = P.Matrix.from_csr(n, n, *csr)
+    Bh = np.random.default_rng(5).standard_normal((n, 3))
+    Bh[:, 1] = O.spmv(*csr, np.sin(np.pi * (x + 1) / (nx + 1)) * np.sin(np.pi * (y + 1) / (nx + 1)))
+    B = torch.as_tensor(Bh, device=DEV)
+    X, its, done = _batch(A, B, None, 1, ortho=P.CGS2, restart=8)
+    Y, ref, _ = _batch(A, B, None, 0, ortho=P.CGS2, restart=8)
+    print(its, ref)
+    assert all(done) and its[0] > 4096 and its[1] < 10, its
+    for q in range(3):
+        r = Bh[:, q] - O.spmv(*csr, np.ascontiguousarray(X[:, q].cpu().numpy()))
+        assert np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(Bh[:, q]), q
+    # the same stopping residual: errors of at most cond(A) = 8 / 0.0011 times it
+    assert float((X - Y).norm()) <= 2 * 7400 * 1e-10 * float(Y.norm())
+
+
+def test_batch_with_columns_that_are_not_finite():
+    """Columns with a NaN or an infinity stop at once and leave the others'
+    bits alone."""
+    n, K = 20000, 5
+    csr = _line(n, 7, n)
+    A = P.Matrix.from_csr(n, n, *csr)
+    B = torch.as_tensor(np.random.default_rng(8).standard_normal((n, K)), device=DEV)
+    X, its, _ = _batch(A, B, None, 1, ortho=P.CGS2)
+    B[17, 1], B[n - 1, 3] = float("nan"), float("inf")
+    for persistent in (1, 0):
+        Y, got, done = _batch(A, B, None, persistent, ortho=P.CGS2)
+        assert [bool(d) for d in done] == [True, False, True, False, True]
+        assert got[1] == 0 and got[3] == 0 and abs(got[0] - its[0]) <= 1
+        if persistent:
+            assert torch.equal(Y[:, ::2], X[:, ::2])
+    Z, got, done = _batch(A, B[:, ::2].contiguous(), None, 1, ortho=P.CGS2)
+    assert all(done) and torch.equal(Z, X[:, ::2])
