@@ -313,10 +313,10 @@ def test_dump_operator_matches_oracle(op, kind, cm, cl, tmp_path):
 @pytest.mark.parametrize("precision", [P.F64, P.F32])
 @pytest.mark.parametrize("level", [4, 5, 7])
 def test_gmres_persistent_cycle_same_bits(level, precision):
-    """The persistent MGS cycle (one cooperative kernel per restart cycle,
-    dot partials exchanged through device memory) gives the bits of the
-    kernel-per-pass form, FP64 and mixed FP32, with the same iteration and
-    restart counts; two runs of it give the same bits."""
+    """The persistent MGS cycle (one kernel per restart cycle, dot partials
+    exchanged through device memory) gives the bits of the launch-per-pass
+    form, FP64 and mixed FP32, with the same iteration and restart counts; two
+    runs of it give the same bits."""
     print("gmres persistent vs per-pass level=%d precision=%d" % (level, precision), flush=True)
     pm, _ = _mesh(level)
     A = P.Matrix.assemble(pm, P.HELMHOLTZ, CM, CL)
@@ -335,7 +335,7 @@ def test_gmres_persistent_cycle_same_bits(level, precision):
     for i in (1, 2):
         assert all(infos[i][k] == infos[0][k] for k in keys), (infos[i], infos[0])
         assert torch.equal(xs[i], xs[0])
-    # one cooperative launch per restart cycle, timed by HIP events
+    # one launch per restart cycle, timed by HIP events
     assert infos[0]["cycle_launches"] == 0
     assert infos[1]["cycle_launches"] == infos[1]["restarts"] and infos[1]["cycle_ms"] > 0
 
@@ -362,13 +362,14 @@ def test_gmres_persistent_cycle_gives_up_cleanly(monkeypatch):
 
 @pytest.mark.parametrize("ortho", [P.CGS2, P.MGS])
 def test_gmres_level8_same_bits_on_fresh_workspaces(ortho):
-    """Level 8 runs the single right-hand-side kernels on 641 workgroups, more
-    than the device holds at once, so workgroups of one launch run one after
-    another.  Each solve on a freshly assembled matrix (a fresh workspace)
-    gives the same bits and iteration count: no block may read a partial
-    another block of the same launch overwrites (the CGS2 step kernel once
-    read the previous step's norm partials from the slot its first-pass dots
-    go to, and its iteration count varied from run to run)."""
+    """Level 8 runs the single right-hand-side kernels on 257 workgroups, one
+    more than there are CUs (fewer than the device holds at once where two
+    fit a CU).  Each solve on a freshly assembled matrix (a fresh workspace)
+    gives the same bits and iteration count: no block may read a partial that
+    another block of the same launch overwrites.  (An earlier shape of 641
+    workgroups, run one after another, showed such a read: the CGS2 step kernel
+    took the previous step's norm partials from the slot that its first-pass
+    dots went to, and its iteration count varied.)"""
     print("gmres level 8 fresh workspaces ortho=%d" % ortho, flush=True)
     pm = P.Mesh.sphere(8)
     Mm = P.Matrix.assemble(pm, P.MASS)
