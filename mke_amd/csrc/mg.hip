@@ -683,8 +683,8 @@ MgcLevel<T, typename MgT<T>::MT> mgc_level(MgLevel& l)
 
 // z = V-cycle(v): v, z are n x KP (finest level); enqueued on s.  Levels 3
 // and below are one launch; above, a level takes four launches for up to
-// MG_FUSE columns and six for more, where the passes are bound by memory and
-// the recomputation of the fused ones would show.
+// MG_FUSE columns (C = 1) and six for more, where the passes are bound by
+// memory and the recomputation of the fused ones would show.
 template <typename T, int C>
 void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
 {
@@ -698,8 +698,8 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
         return;
     }
     const int kc = nlev - 2;  // level 3: with level 2 in one launch
-    const bool fuse = KP <= MG_FUSE;
-    const int l1 = __builtin_ctz((unsigned)KP), lk = l1 - __builtin_ctz((unsigned)C);
+    constexpr bool fuse = C == 1;
+    const int lk = __builtin_ctz((unsigned)KP) - __builtin_ctz((unsigned)C);
     // descend: level 0 takes b = v (read directly), result to z
     const T* bk = v;
     for (int k = 0; k < kc; ++k) {
@@ -710,9 +710,9 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
         T* xa = (k == 0) ? z : B::x0(l);
         hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_jacobi_zero2<T, MT, C>), grid_for(w), dim3(256), 0, s,
                            l.n, lk, E.width, E.col.p, E.val.p, B::dinv(l), bk, xa, om);
-        if (fuse) {
+        if constexpr (fuse) {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual_restrict<T, MT>),
-                               grid_for((size_t)c.n * KP * 8), dim3(256), 0, s, c.n, l.n, l1, E.width,
+                               grid_for((size_t)c.n * KP * 8), dim3(256), 0, s, c.n, l.n, lk, E.width,
                                E.col.p, E.val.p, xa, bk, l.rrp.p, l.ridx.p, B::rw(l), B::b(c));
         } else {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_residual<T, MT, C>), grid_for(w), dim3(256), 0, s,
@@ -734,7 +734,7 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
         const size_t w = (size_t)l.n * KP / C;
         const T* bl = (k == 0) ? v : B::b(l);
         T* xa = (k == 0) ? z : B::x0(l);
-        if (fuse) {
+        if constexpr (fuse) {
             hipLaunchKernelGGL(HIP_KERNEL_NAME(mg_prolong_jacobi<T, MT>), grid_for(w), dim3(256), 0,
                                s, l.n, lk, E.width, E.col.p, E.val.p, B::dinv(l), l.p0.p, l.p1.p,
                                B::x0(c), xa, bl, B::x1(l), om);
@@ -752,13 +752,12 @@ void mg_apply_t(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
 // Columns per thread: 16 bytes of a row where the fused passes (which are
 // launch bound) don't run: a solve of 64 FP32 columns at level 7 9.76 ms with
 // one column per thread, 7.70 ms with four.  Every array of a level starts on
-// 16 bytes and its rows of at least 16 columns are a multiple of them.
+// 16 bytes and its rows of at least 16 columns are a multiple of them; v and
+// z are such vectors too.
 template <typename T>
 void mg_apply_c(phg_mg_s* M, int KP, const T* v, T* z, hipStream_t s)
 {
-    constexpr int C = 16 / sizeof(T);
-    const bool wide = KP > MG_FUSE && ((size_t)v | (size_t)z) % 16 == 0;
-    if (wide) mg_apply_t<T, C>(M, KP, v, z, s);
+    if (KP > MG_FUSE) mg_apply_t<T, 16 / sizeof(T)>(M, KP, v, z, s);
     else mg_apply_t<T, 1>(M, KP, v, z, s);
 }
 
