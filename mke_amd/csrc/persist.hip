@@ -9,8 +9,8 @@
 //
 // What bounds it: the exchanges, about 2.7 us each among 161 workgroups and
 // 1.7 us among 41, and the instructions between them.  Level 7 FP64 MGS 11.5
-// us a step (57 us with a sum per basis vector, 25.0 -> 5.0 ms a solve), level
-// 4 7 us (1.37 -> 0.29 ms a solve), 36,503 rows FP32 CGS2 6.25 -> 1.74 ms.
+// us a step (57 us with a sum per basis vector, 25.0 -> 5.1 ms a solve), level
+// 4 7 us (1.37 -> 0.29 ms a solve), 36,503 rows FP32 CGS2 6.25 -> 1.77 ms.
 // A step has two exchanges: the dots <v_i, w> of all basis vectors
 // in one, ||w|| and, for modified Gram-Schmidt, the dots of the updated w in
 // the other.  The latter are the products <v_i, v_{j+1}> that make

@@ -83,10 +83,10 @@ constexpr int PS_M = 32;      // largest restart
 // a start vector) is written before the second exchange: a launch that
 // continues a solve begins with an exchange of no values, whose 1.7 to 2.7 us
 // are 1 to 2 % of a cycle.  The abort flag is the column's own: the other
-// columns of the launch, which may be far along, go on.  Within a process only
-// launches that fit the device together run at the same time (persist_turns.h).  A cooperative launch would give the
-// same guarantee but is refused to every process of a GPU except the first
-// that asks.
+// columns of the launch, which may be far along, go on.  Within a process
+// only launches that fit the device together run at the same time
+// (persist_turns.h).  A cooperative launch would give the same guarantee but
+// is refused to every process of a GPU except the first that asks.
 struct Hop {
     xch_t* ring;
     int G, slot, e;  // G: slots of a row (padded workgroup count)
