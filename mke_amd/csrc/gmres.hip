@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "krylov.h"
@@ -49,6 +50,7 @@ constexpr int GM_MAXM = 64;
 constexpr int GM_MAXN = 1 << 20; // most rows
 constexpr int GM_RED = 1024;      // threads of the reducing workgroup
 constexpr int GM_BS = KR_STRIDE;  // threads of the others
+constexpr int GM_HALF = 32;       // basis entries of a row in registers at once
 
 struct GmresState {
     double R[GM_MAXM * GM_MAXM];  // rotated (upper triangular) columns
@@ -74,14 +76,21 @@ struct GmresWork {
     DevBuf<double> part;   // G x S block partials
     DevBuf<GmresState> st;
     GmresState* host = nullptr;  // pinned mirror
-    // captured restart cycle
+    // captured restart cycle, in parts
     hipStream_t cap = nullptr;
-    hipGraphExec_t exec = nullptr;
+    hipGraphExec_t exec[4] = {};  // a cycle's chunks and its end, or all in one
+    bool captured = false;
     const void* key[2] = {nullptr, nullptr};
     int key_m = 0, key_ortho = -1;
+    void drop_graphs()
+    {
+        for (auto& e : exec)
+            if (e) (void)hipGraphExecDestroy(e), e = nullptr;
+        captured = false;
+    }
     ~GmresWork()
     {
-        if (exec) (void)hipGraphExecDestroy(exec);
+        drop_graphs();
         if (cap) (void)hipStreamDestroy(cap);
         if (host) (void)hipHostFree(host);
     }
@@ -186,7 +195,7 @@ k_sumsq(int n, int R, const double* __restrict__ b, int S, double* __restrict__ 
 // Arnoldi step j < NV: v_j = W_src / h (stored), W_dst = A v_j, and the block
 // partials of <W_dst, v_i>, i <= j.  Row by row; a row's basis entries are
 // loaded without a branch (past j - 1 the last one again, not used), so that
-// all of them are in flight.
+// all of them are in flight, GM_HALF at a time.
 template <typename VT, typename MT, int NV>
 __global__ void __launch_bounds__(GM_BS)
 k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __restrict__ val,
@@ -195,6 +204,7 @@ k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __re
 {
     __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
     if (!st->active) return;
+    constexpr int N1 = NV < GM_HALF ? NV : GM_HALF;
     const VT inv = (VT)(1.0 / (j == 0 ? st->beta : st->hn));
     const int base = lblock() * GM_BS * R + threadIdx.x;
     double acc[NV];
@@ -204,26 +214,36 @@ k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __re
     for (int r = 0; r < R; ++r) {
         const int row = base + r * GM_BS;
         if (row >= n) break;
-        VT v[NV], vj, w;
+        VT v[N1], vj, w;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] = basis_at(V, ldv, max(min(i, j - 1), 0), row);
+        for (int i = 0; i < N1; ++i) v[i] = basis_at(V, ldv, max(min(i, j - 1), 0), row);
         krylov_rows<VT, MT, false, 1>(n, width, row, col, val, Wsrc, 1, inv, &vj, &w);
         vj = vj * inv;
         V[(size_t)j * ldv + row] = vj;
         Wdst[row] = w;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) acc[i] = fma(to_d(w), to_d(i == j ? vj : v[i]), acc[i]);
+        for (int i = 0; i < N1; ++i) acc[i] = fma(to_d(w), to_d(i == j ? vj : v[i]), acc[i]);
+        if constexpr (NV > N1) {
+#pragma unroll
+            for (int i = N1; i < NV; ++i) v[i - N1] = basis_at(V, ldv, max(min(i, j - 1), 0), row);
+#pragma unroll
+            for (int i = N1; i < NV; ++i)
+                acc[i] = fma(to_d(w), to_d(i == j ? vj : v[i - N1]), acc[i]);
+        }
     }
     dot_partials<NV>(acc, j, sh);
     write_partials(sh, j + 1, false, S, part);
 }
 
 // w -= sum_{i<=j} hc_i v_i, then the block partials of <w, v_i>, i <= j
-// (DOTS) and of ||w||^2 (norm).  For j < NV <= 32, row by row, with the row's
-// v_0..v_j kept in registers from the update to the dots: the basis is read
-// once.  The loads have no branch between them (past j row j again, with a
-// coefficient of 0): with one, level 8's updates with 32 vectors took 95 us
-// instead of 30.
+// (DOTS) and of ||w||^2 (norm).  Row by row, with the row's v_0..v_j kept in
+// registers from the update to the dots: the basis is read once.  The loads
+// have no branch between them (past j row j again, with a coefficient of 0):
+// with one, level 8's updates with 32 vectors took 95 us instead of 30.
+// Above GM_HALF vectors (restarts above 32) the first GM_HALF are read again
+// for their dots: 64 in registers do not fit beside their 64 sums.  A level-7
+// FP64 CGS2 solve with restart 64: 5.46 ms, with the whole basis read twice,
+// eight vectors at a time, 6.41 ms.
 template <typename VT, int NV, bool DOTS>
 __global__ void __launch_bounds__(GM_BS)
 k_update(int n, int R, VT* __restrict__ w, const VT* __restrict__ V, size_t ldv, int j, int norm,
@@ -235,6 +255,7 @@ k_update(int n, int R, VT* __restrict__ w, const VT* __restrict__ V, size_t ldv,
     if ((int)threadIdx.x < NV)
         hs[threadIdx.x] = (int)threadIdx.x <= j ? (VT)st->hc[threadIdx.x] : VT(0);
     __syncthreads();
+    constexpr int N1 = NV < GM_HALF ? NV : GM_HALF;
     const int base = lblock() * GM_BS * R + threadIdx.x;
     double acc[NV], nrm = 0.0;
 #pragma unroll
@@ -243,77 +264,35 @@ k_update(int n, int R, VT* __restrict__ w, const VT* __restrict__ V, size_t ldv,
     for (int r = 0; r < R; ++r) {
         const int row = base + r * GM_BS;
         if (row >= n) break;
-        VT v[NV];
+        VT v[N1];
         VT wr = w[row];
 #pragma unroll
-        for (int i = 0; i < NV; ++i) v[i] = basis_at(V, ldv, min(i, j), row);
+        for (int i = 0; i < N1; ++i) v[i] = basis_at(V, ldv, min(i, j), row);
 #pragma unroll
-        for (int i = 0; i < NV; ++i) wr = kfma(-hs[i], v[i], wr);
+        for (int i = 0; i < N1; ++i) wr = kfma(-hs[i], v[i], wr);
+        if constexpr (NV > N1) {
+#pragma unroll
+            for (int i = N1; i < NV; ++i) v[i - N1] = basis_at(V, ldv, min(i, j), row);
+#pragma unroll
+            for (int i = N1; i < NV; ++i) wr = kfma(-hs[i], v[i - N1], wr);
+        }
         w[row] = wr;
         nrm = fma(to_d(wr), to_d(wr), nrm);
         if (DOTS) {
+            if constexpr (NV > N1) {
 #pragma unroll
-            for (int i = 0; i < NV; ++i) acc[i] = fma(to_d(wr), to_d(v[i]), acc[i]);
+                for (int i = N1; i < NV; ++i) acc[i] = fma(to_d(wr), to_d(v[i - N1]), acc[i]);
+                const int again = opaque(row);  // loaded again, not kept
+#pragma unroll
+                for (int i = 0; i < N1; ++i) v[i] = basis_at(V, ldv, i, again);
+            }
+#pragma unroll
+            for (int i = 0; i < N1; ++i) acc[i] = fma(to_d(wr), to_d(v[i]), acc[i]);
         }
     }
     if (DOTS) dot_partials<NV>(acc, j, sh);
     if (norm) norm_partial(nrm, sh);
     write_partials(sh, DOTS ? j + 1 : 0, norm, S, part);
-}
-
-// The two kernels above for any j < 64 (restarts above 32), two rows at a
-// time, tier by tier: FIRST is the product and its dots, otherwise the update
-// (the basis read once for it and once for the dots).
-template <typename VT, typename MT, bool FIRST>
-__global__ void __launch_bounds__(GM_BS)
-k_long(int n, int R, int width, const int* __restrict__ col, const MT* __restrict__ val,
-       const VT* __restrict__ Wsrc, VT* __restrict__ V, size_t ldv, VT* __restrict__ w, int j,
-       int dots, int norm, int S, double* __restrict__ part, const GmresState* __restrict__ st)
-{
-    __shared__ double sh[GM_BS / 64][GM_MAXM + 1];
-    __shared__ VT hs[GM_MAXM];
-    if (!st->active) return;
-    const int lane = threadIdx.x & 63;
-    if (!FIRST && (int)threadIdx.x < GM_MAXM)
-        hs[threadIdx.x] = (int)threadIdx.x <= j ? (VT)st->hc[threadIdx.x] : VT(0);
-    if (FIRST) norm = 0;
-    __syncthreads();
-    const int base = lblock() * GM_BS * R + threadIdx.x;
-    double nrm = 0.0;
-    for (int i0 = 0; i0 <= j; i0 += KR_T) {
-        // the product or the whole update first, then the dots of this tier
-        double acc[KR_T];
-#pragma unroll
-        for (int q = 0; q < KR_T; ++q) acc[q] = 0.0;
-        for (int r = 0; r < R; ++r) {
-            const int row = base + r * GM_BS;
-            if (row >= n) break;
-            VT wr;
-            if (i0 == 0 && FIRST) {
-                const VT inv = (VT)(1.0 / (j == 0 ? st->beta : st->hn));
-                VT vj;
-                krylov_rows<VT, MT, false, 1>(n, width, row, col, val, Wsrc, 1, inv, &vj, &wr);
-                V[(size_t)j * ldv + row] = vj * inv;
-                w[row] = wr;
-            } else if (i0 == 0) {
-                wr = w[row];
-                for (int k = 0; k <= j; ++k) wr = kfma(-hs[k], V[(size_t)k * ldv + row], wr);
-                w[row] = wr;
-                nrm = fma(to_d(wr), to_d(wr), nrm);
-            } else {
-                wr = w[row];
-            }
-            if (!dots) continue;
-#pragma unroll
-            for (int q = 0; q < KR_T; ++q)
-                acc[q] = fma(to_d(wr), to_d(V[(size_t)min(i0 + q, j) * ldv + row]), acc[q]);
-        }
-        if (!dots) break;
-        const double s = reduce8(acc);
-        if ((lane & 7) == 0) sh[threadIdx.x >> 6][i0 + reduce8_value(lane)] = s;
-    }
-    if (norm) norm_partial(nrm, sh);
-    write_partials(sh, dots ? j + 1 : 0, norm, S, part);
 }
 
 // Adds the block partials of a pass and does the step's small dense work, in
@@ -324,7 +303,7 @@ k_long(int n, int R, int width, const int* __restrict__ col, const MT* __restric
 enum { RED_BNORM, RED_START, RED_FIRST, RED_AGAIN, RED_NORM };
 __global__ void __launch_bounds__(GM_RED)
 k_reduce(int what, int mgs, int j, int nv, int norm, int S, const double* __restrict__ part, int G,
-         GmresState* __restrict__ st)
+         GmresState* __restrict__ st, int* __restrict__ host_active)
 {
     __shared__ double s32[2][32][33];
     __shared__ double s_cs[2 * GM_MAXM], s_g[GM_MAXM], s_carry[GM_MAXM + 1], s_h[GM_MAXM + 8];
@@ -417,7 +396,10 @@ k_reduce(int what, int mgs, int j, int nv, int norm, int S, const double* __rest
             st->hn = hn;
             st->k = j + 1;
             st->iters = o.iters;
-            if (!o.cont) st->active = 0;
+            if (!o.cont) {
+                st->active = 0;
+                *host_active = 0;
+            }
         }
     }
 }
@@ -531,34 +513,38 @@ void update_nv(GmresWork* w, VT* dst, int j, bool dots, bool norm, hipStream_t s
                            dst, V, w->ldv, j, (int)norm, w->S, w->part.p, w->st.p);
 }
 
+// f(vectors of the kernel for step j, as a constant)
+template <typename F>
+void by_step(int j, F f)
+{
+    switch (j / 8) {
+    case 0: return f(std::integral_constant<int, 8>());
+    case 1: return f(std::integral_constant<int, 16>());
+    case 2: return f(std::integral_constant<int, 24>());
+    case 3: return f(std::integral_constant<int, 32>());
+    case 4: return f(std::integral_constant<int, 40>());
+    case 5: return f(std::integral_constant<int, 48>());
+    case 6: return f(std::integral_constant<int, 56>());
+    default: return f(std::integral_constant<int, 64>());
+    }
+}
+
 template <typename VT, typename MT>
 void step(const Ell<MT>& E, GmresWork* w, const VT* src, VT* dst, int j, hipStream_t s)
 {
-    if (j < 8) step_nv<VT, MT, 8>(E, w, src, dst, j, s);
-    else if (j < 16) step_nv<VT, MT, 16>(E, w, src, dst, j, s);
-    else if (j < 24) step_nv<VT, MT, 24>(E, w, src, dst, j, s);
-    else if (j < 32) step_nv<VT, MT, 32>(E, w, src, dst, j, s);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_long<VT, MT, true>), dim3(w->G), dim3(GM_BS), 0, s,
-                           w->n, w->R, E.width, E.col.p, E.val.p, src, (VT*)w->V.p, w->ldv, dst, j,
-                           1, 0, w->S, w->part.p, w->st.p);
+    by_step(j, [&](auto nv) { step_nv<VT, MT, decltype(nv)::value>(E, w, src, dst, j, s); });
 }
 
-template <typename VT, typename MT>
-void update(const Ell<MT>& E, GmresWork* w, VT* dst, int j, bool dots, bool norm, hipStream_t s)
+template <typename VT>
+void update(GmresWork* w, VT* dst, int j, bool dots, bool norm, hipStream_t s)
 {
-    if (j < 8) update_nv<VT, 8>(w, dst, j, dots, norm, s);
-    else if (j < 16) update_nv<VT, 16>(w, dst, j, dots, norm, s);
-    else if (j < 24) update_nv<VT, 24>(w, dst, j, dots, norm, s);
-    else if (j < 32) update_nv<VT, 32>(w, dst, j, dots, norm, s);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_long<VT, MT, false>), dim3(w->G), dim3(GM_BS), 0, s,
-                           w->n, w->R, E.width, E.col.p, E.val.p, (const VT*)nullptr, (VT*)w->V.p,
-                           w->ldv, dst, j, (int)dots, (int)norm, w->S, w->part.p, w->st.p);
+    by_step(j, [&](auto nv) { update_nv<VT, decltype(nv)::value>(w, dst, j, dots, norm, s); });
 }
 
+// Steps j0 .. j1-1 of a cycle of m, then with `end` the cycle's end.
 template <typename VT, typename MT>
-void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, bool cgs, hipStream_t s)
+void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, int j0, int j1, bool end,
+                   bool cgs, hipStream_t s)
 {
     const int n = w->n, G = w->G, S = w->S;
     const size_t ldv = w->ldv;
@@ -569,28 +555,30 @@ void enqueue_cycle(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, int m, bool 
     GmresState* st = w->st.p;
     const int mgs = cgs ? 0 : (sizeof(VT) == 4 ? 2 : 1);
     const dim3 grid(G), block(GM_BS), one(1), red(GM_RED);
-    for (int j = 0; j < m; ++j) {
+    for (int j = j0; j < j1; ++j) {
         VT* src = (j & 1) ? W1 : W0;
         VT* dst = (j & 1) ? W0 : W1;
         step<VT, MT>(E, w, src, dst, j, s);
         hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_FIRST, mgs, j, j + 1, 0, S, part, G,
-                           st);
+                           st, &w->host->active);
         if (cgs) {
-            update<VT, MT>(E, w, dst, j, true, false, s);
+            update<VT>(w, dst, j, true, false, s);
             hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_AGAIN, mgs, j, j + 1, 0, S, part,
-                               G, st);
+                               G, st, &w->host->active);
         }
         const bool dots = !cgs && j + 1 < m;
-        update<VT, MT>(E, w, dst, j, dots, true, s);
+        update<VT>(w, dst, j, dots, true, s);
         hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_NORM, mgs, j, dots ? j + 1 : 0, 1, S,
-                           part, G, st);
+                           part, G, st, &w->host->active);
     }
+    if (!end) return;
     hipLaunchKernelGGL(k_solve_y, one, dim3(64), 0, s, st);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_xupdate<VT>), dim3((n + GM_BS - 1) / GM_BS), block, 0, s,
                        n, V, ldv, st);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual<VT>), grid, block, 0, s, n, w->R, A->ell64.width,
                        A->ell64.col.p, A->ell64.val.p, W0, S, part, st);
-    hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, mgs, 0, 0, 1, S, part, G, st);
+    hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, mgs, 0, 0, 1, S, part, G, st,
+                       &w->host->active);
 }
 
 // iters, cycles: what a solve that is continued from x has done.
@@ -621,24 +609,31 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
     PHG_HIP(hipMemcpyAsync(st, &init, sizeof init, hipMemcpyHostToDevice, s));
     if (!o.use_x0) hipLaunchKernelGGL(k_fill0, dim3((n + 255) / 256), dim3(256), 0, s, n, x);
     hipLaunchKernelGGL(k_sumsq, grid, block, 0, s, n, w->R, b, S, part);
-    hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_BNORM, 0, 0, 0, 1, S, part, G, st);
+    hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_BNORM, 0, 0, 0, 1, S, part, G, st,
+                       &w->host->active);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_residual<VT>), grid, block, 0, s, n, w->R, A->ell64.width,
                        A->ell64.col.p, A->ell64.val.p, W0, S, part, st);
-    hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, 0, 0, 0, 1, S, part, G, st);
+    hipLaunchKernelGGL(k_reduce, one, red, 0, s, (int)RED_START, 0, 0, 0, 1, S, part, G, st,
+                       &w->host->active);
     PHG_HIP(hipGetLastError());
 
-    // the captured cycle; replayed only when built (or found current) here
-    bool graph_ready = false;
+    // the cycle in parts: steps from[c] .. from[c + 1] - 1, the last with its
+    // end.  Above 32 steps chunks end at steps 16, 32 (with 16 or more left)
+    // and m, and after each but the last the host looks whether the solve still
+    // runs: an idle step is 4 or 6 launches of 1.5 us, a look costs 20 us.
+    // Level 5, restart 64, FP64 CGS2 of 25 steps: 1072 -> 810 us.
+    const int parts = m <= 32 ? 1 : m < 48 ? 3 : 4;
+    const int from[5] = {0, parts == 1 ? m : 16, parts == 3 ? m : 32, m, m};
+    const auto enqueue = [&](int c, hipStream_t cs) {
+        enqueue_cycle<VT, MT>(A, E, w, m, from[c], from[c + 1], c == parts - 1, cgs, cs);
+    };
+    // captured; replayed only when built (or found current) here
     if (o.graph) {
-        graph_ready = true;
         const void* key[2] = {E.val.p, A->ell64.val.p};
-        const bool same = w->exec && w->key_m == m && w->key_ortho == o.ortho &&
+        const bool same = w->captured && w->key_m == m && w->key_ortho == o.ortho &&
                           !memcmp(key, w->key, sizeof key);
         if (!same) {
-            if (w->exec) {
-                PHG_HIP(hipGraphExecDestroy(w->exec));
-                w->exec = nullptr;
-            }
+            w->drop_graphs();
             // recorded on the caller's stream; the null stream cannot be
             // captured, so for it on a stream of the workspace (a stream
             // per workspace would also take a share of the process's few
@@ -648,13 +643,16 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
                 if (!w->cap) PHG_HIP(hipStreamCreateWithFlags(&w->cap, hipStreamNonBlocking));
                 cs = w->cap;
             }
-            hipGraph_t g = nullptr;
-            PHG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-            enqueue_cycle<VT, MT>(A, E, w, m, cgs, cs);
-            PHG_HIP(hipStreamEndCapture(cs, &g));
-            hipError_t e = hipGraphInstantiate(&w->exec, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            PHG_HIP(e);
+            for (int c = 0; c < parts; ++c) {
+                hipGraph_t g = nullptr;
+                PHG_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+                enqueue(c, cs);
+                PHG_HIP(hipStreamEndCapture(cs, &g));
+                hipError_t e = hipGraphInstantiate(&w->exec[c], g, nullptr, nullptr, 0);
+                (void)hipGraphDestroy(g);
+                PHG_HIP(e);
+            }
+            w->captured = true;
             memcpy(w->key, key, sizeof key);
             w->key_m = m;
             w->key_ortho = o.ortho;
@@ -664,13 +662,18 @@ int gmres_passes(phg_matrix_s* A, const Ell<MT>& E, GmresWork* w, const double* 
     for (;;) {
         PHG_HIP(hipMemcpyAsync(w->host, st, sizeof(GmresState), hipMemcpyDeviceToHost, s));
         PHG_HIP(hipStreamSynchronize(s));
-        const GmresState& h = *w->host;
-        if (h.converged || !h.active) break;
-        if (graph_ready) {
-            PHG_HIP(hipGraphLaunch(w->exec, s));
-        } else {
-            enqueue_cycle<VT, MT>(A, E, w, m, cgs, s);
-            PHG_HIP(hipGetLastError());
+        if (w->host->converged || !w->host->active) break;
+        for (int c = 0; c < parts; ++c) {
+            if (o.graph) {
+                PHG_HIP(hipGraphLaunch(w->exec[c], s));
+            } else {
+                enqueue(c, s);
+                PHG_HIP(hipGetLastError());
+            }
+            if (c < parts - 2) {
+                PHG_HIP(hipStreamSynchronize(s));
+                if (!*(volatile int*)&w->host->active) c = parts - 2;  // the end is next
+            }
         }
     }
     const GmresState& h = *w->host;
