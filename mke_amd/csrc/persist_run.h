@@ -201,7 +201,7 @@ __device__ __forceinline__ int hop(Hop& h, int nv, bool last, HopLds* l, double*
 // --------------------------------------------------------------- kernel --
 template <typename VT, typename MT>
 struct PArgs {
-    int n, ld, G, Gp, m, width, width64;
+    int n, ld, G, Gp, m, width;  // of both forms of the matrix
     const int* col;
     const MT* val;
     const int* col64;
@@ -326,7 +326,14 @@ __device__ __forceinline__ void take_off(int j, double h, VT (&w)[KR_RPT], const
     }
 }
 
-template <typename VT, typename MT, int ORTHO>
+// PRE: rows of 1 to ELL_MAXW entries, the thread's matrix rows in registers
+// throughout; otherwise rows of any width, read anew in every product.  With
+// PRE `pre` is always true; the test at run time and the loop behind it keep
+// the compiler's schedule of a step (the test left out: level 7 FP64 MGS 5.30
+// instead of 5.06 ms, in six forms that were tried, 36,503 rows FP32 CGS2 1.80
+// instead of 1.77).  256 threads with FP64 vectors are faster without it
+// (level 4 287 instead of 293 us).
+template <typename VT, typename MT, int ORTHO, bool PRE>
 __global__ void __launch_bounds__(BS)
 k_persist(PArgs<VT, MT> a)
 {
@@ -366,8 +373,8 @@ k_persist(PArgs<VT, MT> a)
             r0[r] = b[r];
         }
         if (a.use_x0) {
-            krylov_rows<double, double, false, KR_RPT>(n, a.width64, base, a.col64, a.val64, X, ld,
-                                                       1.0, xo, ax);
+            krylov_rows<double, double, false, KR_RPT, PRE>(n, a.width, base, a.col64, a.val64, X,
+                                                            ld, 1.0, xo, ax);
 #pragma unroll
             for (int r = 0; r < KR_RPT; ++r) r0[r] = b[r] - ax[r];
         }
@@ -404,9 +411,10 @@ k_persist(PArgs<VT, MT> a)
 
     // the thread's matrix rows (past a row's width its last slot with the
     // value 0, past row n row n - 1: every load is in bounds), and its rows of the basis
-    const bool pre = a.width >= 1 && a.width <= ELL_MAXW;
     unsigned sc[KR_RPT][ELL_MAXW];  // byte offsets into W
     MT sv[KR_RPT][ELL_MAXW];
+    const bool pre = PRE && ((BS == 256 && sizeof(VT) == 8) ||
+                             (a.width >= 1 && a.width <= ELL_MAXW));
     if (pre && active) {
 #pragma unroll
         for (int r = 0; r < KR_RPT; ++r) {
@@ -467,8 +475,12 @@ k_persist(PArgs<VT, MT> a)
                 }
             } else {
                 VT xo[KR_RPT];
-                krylov_rows_loop<VT, MT, true, KR_RPT>(n, a.width, opaque(base), a.col, a.val, W,
-                                                       1, inv, xo, w);
+                if constexpr (PRE)
+                    krylov_rows_each<VT, MT, true, KR_RPT>(n, a.width, opaque(base), a.col, a.val,
+                                                           W, 1, inv, xo, w);
+                else
+                    krylov_rows_loop<VT, MT, true, KR_RPT>(n, a.width, opaque(base), a.col, a.val,
+                                                           W, 1, inv, xo, w);
             }
             V.put(j, vj);
             put_dots<VT>(j, w, V, &l);
@@ -526,8 +538,8 @@ k_persist(PArgs<VT, MT> a)
         // r = b - A x in FP64, the next cycle's vector
         double res[KR_RPT], xo[KR_RPT];
         const int rb = opaque(base);
-        krylov_rows<double, double, true, KR_RPT>(n, a.width64, rb, a.col64, a.val64, X, ld, 1.0,
-                                                  xo, res);
+        krylov_rows<double, double, true, KR_RPT, PRE>(n, a.width, rb, a.col64, a.val64, X, ld,
+                                                       1.0, xo, res);
 #pragma unroll
         for (int r = 0; r < KR_RPT; ++r) {
             const int rr = rb + r * KR_STRIDE;
@@ -577,7 +589,7 @@ __global__ void k_ring_reset(xch_t* ring, size_t count, int G, int Gp, int* abor
 
 // Workgroups of the kernel that the device holds at once, per template
 // instance, computed once (thread-safe static initialisation).
-template <typename VT, typename MT, int ORTHO>
+template <typename VT, typename MT, int ORTHO, bool PRE>
 int capacity()
 {
     static const int n = [] {
@@ -585,7 +597,7 @@ int capacity()
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per, (const void*)k_persist<VT, MT, ORTHO>, BS, 0) != hipSuccess)
+                &per, (const void*)k_persist<VT, MT, ORTHO, PRE>, BS, 0) != hipSuccess)
             return 0;
         return cus * per;
     }();
@@ -599,7 +611,7 @@ inline long poll_limit(const char* name, long limit)
 }
 
 // Columns q0 .. q0 + K - 1 of the ld in B and X.
-template <typename VT, typename MT, int ORTHO>
+template <typename VT, typename MT, int ORTHO, bool PRE>
 int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int ld, const double* B,
            double* X, const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles,
            int first, hipStream_t s)
@@ -616,7 +628,6 @@ int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int
     }
     PArgs<VT, MT> a;
     a.n = n, a.ld = ld, a.G = G, a.Gp = Gp, a.m = o.restart, a.width = E.width;
-    a.width64 = A->ell64.width;
     a.col = E.col.p, a.val = E.val.p, a.col64 = A->ell64.col.p, a.val64 = A->ell64.val.p;
     a.dscale = dscale, a.B = B + q0, a.X = X + q0, a.W = (VT*)w->W.p + (size_t)q0 * ldw, a.ldw = ldw;
     a.ring = w->xch.p() + (w->parity ? slots : 0);
@@ -631,7 +642,7 @@ int launch(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int q0, int K, int
     a.max_iters = o.max_iters, a.max_cycles = max_cycles, a.use_x0 = o.use_x0;
     a.stall = stall, a.first = first;
     for (int q = q0; q < q0 + K; ++q) w->host[q].active = -1;  // until the kernel writes it
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_persist<VT, MT, ORTHO>), dim3(G * K), dim3(BS), 0, s, a);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_persist<VT, MT, ORTHO, PRE>), dim3(G * K), dim3(BS), 0, s, a);
     PHG_HIP(hipGetLastError());
     return PHG_OK;
 }
@@ -666,14 +677,14 @@ struct Turn {
     }
 };
 
-template <typename VT, typename MT, int ORTHO>
+template <typename VT, typename MT, int ORTHO, bool PRE>
 int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
         const phg_gmres_opts& o, const double* dscale, bool stall, int max_cycles, int max_rounds,
         int* launches, double* ms, hipStream_t s)
 {
     const int n = A->n_rows, G = workgroups(n);
     // columns of a launch, and launches for all columns, of equal size
-    const int fit = std::min(capacity<VT, MT, ORTHO>(), KR_MAXG) / G;
+    const int fit = std::min(capacity<VT, MT, ORTHO, PRE>(), KR_MAXG) / G;
     if (fit < 1) return PERSIST_NOT_HERE;
     const int rounds = (K + fit - 1) / fit, per = (K + rounds - 1) / rounds;
     if (rounds > max_rounds) return PERSIST_NOT_HERE;
@@ -724,7 +735,7 @@ int run(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* 
                 for (int q = q0; q < q0 + kq; ++q)
                     any = any || (again ? w->host[q].active == -1 : w->host[q].active == 1);
                 if (!any) continue;
-                const int rc = launch<VT, MT, ORTHO>(A, E, w, q0, kq, K, B, X, o, dscale, stall,
+                const int rc = launch<VT, MT, ORTHO, PRE>(A, E, w, q0, kq, K, B, X, o, dscale, stall,
                                                      max_cycles, first, s);
                 if (rc) {
                     (void)hipStreamSynchronize(s);  // those before it, in this turn
@@ -768,10 +779,17 @@ template <typename VT, typename MT, typename... Rest>
 int run_ortho(phg_matrix_s* A, const Ell<MT>& E, PersistWork* w, int K, const double* B, double* X,
               const phg_gmres_opts& o, Rest... rest)
 {
+    const bool pre = E.width >= 1 && E.width <= ELL_MAXW;
     switch (o.ortho) {
-    case PHG_MGS: return run<VT, MT, PHG_MGS>(A, E, w, K, B, X, o, rest...);
-    case PHG_CGS2: return run<VT, MT, PHG_CGS2>(A, E, w, K, B, X, o, rest...);
-    default: return run<VT, MT, PHG_CGS1>(A, E, w, K, B, X, o, rest...);
+    case PHG_MGS:
+        return pre ? run<VT, MT, PHG_MGS, true>(A, E, w, K, B, X, o, rest...)
+                   : run<VT, MT, PHG_MGS, false>(A, E, w, K, B, X, o, rest...);
+    case PHG_CGS2:
+        return pre ? run<VT, MT, PHG_CGS2, true>(A, E, w, K, B, X, o, rest...)
+                   : run<VT, MT, PHG_CGS2, false>(A, E, w, K, B, X, o, rest...);
+    default:
+        return pre ? run<VT, MT, PHG_CGS1, true>(A, E, w, K, B, X, o, rest...)
+                   : run<VT, MT, PHG_CGS1, false>(A, E, w, K, B, X, o, rest...);
     }
 }
 

@@ -335,3 +335,29 @@ def test_batch_with_columns_that_are_not_finite():
             assert torch.equal(Y[:, ::2], X[:, ::2])
     Z, got, done = _batch(A, B[:, ::2].contiguous(), None, 1, ortho=P.CGS2)
     assert all(done) and torch.equal(Z, X[:, ::2])
+
+
+@pytest.mark.parametrize("width", [8, 9, 15, 16, 17, 27])
+def test_rows_wider_than_one_group(width):
+    """Rows around multiples of the eight entries that are loaded together,
+    in both forms of the single and the batched solve and each precision
+    (ragged at the ends of the band)."""
+    n = 2600
+    for ortho, precision in ((P.MGS, P.F64), (P.CGS2, P.F32), (P.MGS, P.BF16)):
+        _check(n, width, ortho=ortho, precision=precision)
+    csr = _line(n, width, width)
+    A = P.Matrix.from_csr(n, n, *csr)
+    Bh = np.random.default_rng(width).standard_normal((n, 5))
+    B = torch.as_tensor(Bh, device=DEV)
+    for opts in (dict(ortho=P.CGS2), dict(ortho=P.CGS1, precision=P.F32),
+                 dict(ortho=P.CGS2, precision=P.BF16)):
+        its = []
+        for persistent in (1, 0):
+            X, i, done = _batch(A, B, None, persistent, **opts)
+            its.append(i)
+            assert all(done)
+            for q in range(5):
+                r = Bh[:, q] - O.spmv(*csr, np.ascontiguousarray(X[:, q].cpu().numpy()))
+                assert np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(Bh[:, q])
+        assert max(abs(a - b) for a, b in zip(*its)) <= 1, its
+    A.close()
