@@ -1108,23 +1108,26 @@ void set_shape_rpt(int n, int kp, int prec, int rpt)
 // How many persistent launches (persist.hip) the K columns may take for that
 // form to be the faster one, from the time per Arnoldi step of both.  The
 // kernels here: 26 us for the four launches of a step with one Gram-Schmidt
-// pass, 43 us for the six with two, and the vectors they read and write at
-// 4.2 TB/s.  A persistent launch: 6.8 to 12 us, and 0.01 us per workgroup of
-// a column.  Of 92 shapes measured in both forms at levels 4 to 7 with 1 to 64
-// columns the model picks the faster one in all; its times are off by up to
-// 22 % (launches) and 29 % (persistent, 7 us steps of one column).  It takes
-// K as it is, not KP: 24 mass columns at level 6 are faster in four persistent
-// launches, 32 as launches.  Per step, here and persistent: level 5 x 8 columns
-// FP64 CGS2 48 and 12 us, level 6 x 64 303 and 144, level 7 x 1 56 and 14,
-// level 7 x 16 277 and 234; level 7 x 16 FP32 CGS1 103 and 145; mass solves
-// (restart 8, CGS1) level 6 x 24 61 and 52, level 6 x 64 101 and 143.
+// pass, 43 us for the six with two, and the vectors that they read and write
+// at 5.8 TB/s (FP32), 5.5 (FP64, two passes) and 4.7 (FP64, one).  A persistent
+// launch: 7 to 13 us, and 0.006 us per workgroup of a column.  Of 197 shapes
+// measured in both forms, 10,000 to 250,000 rows and 1 to 64 columns, the model
+// picks the faster one in 196 (the other: 7 %); its times are off by up to 30 %
+// (launches) and 70 % (persistent mass solves of one column), far from the
+// line.  It takes K as it is, not KP: 24 mass columns at level 6 are
+// faster in four persistent launches, 32 and 48 as launches.  Per step, here and
+// persistent: level 5 x 8 columns FP64 CGS2 48 and 12 us, level 6 x 64 303 and
+// 144, level 7 x 1 55 and 14, level 7 x 16 243 and 224; level 7 FP32 CGS2 x 10
+// 136 and 112, x 14 136 and 158; mass solves (restart 8, CGS1) level 6 x 24
+// 60 and 49, x 48 90 and 98.
 int persistent_rounds(int n, int kp, int m, bool f64, bool twice)
 {
     const double passes = twice ? 2.0 : 1.0, es = f64 ? 8.0 : 4.0;
     const double vectors = 0.5 * (m + 1) * (passes + 1.0) + 5.0 + 16.0 / m;
-    const double here = 9.0 + 17.0 * passes + (double)n * kp * es * vectors / 4.2e6;
-    const double there = (f64 ? 9.0 : 6.8) + (passes - 1.0) * (f64 ? 3.0 : 2.7) +
-                         0.01 * n / 1024.0 + 24.0 / m;
+    const double rate = f64 ? (twice ? 5.5e6 : 4.7e6) : 5.8e6;  // bytes per us
+    const double here = 9.0 + 17.0 * passes + (double)n * kp * es * vectors / rate;
+    const double there = (f64 ? 9.2 : 6.2) + (passes - 1.0) * (f64 ? 3.0 : 2.7) +
+                         0.006 * n / 1024.0 + 24.0 / m;
     return (int)(here / there);
 }
 
