@@ -195,8 +195,12 @@ k_sumsq(int n, int R, const double* __restrict__ b, int S, double* __restrict__ 
 // Arnoldi step j < NV: v_j = W_src / h (stored), W_dst = A v_j, and the block
 // partials of <W_dst, v_i>, i <= j.  Row by row; a row's basis entries are
 // loaded without a branch (past j - 1 the last one again, not used), so that
-// all of them are in flight, GM_HALF at a time.
-template <typename VT, typename MT, int NV>
+// all of them are in flight, GM_HALF at a time.  SHORT: matrix rows of 1 to
+// ELL_MAXW entries, tested at run time all the same (with the wide rows' loop
+// behind the test instead of one entry by entry a level-8 solve took 0.7 %
+// longer, without the test 6 %: the branch keeps the basis loads and the
+// gathers in their order).
+template <typename VT, typename MT, int NV, bool SHORT>
 __global__ void __launch_bounds__(GM_BS)
 k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __restrict__ val,
             const VT* __restrict__ Wsrc, VT* __restrict__ V, size_t ldv, VT* __restrict__ Wdst,
@@ -217,7 +221,12 @@ k_step_spmv(int n, int R, int width, const int* __restrict__ col, const MT* __re
         VT v[N1], vj, w;
 #pragma unroll
         for (int i = 0; i < N1; ++i) v[i] = basis_at(V, ldv, max(min(i, j - 1), 0), row);
-        krylov_rows<VT, MT, false, 1>(n, width, row, col, val, Wsrc, 1, inv, &vj, &w);
+        if (SHORT && width >= 1 && width <= ELL_MAXW)
+            krylov_rows<VT, MT, false, 1, true>(n, width, row, col, val, Wsrc, 1, inv, &vj, &w);
+        else if (SHORT)
+            krylov_rows_each<VT, MT, false, 1>(n, width, row, col, val, Wsrc, 1, inv, &vj, &w);
+        else
+            krylov_rows_loop<VT, MT, false, 1>(n, width, row, col, val, Wsrc, 1, inv, &vj, &w);
         vj = vj * inv;
         V[(size_t)j * ldv + row] = vj;
         Wdst[row] = w;
@@ -493,12 +502,12 @@ int prepare_passes(GmresWork* w)
     return PHG_OK;
 }
 
-template <typename VT, typename MT, int NV>
+template <typename VT, typename MT, int NV, bool SHORT>
 void step_nv(const Ell<MT>& E, GmresWork* w, const VT* src, VT* dst, int j, hipStream_t s)
 {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_step_spmv<VT, MT, NV>), dim3(w->G), dim3(GM_BS), 0, s, w->n,
-                       w->R, E.width, E.col.p, E.val.p, src, (VT*)w->V.p, w->ldv, dst, j, w->S,
-                       w->part.p, w->st.p);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_step_spmv<VT, MT, NV, SHORT>), dim3(w->G), dim3(GM_BS), 0, s,
+                       w->n, w->R, E.width, E.col.p, E.val.p, src, (VT*)w->V.p, w->ldv, dst, j,
+                       w->S, w->part.p, w->st.p);
 }
 template <typename VT, int NV>
 void update_nv(GmresWork* w, VT* dst, int j, bool dots, bool norm, hipStream_t s)
@@ -532,7 +541,11 @@ void by_step(int j, F f)
 template <typename VT, typename MT>
 void step(const Ell<MT>& E, GmresWork* w, const VT* src, VT* dst, int j, hipStream_t s)
 {
-    by_step(j, [&](auto nv) { step_nv<VT, MT, decltype(nv)::value>(E, w, src, dst, j, s); });
+    by_step(j, [&](auto nv) {
+        constexpr int NV = decltype(nv)::value;
+        if (E.width >= 1 && E.width <= ELL_MAXW) step_nv<VT, MT, NV, true>(E, w, src, dst, j, s);
+        else step_nv<VT, MT, NV, false>(E, w, src, dst, j, s);
+    });
 }
 
 template <typename VT>

@@ -189,7 +189,7 @@ __device__ __forceinline__ void krylov_rows_loop(int n, int width, int base,
     }
 }
 
-// The same entry by entry (persist_run.h has the reason).
+// The same entry by entry (k_step_spmv and k_persist have the reason).
 template <typename VT, typename MT, bool AGENT, int RG>
 __device__ __forceinline__ void krylov_rows_each(int n, int width, int base,
                                                  const int* __restrict__ col,
