@@ -1109,23 +1109,26 @@ void set_shape_rpt(int n, int kp, int prec, int rpt)
 // form to be the faster one, from the time per Arnoldi step of both.  The
 // kernels here: 26 us for the four launches of a step with one Gram-Schmidt
 // pass, 43 us for the six with two, and the vectors that they read and write
-// at 5.8 TB/s (FP32), 5.5 (FP64, two passes) and 4.7 (FP64, one).  A persistent
-// launch: 7 to 13 us, and 0.006 us per workgroup of a column.  Of 197 shapes
-// measured in both forms, 10,000 to 250,000 rows and 1 to 64 columns, the model
-// picks the faster one in 196 (the other: 7 %); its times are off by up to 30 %
-// (launches) and 70 % (persistent mass solves of one column), far from the
-// line.  It takes K as it is, not KP: 24 mass columns at level 6 are
-// faster in four persistent launches, 32 and 48 as launches.  Per step, here and
-// persistent: level 5 x 8 columns FP64 CGS2 48 and 12 us, level 6 x 64 303 and
-// 144, level 7 x 1 55 and 14, level 7 x 16 243 and 224; level 7 FP32 CGS2 x 10
-// 136 and 112, x 14 136 and 158; mass solves (restart 8, CGS1) level 6 x 24
-// 60 and 49, x 48 90 and 98.
+// at 6 TB/s, less for 32 and 64 columns and beyond 0.5 GB a step (level 7 x 64:
+// 3.9 to 4.4).  A persistent launch: 7 to 13 us, and 0.006 us per workgroup of
+// a column.  Of 292 shapes measured in both forms, 10,000 to 250,000 rows and
+// 1 to 64 columns, the model picks the faster one in 291 (the other: 7 %); its
+// times are off by up to 31 % (launches) and 72 % (persistent mass solves of one
+// column), far from the line.  It takes K as it is, not KP: 24 mass columns
+// at level 6 are faster in four persistent launches, 32 and 48 as launches.
+// Per step, here and persistent: level 5 x 8 columns FP64 CGS2 48 and 12 us,
+// level 6 x 64 262 and 138, level 7 x 1 55 and 14, x 16 244 and 224, x 64 1036 and
+// 898; level 7 FP32 CGS2 x 10 136 and 112, x 14 136 and 158, x 33 576 and 377,
+// x 64 598 and 730; mass solves (restart 8, CGS1) level 6 x 24 60 and 49, x 48
+// 90 and 98.
 int persistent_rounds(int n, int kp, int m, bool f64, bool twice)
 {
     const double passes = twice ? 2.0 : 1.0, es = f64 ? 8.0 : 4.0;
     const double vectors = 0.5 * (m + 1) * (passes + 1.0) + 5.0 + 16.0 / m;
-    const double rate = f64 ? (twice ? 5.5e6 : 4.7e6) : 5.8e6;  // bytes per us
-    const double here = 9.0 + 17.0 * passes + (double)n * kp * es * vectors / rate;
+    const double bytes = (double)n * kp * es * vectors;
+    const double rate = 6e6 / (1.0 + 0.12 * std::max(0.0, std::log2(kp / 16.0))) /  // bytes per us
+                        (1.0 + 0.03 * std::max(0.0, std::log2(bytes / 0.5e9)));
+    const double here = 9.0 + 17.0 * passes + bytes / rate;
     const double there = (f64 ? 9.2 : 6.2) + (passes - 1.0) * (f64 ? 3.0 : 2.7) +
                          0.006 * n / 1024.0 + 24.0 / m;
     return (int)(here / there);
